@@ -62,7 +62,7 @@ def sketch_work(lengths):
 
 def kernel_name(b):
     if b["kind"] == "window":
-        return "k_align_win<%d>" % b["width"]
+        return ("k_align_win<%d>" if b["width"] <= 8 else "k_align_lanes<%d>") % b["width"]
     if b["kind"] == "wave":
         return "k_align_wave<%d>" % b["width"]
     if b["kind"] == "seg":

@@ -229,20 +229,19 @@ int ngia_db_band_jobs(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t ba
 
 /* Length bins of the last batched graph.  No reference counterpart (the
  * reference aligns every band's jobs in one kernel_dynamic launch).  A pair's
- * bin follows from its band window W = lsft/32 + ceil(rsft/32) words:
- * W <= 16 -> a window bin, aligned by the shape the tuning picks for its size
- * (one thread per pair by default); W <= 21 -> 8 lanes per pair with three
- * words per lane, eight pairs per wavefront; W <= 30 -> 16 lanes per pair with
- * two words per lane, four pairs per wavefront; W = 31 ->
- * 32 lanes per pair, two pairs per wavefront; W <= 45 and W <= 60 -> 16 lanes
- * per pair with three and four words per lane; W <= 64*K - K + 1 -> a
- * wavefront per pair with K words per lane; wider -> the plain kernel;
- * length-rejected or empty targets score 0 without a kernel.  A bin of 17..30
- * words holding fewer than 32,768 pairs goes to 32 lanes per pair, one of
- * 32..60 words to a wavefront per pair (NGIA_SEG2_MIN in the environment of
- * ngia_open overrides the limit). */
+ * bin follows from its band window W = lsft/32 + ceil(rsft/32) words and, under
+ * ngia_tuning or its defaults, the bin's size: W <= 16 -> a window bin (one
+ * thread per pair) or the shape the tuning picks; W <= 60 -> one thread per
+ * pair (window bins of up to 40 words) when the pairs are many, else several
+ * words per lane (W <= 21 on 8 lanes per pair, <= 30 and 32..60 on 16), or one
+ * word per lane on 32 lanes (W <= 31) or a wavefront per pair (W >= 32) when
+ * they are few; W <= 64*K - K + 1 -> a wavefront per pair with K words per
+ * lane; wider -> the plain kernel; length-rejected or empty targets score 0
+ * without a kernel.  NGIA_SEG2_MIN in the environment of ngia_open keeps
+ * windows of 17..60 words off one thread per pair and sets the size below
+ * which they take one word per lane or a wavefront (default 32,768). */
 #define NGIA_BIN_ZERO 0u
-#define NGIA_BIN_WINDOW 1u   /* k_align_win<W>: one thread per pair; width = W */
+#define NGIA_BIN_WINDOW 1u   /* k_align_win<W>, k_align_lanes: one thread per pair; width = W */
 #define NGIA_BIN_WAVE 2u     /* k_align_wave<K>: one wavefront per pair; width = K */
 #define NGIA_BIN_PLAIN 3u
 #define NGIA_BIN_SEG 4u      /* k_align_seg<G>: 64/G pairs per wavefront; width = G */
@@ -272,7 +271,7 @@ int ngia_db_bin_stats(ngia_ctx* ctx, ngia_db* db, ngia_bin_stat* out, uint32_t c
  * one word per lane), 8 lanes of two words per pair, or a wavefront per pair.
  * Which is fastest depends on W, the bin's size, the identity (pair length)
  * and the device. */
-#define NGIA_SHAPE_WINDOW 0u  /* k_align_win<W> */
+#define NGIA_SHAPE_WINDOW 0u  /* k_align_win<W> or k_align_lanes: one thread per pair */
 #define NGIA_SHAPE_SEG16 1u   /* k_align_seg<16>: four pairs per wavefront (W <= 15) */
 #define NGIA_SHAPE_SEG32 2u   /* k_align_seg<32>: two pairs per wavefront */
 #define NGIA_SHAPE_WAVE 3u    /* k_align_wave<1> */
@@ -284,14 +283,17 @@ int ngia_db_bin_stats(ngia_ctx* ctx, ngia_db* db, ngia_bin_stat* out, uint32_t c
  * 32..45 and 46..60 (four 16-lane segments of three and four words, or a
  * wavefront per pair). */
 #define NGIA_LONG_GROUPS 4
-#define NGIA_LONG_DEFAULT 0u /* several words per lane from 32,768 pairs (NGIA_SEG2_MIN) */
-#define NGIA_LONG_MULTI 1u   /* several words per lane */
+#define NGIA_LONG_DEFAULT 0u /* by size: one lane per pair, several words per lane, or one */
+#define NGIA_LONG_MULTI 1u   /* several words per lane; from 65,536 pairs the whole window of
+                              * up to 40 words on one lane */
 #define NGIA_LONG_SINGLE 2u  /* one word per lane, or a wavefront per pair */
 typedef struct {
   /* window bin W holding c pairs takes shape[W][k], k the last size class with
    * class_size[k] <= c (class 0 below class_size[0]); class sizes ascend, 0
-   * ends the list.  A fresh context's table is all zero: every window bin on
-   * one thread per pair. */
+   * ends the list.  A fresh context's table is empty (all zero): window bins
+   * of up to 8 words take one thread per pair, wider ones too when the round
+   * holds enough such work to fill the device, else 8 or 32 lanes or a
+   * wavefront per pair. */
   uint32_t class_size[NGIA_TUNE_CLASSES];
   uint32_t shape[17][NGIA_TUNE_CLASSES];
   /* the same for databases whose residues use at most five codes (DNA), whose

@@ -165,13 +165,13 @@ void enqueue_bins(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
   bin_pairs(db->pairs.as<uint2>(), npairs, len, thr, db->bin_of.as<uint32_t>(), dc->bin_cnt,
             dc->bin_off, dc->cursor, db->list.as<uint32_t>(), dc->bin_tiles, db->score.as<uint32_t>(),
             ctx->wave_kmax, dc->remap, db->compact ? ctx->route_compact : ctx->route, ctx->seg2_min,
-            grid, s);
+            ctx->lane_fill, db->compact, grid, s);
 }
 
 // Part 2: the alignment kernels of the bins in `mask` (bit b: bin b holds
 // pairs), then the passing pairs as raw edges (capturable), on stream s and,
 // unless `serial`, the side streams.
-void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t mask,
+void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, uint64_t mask,
                    bool time_align, bool tally, hipStream_t s, bool serial = false) {
   const uint32_t n = db->n;
   const float thr = (float)identity / 100.0f;
@@ -187,18 +187,17 @@ void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t mask,
     if (tally) a.tally = &dc->run_tiles[bin];
     return a;
   };
-  // The bins run concurrently, forked onto the side streams and joined back.
-  // Every wave bin below K = 16 is latency bound (one pair per wavefront, the
-  // bin lasts as long as its longest pair), so each gets a side stream of its
-  // own and starts at the fork: K = 8 on side stream 0, K = 4 on 1, K = 2 on
-  // 2, K = 1 on 3.  The window bins (throughput bound) that hold pairs follow
-  // round-robin on side streams 0, 3 and 2, widest first.  K = 32 and 16 (128
-  // and 64 KiB of LDS per block), when they hold pairs, run before the fork:
-  // launched beside the others, their blocks would wait for a CU with that
-  // much free LDS, which the other bins' persistent blocks hold until they
-  // finish.
+  // The bins run concurrently, forked onto the side streams in turn and joined
+  // back: the wavefront bins first (latency bound: one pair per wavefront,
+  // the bin lasts as long as its longest pair), then the widest windows.
+  // K = 32 and 16 (128 and 64 KiB of LDS per block), when they hold pairs, run
+  // before the fork: launched beside the others, their blocks would wait for
+  // a CU with that much free LDS, which the other bins' persistent blocks hold
+  // until they finish.
   if (time_align) NGIA_HIP(hipEventRecord(ctx->ev[2], s));
   const bool fork = !ctx->serial_bins && !serial;
+  int turn = 0;
+  auto next = [&] { return fork ? ctx->side[turn++ % kSideStreams] : s; };
   auto mark = [&](int bin, int end, hipStream_t q) {
     if (time_align) NGIA_HIP(hipEventRecord(ctx->bin_ev[2 * bin + end], q));
   };
@@ -217,10 +216,12 @@ void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t mask,
     NGIA_HIP(hipEventRecord(ctx->fork, s));
     for (int k = 0; k < kSideStreams; k++) NGIA_HIP(hipStreamWaitEvent(ctx->side[k], ctx->fork, 0));
   }
-  for (int k = 3; k >= 0; k--) wave(k, fork ? ctx->side[3 - k] : s);
-  // The segmented bins (several pairs per wavefront) follow K = 8 and K = 1.
-  auto seg = [&](int bin, hipStream_t q) {
+  for (int k = 3; k >= 0; k--)
+    if (holds(kBinWave0 + k)) wave(k, next());
+  // The segmented bins (several pairs per wavefront).
+  auto seg = [&](int bin) {
     if (!holds(bin)) return;
+    hipStream_t q = next();
     mark(bin, 0, q);
     const int G = seg_lanes(bin), K = seg_words(bin);
     launch_align_seg(G, K, args(bin), db->pairs.as<uint2>(), db->list.as<uint32_t>(),
@@ -228,18 +229,42 @@ void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t mask,
                      ctx->prop.multiProcessorCount * seg_blocks_per_cu(G, K), q);
     mark(bin, 1, q);
   };
-  seg(kBinSeg16x4, fork ? ctx->side[2] : s);
-  seg(kBinSeg16x3, fork ? ctx->side[3] : s);
-  seg(kBinSeg8x3, fork ? ctx->side[1] : s);
-  seg(kBinSeg8x2, fork ? ctx->side[2] : s);
-  seg(kBinSeg16x2, fork ? ctx->side[0] : s);
-  seg(kBinSeg32, fork ? ctx->side[0] : s);
-  seg(kBinSeg16, fork ? ctx->side[3] : s);
-  static constexpr int kWinStreams[3] = {0, 3, 2};
-  int slot = 0;
-  for (int W = kWinMax; W >= 2; W--) {
+  // One lane per pair, a launch per width class over the bins that hold
+  // pairs; the timed form launches each bin by itself.  Compact alphabets
+  // keep k_align_win up to kWinMax words.
+  const int win_max = a0.slots ? kWinMax : kWinLds;
+  const uint32_t cus = (uint32_t)ctx->prop.multiProcessorCount;
+  auto lanes = [&](int cls, int wlo, int whi, hipStream_t q) {
+    launch_align_lanes(cls, a0, db->pairs.as<uint2>(), db->list.as<uint32_t>(), dc->bin_off, dc->bin_cnt,
+                       dc->queue[0], db->score.as<uint32_t>(), tally ? dc->run_tiles : nullptr,
+                       (uint32_t)wlo, (uint32_t)whi, cus, (uint64_t)n * bands, q);
+  };
+  auto lane_bins = [&](int cls) {
+    int wlo = 0, whi = 0;  // the widths of this class that hold pairs
+    for (int W = kLaneMax; W >= 2; W--) {
+      if (lane_class(W) != cls || !holds(lane_bin(W)) || (W > kWinLds && W <= win_max)) continue;
+      wlo = W;
+      if (!whi) whi = W;
+    }
+    if (!whi) return;
+    hipStream_t q = next();
+    if (!time_align) return lanes(cls, wlo, whi, q);
+    for (int W = whi; W >= wlo; W--) {
+      if (!holds(lane_bin(W))) continue;
+      mark(lane_bin(W), 0, q);
+      lanes(cls, W, W, q);
+      mark(lane_bin(W), 1, q);
+    }
+  };
+  lane_bins(3);
+  lane_bins(2);
+  for (const int bin : {kBinSeg16x4, kBinSeg16x3, kBinSeg8x3, kBinSeg16x2}) seg(bin);
+  lane_bins(1);
+  for (const int bin : {kBinSeg32, kBinSeg16, kBinSeg8x2}) seg(bin);
+  lane_bins(0);
+  for (int W = win_max; W >= 2; W--) {
     if (!holds(W)) continue;
-    hipStream_t q = fork ? ctx->side[kWinStreams[slot++ % 3]] : s;
+    hipStream_t q = next();
     mark(W, 0, q);
     launch_align_win(W, args(W), db->pairs.as<uint2>(), db->list.as<uint32_t>(), &dc->bin_off[W],
                      &dc->bin_cnt[W], dc->queue[W], db->score.as<uint32_t>(),
@@ -352,6 +377,7 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
   }
   key.push_back(db->t0);
   key.push_back(ctx->seg2_min);
+  key.push_back(ctx->lane_fill);
   const bool reuse = db->gexec && db->g_identity == identity && db->g_bands == bands &&
                      db->g_key == key;
   if (!eager && !reuse) {
@@ -371,12 +397,12 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
   d2h(ctx->pin + kPinCnt, db->counters.as<Counters>()->bin_cnt, sizeof(cnt), s);
   NGIA_HIP(hipStreamSynchronize(s));
   std::memcpy(cnt, ctx->pin + kPinCnt, sizeof(cnt));
-  uint32_t mask = 0;
+  uint64_t mask = 0;
   for (int b = 0; b < kBins; b++)
-    if (cnt[b]) mask |= 1u << b;
+    if (cnt[b]) mask |= 1ull << b;
   if (((mask >> kBinPlain) & 1u) && ensure_plain_bin_space(db, bands)) {
     // captures that launch the plain bin hold the old buffers
-    std::vector<std::pair<uint32_t, hipGraphExec_t>> keep;
+    std::vector<std::pair<uint64_t, hipGraphExec_t>> keep;
     for (auto& e : db->gexec2) {
       if ((e.first >> kBinPlain) & 1u)
         (void)hipGraphExecDestroy(e.second);
@@ -387,7 +413,7 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
   }
   if (eager) {
     // Same kernels without the graph, with events around the alignment phase.
-    enqueue_align(ctx, db, identity, mask, /*time_align=*/true, tally, s);
+    enqueue_align(ctx, db, identity, bands, mask, /*time_align=*/true, tally, s);
   } else {
     hipGraphExec_t g2 = nullptr;
     for (const auto& e : db->gexec2)
@@ -397,7 +423,7 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
         for (auto& e : db->gexec2) (void)hipGraphExecDestroy(e.second);
         db->gexec2.clear();
       }
-      g2 = capture(s, [&] { enqueue_align(ctx, db, identity, mask, false, false, s); });
+      g2 = capture(s, [&] { enqueue_align(ctx, db, identity, bands, mask, false, false, s); });
       db->gexec2.emplace_back(mask, g2);
     }
     NGIA_HIP(hipGraphLaunch(g2, s));
@@ -440,7 +466,7 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
   uint32_t launches = 0;
   for (int b = 0; b < kBins; b++) {
     const bool aligner = b == kBinPlain || is_seg_bin(b) ||
-                         (b >= 2 && b <= kWinMax) ||
+                         bin_width(b) >= 2 ||
                          (b >= kBinWave0 && b < kBinPlain && (1u << (b - kBinWave0)) <= ctx->wave_kmax);
     const bool launched = aligner && ((mask >> b) & 1u);
     launches += launched;
@@ -483,6 +509,12 @@ void bucket_rows(ngia_ctx* ctx, ngia_db* db, hipStream_t s) {
 // step measured the same, and the log-normal set's 8,192-record head at
 // -i 50 lost 1%; with 128, 11.6 against 11.3 ms on the heavy-tailed set.
 constexpr uint32_t kHeadMax = 8192;
+// Bins of 32..kLaneMax words.
+constexpr uint64_t head_lane_mask() {
+  uint64_t m = 0;
+  for (int W = 32; W <= kLaneMax; W++) m |= 1ull << lane_bin(W);
+  return m;
+}
 uint32_t head_records(const ngia_db* db, float thr, uint32_t min_window) {
   uint32_t h = 0;
   const uint32_t cap = std::min<uint32_t>(db->n, kHeadMax);
@@ -594,13 +626,13 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
     ngia_db* hd = step_head(ctx, db, h);
     hd->rep.ensure(256ull * h);
     ensure_batched_space(hd, bands);
-    uint32_t mask = 0;
-    for (uint32_t k = 0; (1u << k) <= ctx->wave_kmax; k++) mask |= 1u << (kBinWave0 + k);
+    uint64_t mask = 0;
+    for (uint32_t k = 0; (1u << k) <= ctx->wave_kmax; k++) mask |= 1ull << (kBinWave0 + k);
     // a head window below 61 words lets head pairs into the 3- and 4-word bins
-    if (ctx->head_window < 61) mask |= (1u << kBinSeg16x3) | (1u << kBinSeg16x4);
+    if (ctx->head_window < 61) mask |= head_lane_mask() | (1ull << kBinSeg16x3) | (1ull << kBinSeg16x4);
     if (head_may_need_plain(ctx, hd->max_len, thr)) {
       ensure_plain_bin_space(hd, bands);
-      mask |= 1u << kBinPlain;
+      mask |= 1ull << kBinPlain;
     }
     // the rest's sketch first, so that the context stream is busy while the
     // host enqueues the head's round
@@ -613,7 +645,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
     NGIA_HIP(hipEventRecord(ctx->head_rows, q));
     launch_bucket_small(sig, h, hd->rep.as<uint32_t>(), q);
     enqueue_bins(ctx, hd, identity, bands, q);
-    enqueue_align(ctx, hd, identity, mask, false, false, q, /*serial=*/true);
+    enqueue_align(ctx, hd, identity, bands, mask, false, false, q, /*serial=*/true);
     NGIA_HIP(hipEventRecord(ctx->head_done, q));
     hr.db = hd;
     hr.done = ctx->head_done;
@@ -664,6 +696,10 @@ extern "C" int ngia_open(int device, ngia_ctx** out) {
     ctx->bucket_small = bs && bs[0] == '1';
     const char* s2 = std::getenv("NGIA_SEG2_MIN");
     ctx->seg2_min = s2 ? (uint32_t)std::strtoul(s2, nullptr, 10) : kSeg2MinPairs;
+    const char* lf = std::getenv("NGIA_LANE_FILL");
+    ctx->lane_fill = lf ? (uint32_t)std::strtoul(lf, nullptr, 10)
+                     : s2 ? 0xFFFFFFFFu  // NGIA_SEG2_MIN asks for the segmented shapes
+                          : kLaneFill;
     const char* sb = std::getenv("NGIA_SERIAL_BINS");
     ctx->serial_bins = sb && sb[0] == '1';
     const char* rl = std::getenv("NGIA_RAW_LCS");
@@ -949,9 +985,9 @@ extern "C" int ngia_db_bin_stats(ngia_ctx* ctx, ngia_db* db, ngia_bin_stat* out,
     if (b == kBinZero) {
       o.kind = NGIA_BIN_ZERO;
       o.width = 0;
-    } else if (b <= kWinMax) {
+    } else if (bin_width(b)) {
       o.kind = NGIA_BIN_WINDOW;
-      o.width = (uint32_t)b;
+      o.width = (uint32_t)bin_width(b);
     } else if (b < kBinPlain) {
       o.kind = NGIA_BIN_WAVE;
       o.width = 1u << (b - kBinWave0);

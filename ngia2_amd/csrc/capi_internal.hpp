@@ -78,7 +78,7 @@ struct Counters {
 constexpr size_t kCounterStats = offsetof(Counters, queue);
 // Offsets into ngia_ctx::pin.
 constexpr size_t kPinOverflow = 0, kPinUnique = 8, kPinPairs = 16, kPinHeadPairs = 24,
-                 kPinCnt = 64, kPinCounters = 256, kPinHeadCounters = kPinCounters + kCounterStats,
+                 kPinCnt = 64, kPinCounters = 512, kPinHeadCounters = kPinCounters + kCounterStats,
                  kPinBytes = kPinHeadCounters + kCounterStats;
 static_assert(kPinCnt + 4 * kBins <= kPinCounters, "pinned slots overlap");
 
@@ -118,6 +118,9 @@ struct ngia_ctx {
   // kernel, one word per lane (env NGIA_SEG2_MIN; 0 keeps every such bin on
   // two words per lane)
   uint32_t seg2_min = ngia::kSeg2MinPairs;
+  // how much lane work makes one lane per pair pay (env NGIA_LANE_FILL; 0:
+  // always, all ones: never)
+  uint32_t lane_fill = ngia::kLaneFill;
   bool raw_lcs = false;  // env NGIA_RAW_LCS=1: alignment kernels store LCS lengths, not scores
   // env NGIA_FULL_ALPHABET=1: the window kernels keep the 16-code table even
   // for a compact alphabet
@@ -177,7 +180,7 @@ struct ngia_db {
   uint32_t g_identity = 0, g_bands = 0;
   std::vector<uintptr_t> g_key;
   // the alignment part, one capture per set of bins that hold pairs
-  std::vector<std::pair<uint32_t, hipGraphExec_t>> gexec2;
+  std::vector<std::pair<uint64_t, hipGraphExec_t>> gexec2;
   // per-bin figures of the last batched graph
   bool have_bins = false;
   ngia::Counters last{};

@@ -323,10 +323,9 @@ void pair_emit(const uint32_t* rep, uint32_t n, uint32_t bands, const uint64_t* 
   NGIA_HIP(hipGetLastError());
 }
 
-// Bin of a pair by its band window: W = a + c words.  Bins 2..kWinMax go to
-// k_align_win<W>; windows of up to 60 words to the segmented bins (8 lanes
-// per pair with 3 words per lane up to 21 words, 16 lanes with 2 at 22-30,
-// 32 lanes with one at 31, 16 lanes with 3 or 4 at 32-60);
+// Bin of a pair by its band window: W = a + c words.  A bin per width up to
+// kLaneMax words, which k_bin_offsets routes to the shape that aligns it; two
+// bins of the segmented kernels up to 60 words;
 // larger windows to k_align_wave<K> with the smallest K in {1,2,4,...,32}
 // with 64K >= W + K - 1 (the wave trails the band bottom in steps of K
 // words); T == 0 scores 0 at once (its LCS is 0, so the pass test fails);
@@ -341,9 +340,7 @@ __device__ inline uint32_t pair_bin(uint32_t R, uint32_t T, float thr, uint32_t 
   const uint32_t a = bd.lsft / 32, c = (bd.rsft + 31) / 32, W = a + c;
   *tiles = ref_tiles(R, T, thr, (T + 31) / 32);
   if (W <= (uint32_t)kWinMax) return W;  // W >= 2 whenever T > 0
-  if (W <= 21) return kBinSeg8x3;
-  if (W <= 30) return kBinSeg16x2;
-  if (W <= 31) return kBinSeg32;
+  if (W <= (uint32_t)kLaneMax) return (uint32_t)lane_bin((int)W);
   if (W <= 45) return kBinSeg16x3;
   if (W <= 60) return kBinSeg16x4;
   for (uint32_t k = 0, K = 1; K <= kmax; k++, K <<= 1)
@@ -383,54 +380,109 @@ __global__ void k_bin_count(const uint2* __restrict__ pairs, const uint64_t* __r
 
 // Route window bins by the tuned shapes (remap[b] = the bin that aligns bin
 // b's pairs, counts and tiles moved along), then bin_off[b] = exclusive prefix
-// of bin_cnt; also resets the scatter cursors.
-__global__ void k_bin_offsets(uint32_t* __restrict__ bin_cnt, uint32_t* __restrict__ bin_off,
-                              uint32_t* __restrict__ cursor, uint32_t* __restrict__ remap,
-                              unsigned long long* __restrict__ bin_tiles, RouteTable route,
-                              uint32_t seg2_min) {
-  if (threadIdx.x == 0) {
-    for (int b = 0; b < kBins; b++) remap[b] = (uint32_t)b;
-    for (int W = 2; W <= kWinMax; W++) {
-      if (!bin_cnt[W]) continue;
-      const uint32_t to = route_window_bin(route, (uint32_t)W, bin_cnt[W]);
-      if (to == (uint32_t)W) continue;
-      remap[W] = to;
-      bin_cnt[to] += bin_cnt[W];
-      bin_tiles[to] += bin_tiles[W];
-      bin_cnt[W] = 0;
-      bin_tiles[W] = 0;
-    }
-    // Windows of 17-30 words: several words per lane (four or eight pairs
-    // per wavefront) when the bin has the pairs to fill the device that way;
-    // a smaller bin (long pairs, every segment in flight at once either way)
-    // keeps one word per lane, whose per-character chain is shorter.
-    // Likewise windows of 32-60 words: three or four words per lane, or a
-    // wavefront per pair.
-    // The tuned table decides by the bin's size class, or leaves it to the
-    // size limit seg2_min (NGIA_LONG_DEFAULT).
-    auto fold = [&](int from, int to, int group) {
-      const uint32_t n2 = bin_cnt[from];
-      const uint32_t choice = route.lng[group][route_class(route, n2)];
-      if (n2 && (choice == NGIA_LONG_SINGLE || (choice == NGIA_LONG_DEFAULT && n2 < seg2_min))) {
-        remap[from] = (uint32_t)to;
-        bin_cnt[to] += n2;
-        bin_tiles[to] += bin_tiles[from];
-        bin_cnt[from] = 0;
-        bin_tiles[from] = 0;
-      }
+// of bin_cnt; also resets the scatter cursors.  One thread routes, over
+// copies in LDS: a chain of dependent global accesses took longer than the
+// counting.
+__global__ __launch_bounds__(64) void k_bin_offsets(uint32_t* __restrict__ bin_cnt,
+                                                    uint32_t* __restrict__ bin_off,
+                                                    uint32_t* __restrict__ cursor,
+                                                    uint32_t* __restrict__ remap,
+                                                    unsigned long long* __restrict__ bin_tiles,
+                                                    RouteTable route, uint32_t seg2_min,
+                                                    uint32_t lane_fill, bool compact) {
+  __shared__ uint32_t cnt[kBins], to_bin[kBins], off[kBins + 1];
+  __shared__ unsigned long long tiles[kBins];
+  static_assert(kBins <= 64, "one thread per bin");
+  const uint32_t t = threadIdx.x;
+  if (t < (uint32_t)kBins) {
+    cnt[t] = bin_cnt[t];
+    tiles[t] = bin_tiles[t];
+    to_bin[t] = t;
+    cursor[t] = 0;
+  }
+  __syncthreads();
+  if (t == 0) {
+    auto move = [&](int from, int to) {
+      if (!cnt[from] || from == to) return;
+      to_bin[from] = (uint32_t)to;
+      cnt[to] += cnt[from];
+      tiles[to] += tiles[from];
+      cnt[from] = 0;
+      tiles[from] = 0;
     };
-    fold(kBinSeg8x3, kBinSeg32, 0);
-    fold(kBinSeg16x2, kBinSeg32, 1);
-    fold(kBinSeg16x3, kBinWave0, 2);
-    fold(kBinSeg16x4, kBinWave0, 3);
+    const bool tuned = route.class_size[0] != 0;
+    // Whether one lane per pair pays for `c` pairs of `t` tiles in all.
+    unsigned long long total = 0;
+    for (int W = kWinLds + 1; W <= kLaneMax; W++) total += tiles[lane_bin(W)];
+    const bool lanes_off = lane_fill == 0xFFFFFFFFu;
+    auto lanes_pay = [&](uint32_t c, unsigned long long t) {
+      return !lanes_off && total * c >= (unsigned long long)lane_fill * t;
+    };
+    // Window bins: the tuned shape; without a table, kWinLds+1..kWinMax words
+    // by lanes_pay, and where it does not pay a wavefront or a segment per
+    // pair.  Compact alphabets have their own window kernels.
+    uint32_t small = 0;
+    for (int W = 2; W <= kWinMax; W++) {
+      if (!cnt[W]) continue;
+      if (tuned) {
+        move(W, (int)route_window_bin(route, (uint32_t)W, cnt[W]));
+      } else if (!compact && !lanes_off && W > kWinLds && !lanes_pay(cnt[W], tiles[W])) {
+        small += cnt[W];
+      }
+      if (!compact && W <= kWinLds && cnt[W] < kLowLanePairs) move(W, lane_bin(W));
+    }
+    if (small)
+      for (int W = kWinLds + 1; W <= kWinMax; W++)
+        if (cnt[W] && !lanes_pay(cnt[W], tiles[W]))
+          move(W, small <= kWavePairs ? kBinWave0 : W <= 14 ? kBinSeg8x2 : kBinSeg32);
+    // Windows of 17-60 words in four groups (and W = 31 by itself).  Up to
+    // kLaneMax words a group may keep one lane per pair, a bin per width.
+    // Else: several words per lane (four or eight pairs per wavefront) when
+    // the group has the pairs to fill the device that way; a smaller one
+    // (long pairs, every segment in flight at once either way) one word per
+    // lane, whose per-character chain is shorter, or a wavefront per pair.
+    // The tuned table decides by the group's size class, or leaves it to
+    // lanes_pay and the size limit seg2_min (NGIA_LONG_DEFAULT).
+    auto group = [&](int w0, int w1, int extra, int multi, int single, int g) {
+      uint32_t n2 = extra >= 0 ? cnt[extra] : 0u, nl = 0;
+      unsigned long long tl = 0;
+      for (int W = w0; W <= w1; W++) {
+        nl += cnt[lane_bin(W)];
+        tl += tiles[lane_bin(W)];
+      }
+      n2 += nl;
+      if (!n2) return;
+      const uint32_t choice =
+          g < 0 || !tuned ? NGIA_LONG_DEFAULT : route.lng[g][route_class(route, n2)];
+      const bool lanes = choice == NGIA_LONG_MULTI ? !lanes_off && n2 >= kLaneMinPairs
+                                                   : choice == NGIA_LONG_DEFAULT && lanes_pay(nl, tl);
+      const bool several = choice == NGIA_LONG_MULTI ||
+                           (choice == NGIA_LONG_DEFAULT && n2 >= seg2_min);
+      const int to = several ? multi : single;
+      if (!lanes)
+        for (int W = w0; W <= w1; W++) move(lane_bin(W), to);
+      if (extra >= 0) move(extra, to);  // the windows too wide for a lane
+    };
+    group(17, 21, -1, kBinSeg8x3, kBinSeg32, 0);
+    group(22, 30, -1, kBinSeg16x2, kBinSeg32, 1);
+    group(31, 31, -1, kBinSeg32, kBinSeg32, -1);
+    group(32, kLaneMax, kBinSeg16x3, kBinSeg16x3, kBinWave0, 2);
+    group(1, 0, kBinSeg16x4, kBinSeg16x4, kBinWave0, 3);
     uint32_t s = 0;
     for (int b = 0; b < kBins; b++) {
-      bin_off[b] = s;
-      cursor[b] = 0;
-      s += bin_cnt[b];
+      off[b] = s;
+      s += cnt[b];
     }
-    bin_off[kBins] = s;
+    off[kBins] = s;
   }
+  __syncthreads();
+  if (t < (uint32_t)kBins) {
+    bin_cnt[t] = cnt[t];
+    bin_tiles[t] = tiles[t];
+    remap[t] = to_bin[t];
+    bin_off[t] = off[t];
+  }
+  if (t == 0) bin_off[kBins] = off[kBins];
 }
 
 // Scatter pair indices into their bin's segment.  A block takes tiles of
@@ -470,15 +522,15 @@ __global__ __launch_bounds__(256) void k_bin_scatter(const uint64_t* __restrict_
 void bin_pairs(const uint2* pairs, const uint64_t* npairs, const uint32_t* len, float thr,
                uint32_t* bin_of, uint32_t* bin_cnt, uint32_t* bin_off, uint32_t* cursor,
                uint32_t* list, unsigned long long* bin_tiles, uint32_t* score, uint32_t kmax,
-               uint32_t* remap, const RouteTable& route, uint32_t seg2_min, uint32_t grid,
-               hipStream_t s) {
+               uint32_t* remap, const RouteTable& route, uint32_t seg2_min, uint32_t lane_fill,
+               bool compact, uint32_t grid, hipStream_t s) {
   // A sixteenth of the grid: every block ends with one global atomic per
   // nonempty bin, and a few bins take nearly all pairs, so those counters
   // see one atomic per block.
   hipLaunchKernelGGL(k_bin_count, dim3(std::max(grid / 16, 1u)), dim3(256), 0, s, pairs, npairs, len,
                      thr, kmax, bin_of, bin_cnt, bin_tiles, score);
   hipLaunchKernelGGL(k_bin_offsets, dim3(1), dim3(64), 0, s, bin_cnt, bin_off, cursor, remap,
-                     bin_tiles, route, seg2_min);
+                     bin_tiles, route, seg2_min, lane_fill, compact);
   hipLaunchKernelGGL(k_bin_scatter, dim3(grid), dim3(256), 0, s, npairs, bin_of, remap, bin_off,
                      cursor, list);
   NGIA_HIP(hipGetLastError());

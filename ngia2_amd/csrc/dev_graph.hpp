@@ -25,8 +25,29 @@ constexpr int kBinSeg16x3 = kBinSeg16x2 + 1;
 constexpr int kBinSeg16x4 = kBinSeg16x3 + 1;
 constexpr int kBinSeg8x3 = kBinSeg16x4 + 1;
 constexpr int kBinSeg8x2 = kBinSeg8x3 + 1;
-constexpr int kBins = kBinSeg8x2 + 1;
-static_assert(kBins <= 32, "bin masks are 32-bit");
+// Bins of one lane per pair with the whole window in registers
+// (k_align_lanes): windows of kWinMax+1 .. kLaneMax words have a bin per width
+// of their own; kWinLds+1 .. kWinMax share the window bin (k_align_win
+// aligns those widths of compact alphabets only); 2 .. kWinLds have a second
+// bin, where k_bin_offsets moves the few pairs that do not pay for
+// k_align_win<W>, a launch per width.
+constexpr int kWinLds = 8;
+constexpr int kLaneMax = 40;
+constexpr int kBinLane0 = kBinSeg8x2 + 1;
+constexpr int kBinLow0 = kBinLane0 + kLaneMax - kWinMax;
+constexpr int kBins = kBinLow0 + kWinLds - 1;
+static_assert(kBins <= 64, "bin masks are 64-bit");
+// The bin of a window of W words, 2..kLaneMax, on one lane per pair.
+__host__ __device__ constexpr int lane_bin(int W) {
+  return W <= kWinLds ? kBinLow0 + W - 2 : W <= kWinMax ? W : kBinLane0 + W - kWinMax - 1;
+}
+// The window width of bin b, 0 when it is not one of a single width.
+constexpr int bin_width(int b) {
+  return b >= kBinLow0    ? b - kBinLow0 + 2
+         : b >= kBinLane0 ? b - kBinLane0 + kWinMax + 1
+         : b <= kWinMax   ? b
+                          : 0;
+}
 // A kBinSeg16x2 or kBinSeg8x3 bin of fewer pairs goes to kBinSeg32, a
 // kBinSeg16x3 or x4 bin to k_align_wave<1> (k_bin_offsets; the seg2_min
 // argument of bin_pairs, NGIA_SEG2_MIN): on the heavy-tailed set at -i 90 its
@@ -34,6 +55,21 @@ static_assert(kBins <= 32, "bin masks are 32-bit");
 // log-normal set's 0.37M and 2.3M at -i 70 and 50 took 22% and 20% less
 // time.
 constexpr uint32_t kSeg2MinPairs = 32768;
+// One lane per pair is the cheapest form per word and character (its rate is
+// twice the segmented kernels') and the slowest for a single pair.  Without a
+// tuned table a bin takes it when the round's lane work would keep the device
+// busy for longer than one of the bin's pairs takes: total reference tiles
+// >= kLaneFill x the tiles of an average pair of the bin.
+constexpr uint32_t kLaneFill = 131072;
+// With a tuned table, a group of 17-40-word windows routed to several words
+// per lane takes one lane per pair from this many pairs on.
+constexpr uint32_t kLaneMinPairs = 65536;
+// A window bin of 2..kWinLds words with fewer pairs goes to its lane bin.
+constexpr uint32_t kLowLanePairs = 16384;
+// Window bins of kWinLds+1..kWinMax words that take neither: with at most
+// this many pairs among them a wavefront per pair, else the segmented
+// kernels.
+constexpr uint32_t kWavePairs = 2048;
 // The segmented bins and their (lanes per pair, words per lane).
 constexpr bool is_seg_bin(int b) { return b >= kBinSeg16 && b <= kBinSeg8x2; }
 constexpr int seg_lanes(int b) {
@@ -61,7 +97,7 @@ constexpr int kTuneClasses = NGIA_TUNE_CLASSES;
 // (17..21, 22..30, 32..45, 46..60 words) in size class k.
 constexpr int kLongGroups = NGIA_LONG_GROUPS;
 struct RouteTable {
-  uint32_t class_size[kTuneClasses];
+  uint32_t class_size[kTuneClasses];  // class_size[0] == 0: no table
   uint8_t shape[kWinMax + 1][kTuneClasses];
   uint8_t lng[kLongGroups][kTuneClasses];
 };
@@ -112,8 +148,18 @@ void pair_emit(const uint32_t* rep, uint32_t n, uint32_t bands, const uint64_t* 
 void bin_pairs(const uint2* pairs, const uint64_t* npairs, const uint32_t* len, float thr,
                uint32_t* bin_of, uint32_t* bin_cnt, uint32_t* bin_off, uint32_t* cursor,
                uint32_t* list, unsigned long long* bin_tiles, uint32_t* score, uint32_t kmax,
-               uint32_t* remap, const RouteTable& route, uint32_t seg2_min, uint32_t grid,
-               hipStream_t s);
+               uint32_t* remap, const RouteTable& route, uint32_t seg2_min, uint32_t lane_fill,
+               bool compact, uint32_t grid, hipStream_t s);
+// One lane per pair over the window bins wlo..whi of a width class (0..3:
+// 2-8, 9-16, 17-24 and 25-40 words), widest first; bin_off, bin_cnt, queue
+// (kQueueWords words a bin) and tally are indexed by bin.  max_pairs bounds
+// the pairs of the launch.
+constexpr int kLaneClasses = 4;
+constexpr int lane_class(int W) { return W <= 8 ? 0 : W <= 16 ? 1 : W <= 24 ? 2 : 3; }
+void launch_align_lanes(int cls, const AlignArgs& a, const uint2* pairs, const uint32_t* list,
+                        const uint32_t* bin_off, const uint32_t* bin_cnt, uint32_t* queue,
+                        uint32_t* score, unsigned long long* tally, uint32_t wlo, uint32_t whi,
+                        uint32_t cus, uint64_t max_pairs, hipStream_t stream);
 void plain_bin_jobs(const uint2* pairs, const uint32_t* list, const uint32_t* bin_off,
                     const uint32_t* bin_cnt, uint32_t* jobs, hipStream_t s);
 void plain_bin_scores(const uint32_t* list, const uint32_t* bin_off, const uint32_t* bin_cnt,

@@ -467,7 +467,7 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
   bin_pairs(ln.pairs.as<uint2>(), np, sv->lengths.as<uint32_t>(), sv->thr, ln.bin_of.as<uint32_t>(),
             dc->bin_cnt, dc->bin_off, dc->cursor, ln.list.as<uint32_t>(), dc->bin_tiles,
             ln.score.as<uint32_t>(), sv->ctx->wave_kmax, dc->remap, sv->ctx->route,
-            sv->ctx->seg2_min, grid, s);
+            sv->ctx->seg2_min, sv->ctx->lane_fill, false, grid, s);
   AlignArgs aa;
   aa.packed = sv->packed.as<uint32_t>();
   aa.word_off = sv->word_off.as<uint64_t>();
@@ -491,7 +491,11 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
                                         sv->ctx->prop.multiProcessorCount * seg_blocks_per_cu(G, K)),
                      s);
   }
-  for (int W = kWinMax; W >= 2; W--)
+  for (int cls = kLaneClasses - 1; cls >= 0; cls--)
+    launch_align_lanes(cls, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), dc->bin_off, dc->bin_cnt,
+                       dc->queue[0], ln.score.as<uint32_t>(), nullptr, 2, kLaneMax,
+                       (uint32_t)sv->ctx->prop.multiProcessorCount, 64ull * Q, s);
+  for (int W = kWinLds; W >= 2; W--)
     launch_align_win(W, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), &dc->bin_off[W],
                      &dc->bin_cnt[W], dc->queue[W], ln.score.as<uint32_t>(),
                      std::min<uint32_t>(Q, persistent_blocks(sv->ctx, win_lds_bytes(W))), s);

@@ -123,16 +123,20 @@ extern "C" int ngia_autotune(ngia_ctx* ctx, uint32_t identity, ngia_tune_point* 
     pairs.ensure(8ull * kTunePairs);
     list.ensure(4ull * kTuneList);
     score.ensure(4ull * kTunePairs);
-    ctr.ensure(4ull * (kQueueStride + kQueueWords));  // [0] offset, [1] count; the work queue
+    // offset and count of each bin, then the work queues: the kernels of one
+    // pair per lane take them indexed by bin, the others one bin's
+    ctr.ensure(4ull * (2 * kBins + kBins * kQueueWords));
+    fill_u32(ctr.as<uint32_t>(), 0, 2 * kBins, s);
     std::vector<uint2> hp(kTunePairs);
     std::vector<uint32_t> hl(kTuneList);
     for (uint32_t i = 0; i < kTunePairs; i++) hp[i] = make_uint2(2 * i, 2 * i + 1);
     for (uint32_t i = 0; i < kTuneList; i++) hl[i] = i % kTunePairs;
     h2d(pairs.p, hp.data(), 8ull * kTunePairs, s);
     h2d(list.p, hl.data(), 4ull * kTuneList, s);
-    uint32_t* off = ctr.as<uint32_t>();
-    uint32_t* cnt = off + 1;
-    uint32_t* work = off + kQueueStride;
+    uint32_t* offs = ctr.as<uint32_t>();
+    uint32_t* cnts = offs + kBins;
+    uint32_t* queues = cnts + kBins;
+    const uint32_t cus = (uint32_t)ctx->prop.multiProcessorCount;
     uint32_t np = 0;
     ngia::RouteTable route{}, route_compact{};
     for (int k = 0; k < kNumCounts; k++) route.class_size[k] = route_compact.class_size[k] = kTuneCounts[k];
@@ -183,14 +187,20 @@ extern "C" int ngia_autotune(ngia_ctx* ctx, uint32_t identity, ngia_tune_point* 
       AlignArgs aa = align_args(&db, thr);
       for (int k = 0; k < kNumCounts; k++) {
         const uint32_t n = kTuneCounts[k];
-        const uint32_t zero = 0;
-        h2d(off, &zero, 4, s);
+        const int bin = !dna && n < kLowLanePairs ? lane_bin(W) : W;
+        const uint32_t* off = offs + bin;
+        uint32_t* cnt = cnts + bin;
+        uint32_t* work = queues + (size_t)bin * kQueueWords;
         h2d(cnt, &n, 4, s);
         double ms[kShapes] = {0, 0, 0, 0, 0};
         for (uint32_t sh = kShapeWindow; sh < kShapes; sh++) {
           if (!shape_fits(sh, (uint32_t)W)) continue;
           ms[sh] = time_kernel(ctx, [&] {
-            if (sh == kShapeWindow)
+            if (sh == kShapeWindow && !aa.slots && (W > kWinLds || n < kLowLanePairs))
+              launch_align_lanes(lane_class(W), aa, pairs.as<uint2>(), list.as<uint32_t>(), offs, cnts,
+                                 queues, score.as<uint32_t>(), nullptr, (uint32_t)W, (uint32_t)W, cus,
+                                 n, s);
+            else if (sh == kShapeWindow)
               launch_align_win(W, aa, pairs.as<uint2>(), list.as<uint32_t>(), off, cnt, work,
                                score.as<uint32_t>(), persistent_blocks(ctx, win_lds_bytes(W, aa.slots != nullptr)), s);
             else if (sh == kShapeWave)
@@ -231,13 +241,19 @@ extern "C" int ngia_autotune(ngia_ctx* ctx, uint32_t identity, ngia_tune_point* 
       AlignArgs aa = align_args(&db, thr);
       for (int k = 0; k < kNumCounts; k++) {
         const uint32_t n = kTuneCounts[k];
-        const uint32_t zero = 0;
-        h2d(off, &zero, 4, s);
+        const int bin = lg.W <= (uint32_t)kLaneMax ? lane_bin((int)lg.W) : kBinSeg16x4;
+        const uint32_t* off = offs + bin;
+        uint32_t* cnt = cnts + bin;
+        uint32_t* work = queues + (size_t)bin * kQueueWords;
         h2d(cnt, &n, 4, s);
         double ms[kShapes] = {0, 0, 0, 0, 0};
         for (int which = 0; which < 2; which++) {
           ms[which] = time_kernel(ctx, [&] {
-            if (which == 0)
+            if (which == 0 && lg.W <= (uint32_t)kLaneMax && n >= kLaneMinPairs && ctx->lane_fill != 0xFFFFFFFFu)
+              launch_align_lanes(lane_class((int)lg.W), aa, pairs.as<uint2>(), list.as<uint32_t>(),
+                                 offs, cnts, queues, score.as<uint32_t>(), nullptr, lg.W, lg.W, cus, n,
+                                 s);
+            else if (which == 0)
               launch_align_seg(lg.g_multi, lg.k_multi, aa, pairs.as<uint2>(), list.as<uint32_t>(),
                                off, cnt, work, score.as<uint32_t>(),
                                ctx->prop.multiProcessorCount * seg_blocks_per_cu(lg.g_multi, lg.k_multi),
