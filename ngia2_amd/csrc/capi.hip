@@ -487,6 +487,28 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
   }
 }
 
+// Signatures of records [first, n) on the context stream: the four-letter walk
+// where the database's letters allow it, else a hash per window and band.
+void sketch_records(ngia_ctx* ctx, ngia_db* db, uint32_t first) {
+  const uint32_t n = db->n - first;
+  uint32_t* sig = db->sig.as<uint32_t>() + 64ull * first;
+  const uint64_t* coff = db->code_off.as<uint64_t>() + first;
+  const uint32_t* len = db->lengths.as<uint32_t>() + first;
+  if (!db->walk_code) {
+    launch_sketch(db->codes.as<uint8_t>(), coff, len, n, sig, ctx->stream);
+    return;
+  }
+  if (ctx->walk_code != db->walk_code) {
+    ctx->walk_code = 0;
+    ctx->walk_table.ensure(walk_table_bytes());
+    launch_walk_table(db->walk_code, ctx->walk_table.p, ctx->stream);
+    ctx->walk_code = db->walk_code;
+  }
+  launch_sketch_walk(db->packed.as<uint32_t>(), db->word_off.as<uint64_t>() + first,
+                     db->codes.as<uint8_t>(), coff, len, n, db->walk_code, ctx->walk_table.p,
+                     (uint32_t)ctx->prop.multiProcessorCount, sig, ctx->stream);
+}
+
 // The database's representative rows from its signatures: one block per band
 // (no scratch, no host synchronisation) up to kBucketSmallMax records, the
 // partitioned or full sort beyond (or always, under NGIA_BUCKET_WIDE).
@@ -636,7 +658,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
     }
     // the rest's sketch first, so that the context stream is busy while the
     // host enqueues the head's round
-    launch_sketch(codes, coff + h, len + h, n - h, sig + 64ull * h, s);
+    sketch_records(ctx, db, h);
     hipStream_t q = ctx->side[1];
     NGIA_HIP(hipStreamWaitEvent(q, ctx->ev[6], 0));  // after the previous step's use
     fill_u32(sig, 0xFFFFFFFFu, 64ull * h, q);
@@ -651,7 +673,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
     hr.done = ctx->head_done;
     NGIA_HIP(hipStreamWaitEvent(s, ctx->head_rows, 0));
   } else {
-    launch_sketch(codes, coff, len, n, sig, s);
+    sketch_records(ctx, db, 0);
   }
   bucket_rows(ctx, db, s);
   db->have_sig = true;
@@ -802,8 +824,7 @@ extern "C" int ngia_db_sketch(ngia_ctx* ctx, ngia_db* db) {
   return guarded(ctx, [&] {
     db->sig.ensure(256ull * std::max<uint32_t>(db->n, 1));
     NGIA_HIP(hipEventRecord(ctx->ev[6], ctx->stream));
-    launch_sketch(db->codes.as<uint8_t>(), db->code_off.as<uint64_t>(), db->lengths.as<uint32_t>(),
-                  db->n, db->sig.as<uint32_t>(), ctx->stream);
+    sketch_records(ctx, db, 0);
     NGIA_HIP(hipEventRecord(ctx->ev[7], ctx->stream));
     NGIA_HIP(hipStreamSynchronize(ctx->stream));
     ctx->timing.sketch_ms = event_ms(ctx->ev[6], ctx->ev[7]);

@@ -125,6 +125,10 @@ struct ngia_ctx {
   // env NGIA_FULL_ALPHABET=1: the window kernels keep the 16-code table even
   // for a compact alphabet
   bool full_alphabet = false;
+  // the 8-mer lists of the four-letter sketch (k_walk_table), for the letters
+  // of walk_code (0: none yet); used on the context stream only
+  ngia::DevBuf walk_table;
+  uint32_t walk_code = 0;
   ngia_timing timing{};    // device time of the last sketch / bucket / graph
   // this device's copy of the row scratch of ngia_align_noalloc (noalloc.hip)
   uint32_t* noalloc_scratch = nullptr;
@@ -169,6 +173,8 @@ struct ngia_db {
   bool compact = false;
   ngia::DevBuf slot_codes;
   uint32_t slot_code = 0;
+  // four-letter sketch: sym_code of launch_sketch_walk (0: off)
+  uint32_t walk_code = 0;
   // graph workspace
   ngia::DevBuf flags, pos, sums, jobs, ekeys, escores, ekeys_tmp, escores_tmp, fin_temp;
   ngia::DevBuf counters, cnt, keep, off, pairs, score, bin_of, list, plain_scratch, plain_jobs,
@@ -280,6 +286,27 @@ inline uint32_t persistent_blocks(const ngia_ctx* ctx, size_t lds_bytes) {
   return cu * per_cu;
 }
 
+// The letters of the four-letter sketch: the database's four most frequent
+// codes (all of them when there are no more than four).
+inline void walk_letters(ngia_db* db, uint32_t nslots, uint64_t bytes, hipStream_t s) {
+  uint32_t rare = 0;  // the slot left out
+  if (nslots > 4) {
+    DevBuf count;
+    count.ensure(8 * (kSlotCodes + 1));
+    fill_u32(count.as<uint32_t>(), 0, 2 * (kSlotCodes + 1), s);
+    launch_slot_count(db->slot_codes.as<uint8_t>(), bytes, count.as<unsigned long long>(), s);
+    unsigned long long c[kSlotCodes + 1];
+    d2h(c, count.p, sizeof(c), s);
+    NGIA_HIP(hipStreamSynchronize(s));
+    rare = 1;
+    for (uint32_t k = 2; k <= nslots; k++)
+      if (c[k] < c[rare]) rare = k;
+  }
+  db->walk_code = 0;
+  for (uint32_t k = 1, y = 0; k <= nslots; k++)
+    if (k != rare) db->walk_code |= ((db->slot_code >> (4 * (k - 1))) & 0xFu) << (4 * y++);
+}
+
 inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64_t n_words,
                const uint64_t* word_off, const uint32_t* lengths, uint32_t n) {
   std::vector<uint32_t> len_v;
@@ -318,6 +345,7 @@ inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64
   // present codes in ascending order -> 1..), a table of kSlotCodes + 1
   // entries per word in place of 16.
   db->compact = false;
+  db->walk_code = 0;
   db->slot_codes.release();
   if (acc && !(ctx->full_alphabet)) {
     DevBuf present;
@@ -340,6 +368,7 @@ inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64
       launch_code_slots(db->codes.as<uint8_t>(), acc, lut, db->slot_codes.as<uint8_t>(), s);
       db->compact = true;
       db->slot_code = slot_code;
+      if (acc >= kWalkResidues) walk_letters(db, slot, acc, s);
     }
   }
   NGIA_HIP(hipStreamSynchronize(s));

@@ -112,6 +112,36 @@ void launch_code_slots(const uint8_t* codes, uint64_t bytes, uint64_t lut, uint8
   NGIA_HIP(hipGetLastError());
 }
 
+__global__ __launch_bounds__(256) void k_slot_count(const uint32_t* __restrict__ slots, uint64_t words,
+                                                    unsigned long long* __restrict__ counts) {
+  __shared__ uint32_t acc[kSlotCodes + 1];
+  if (threadIdx.x <= kSlotCodes) acc[threadIdx.x] = 0;
+  __syncthreads();
+  uint32_t c[kSlotCodes + 1] = {};
+  for (uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < words;
+       k += (uint64_t)gridDim.x * 256) {
+    const uint32_t w = slots[k];
+    #pragma unroll
+    for (int b = 0; b < 4; b++)
+      #pragma unroll
+      for (uint32_t s = 0; s <= kSlotCodes; s++) c[s] += ((w >> (8 * b)) & 0xFFu) == s;
+  }
+  #pragma unroll
+  for (uint32_t s = 0; s <= kSlotCodes; s++) atomicAdd(&acc[s], c[s]);
+  __syncthreads();
+  if (threadIdx.x <= kSlotCodes) atomicAdd(&counts[threadIdx.x], (unsigned long long)acc[threadIdx.x]);
+}
+
+void launch_slot_count(const uint8_t* slots, uint64_t bytes, unsigned long long* counts,
+                       hipStream_t stream) {
+  const uint64_t words = bytes / 4;
+  if (words == 0) return;
+  const uint32_t grid = (uint32_t)std::min<uint64_t>((words + 255) / 256, 4096);
+  hipLaunchKernelGGL(k_slot_count, dim3(grid), dim3(256), 0, stream, (const uint32_t*)slots, words,
+                     counts);
+  NGIA_HIP(hipGetLastError());
+}
+
 // The 15 match masks of one rep word from its 4 bit planes: mask[k] has bit
 // r set iff residue r of the word has code k (buildGraph.hpp:220-225).
 __device__ inline void peq_masks(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3,

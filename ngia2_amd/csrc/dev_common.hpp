@@ -108,6 +108,12 @@ void launch_code_set(const uint8_t* codes, uint64_t bytes, uint32_t* present, hi
 // slots[k] = slot of codes[k] under lut (slot of code c in bits 4c..4c+3).
 void launch_code_slots(const uint8_t* codes, uint64_t bytes, uint64_t lut, uint8_t* slots,
                        hipStream_t stream);
+// counts[s] += the residues of slot s, s <= kSlotCodes.
+void launch_slot_count(const uint8_t* slots, uint64_t bytes, unsigned long long* counts,
+                       hipStream_t stream);
+// Databases of fewer residues keep the plain sketch: its lists take about 50 us
+// to make, the plain sketch of a million residues 20.
+constexpr uint64_t kWalkResidues = 4000000;
 void launch_codes(const uint32_t* packed, const uint64_t* word_off, const uint64_t* code_off,
                   uint32_t n, uint8_t* codes, hipStream_t stream);
 

@@ -176,7 +176,15 @@ void finalize_edges(uint64_t* keys, uint32_t* scores, uint64_t m, uint32_t n, ui
                     uint32_t* scores_tmp, void* temp, size_t temp_bytes,
                     unsigned long long* d_unique, hipStream_t s);
 
-// Sketch over byte codes (dev_sketch.hip).
+// Sketch over byte codes (dev_sketch.hip).  The walk form, for databases of at
+// most four letters beside rare others: sym_code holds the code of letter y
+// in bits 4y..; table (walk_table_bytes) is made by launch_walk_table(sym_code).
+size_t walk_table_bytes();
+void launch_walk_table(uint32_t sym_code, void* table, hipStream_t stream);
+void launch_sketch_walk(const uint32_t* packed, const uint64_t* word_off, const uint8_t* codes,
+                        const uint64_t* code_off, const uint32_t* lengths, uint32_t n,
+                        uint32_t sym_code, const void* table, uint32_t cus, uint32_t* sig,
+                        hipStream_t stream);
 void launch_sketch(const uint8_t* codes, const uint64_t* code_off, const uint32_t* lengths,
                    uint32_t n, uint32_t* sig, hipStream_t stream);
 
