@@ -149,14 +149,15 @@ void graph_plain(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
 
 // Part 1: candidates and bins (capturable: fixed grids, device-side counts),
 // on stream s; targets from db->t0 on.
-void enqueue_bins(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, hipStream_t s) {
+void enqueue_bins(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, hipStream_t s,
+                  const FastRound& fast = FastRound()) {
   const uint32_t n = db->n;
   const float thr = (float)identity / 100.0f;
   Counters* dc = db->counters.as<Counters>();
   const uint32_t* len = db->lengths.as<uint32_t>();
   fill_u32(db->counters.as<uint32_t>(), 0, sizeof(Counters) / 4, s);
   pair_count(db->rep.as<uint32_t>(), len, n, db->t0, bands, thr, db->cnt.as<uint32_t>(),
-             db->keep.as<uint64_t>(), &dc->total_cand, s);
+             db->keep.as<uint64_t>(), &dc->total_cand, s, fast);
   scan_u32(db->cnt.as<uint32_t>(), n, db->off.as<uint64_t>(), db->sums.as<uint64_t>(), s);
   pair_emit(db->rep.as<uint32_t>(), n, bands, db->keep.as<uint64_t>(), db->off.as<uint64_t>(),
             db->pairs.as<uint2>(), s);
@@ -169,15 +170,12 @@ void enqueue_bins(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
 }
 
 // Part 2: the alignment kernels of the bins in `mask` (bit b: bin b holds
-// pairs), then the passing pairs as raw edges (capturable), on stream s and,
-// unless `serial`, the side streams.
-void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, uint64_t mask,
-                   bool time_align, bool tally, hipStream_t s, bool serial = false) {
+// pairs), capturable, on stream s and, unless `serial`, the side streams.
+void enqueue_scores(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, uint64_t mask,
+                    bool time_align, bool tally, hipStream_t s, bool serial) {
   const uint32_t n = db->n;
   const float thr = (float)identity / 100.0f;
   Counters* dc = db->counters.as<Counters>();
-  const uint64_t* npairs = db->off.as<uint64_t>() + n;
-  const uint32_t grid = persistent_blocks(ctx, 0) * 4;
   const AlignArgs a0 = align_args(db, thr);
   auto holds = [&](int bin) { return ((mask >> bin) & 1u) != 0; };
   // The arguments of bin b's kernel: with the tally on, it counts the
@@ -289,8 +287,15 @@ void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
     plain_bin_scores(db->list.as<uint32_t>(), dc->bin_off, dc->bin_cnt,
                      db->plain_jobs.as<uint32_t>(), db->score.as<uint32_t>(), s);
   }
-  pairs_to_edges(db->pairs.as<uint2>(), npairs, db->score.as<uint32_t>(), db->ekeys.as<uint64_t>(),
-                 db->escores.as<uint32_t>(), &dc->ecount, grid, s);
+}
+
+// Part 2 of a graph round: the scores, then the passing pairs as raw edges.
+void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, uint64_t mask,
+                   bool time_align, bool tally, hipStream_t s, bool serial = false) {
+  enqueue_scores(ctx, db, identity, bands, mask, time_align, tally, s, serial);
+  pairs_to_edges(db->pairs.as<uint2>(), db->off.as<uint64_t>() + db->n, db->score.as<uint32_t>(),
+                 db->ekeys.as<uint64_t>(), db->escores.as<uint32_t>(),
+                 &db->counters.as<Counters>()->ecount, persistent_blocks(ctx, 0) * 4, s);
 }
 
 // Capture what fn enqueues on stream s into an instantiated graph.
@@ -313,8 +318,9 @@ hipGraphExec_t capture(hipStream_t s, F fn) {
   return ge;
 }
 
-// Workspace of one batched round over db (sized for every target).
-void ensure_batched_space(ngia_db* db, uint32_t bands) {
+// Workspace of one batched round over db up to the scores (sized for every
+// target).
+void ensure_pair_space(ngia_db* db, uint32_t bands) {
   const uint32_t n = db->n;
   const uint64_t cap = std::max<uint64_t>((uint64_t)n * bands, 1);  // distinct <= candidates <= n*bands
   db->counters.ensure(sizeof(Counters));
@@ -326,7 +332,12 @@ void ensure_batched_space(ngia_db* db, uint32_t bands) {
   db->score.ensure(4 * cap);
   db->bin_of.ensure(4 * cap);
   db->list.ensure(4 * cap);
-  ensure_edge_space(db, cap);
+}
+
+// The same with the edge list.
+void ensure_batched_space(ngia_db* db, uint32_t bands) {
+  ensure_pair_space(db, bands);
+  ensure_edge_space(db, std::max<uint64_t>((uint64_t)db->n * bands, 1));
 }
 
 // The plain bin holds only windows wider than 64 x 32 words (records of
@@ -507,6 +518,75 @@ void sketch_records(ngia_ctx* ctx, ngia_db* db, uint32_t first) {
   launch_sketch_walk(db->packed.as<uint32_t>(), db->word_off.as<uint64_t>() + first,
                      db->codes.as<uint8_t>(), coff, len, n, db->walk_code, ctx->walk_table.p,
                      (uint32_t)ctx->prop.multiProcessorCount, sig, ctx->stream);
+}
+
+// The fast mode by the batched kernels.  The reference takes the bands one by
+// one and aligns a target while it has no parent (fastClustering.hpp:249-352); a
+// target's parent depends on its own bands alone, and a representative that
+// failed once fails again.  So a round scores the distinct pairs of several
+// bands at once, and k_fast_resolve picks each target's first passing band.
+// Large databases take kFastBands bands first: targets that find a parent there
+// need no more alignments.  Returns the reference's pair count, which counts
+// the bands up to the passing one.
+constexpr uint32_t kFastBands = 8;
+constexpr uint32_t kFastSplit = 50000;
+// The database of the fast mode: db's records and rows (views) with a round
+// workspace of its own, since the pairs and scores of db's last graph stay
+// readable.
+ngia_db* fast_db(ngia_ctx* ctx, ngia_db* db) {
+  if (!db->fast) db->fast = std::make_unique<ngia_db>();
+  ngia_db* f = db->fast.get();
+  f->ctx = ctx;
+  f->n = db->n;
+  f->n_words = db->n_words;
+  f->max_len = db->max_len;
+  f->packed.view(db->packed.p, db->packed.bytes);
+  f->word_off.view(db->word_off.p, db->word_off.bytes);
+  f->lengths.view(db->lengths.p, db->lengths.bytes);
+  f->codes.view(db->codes.p, db->codes.bytes);
+  f->code_off.view(db->code_off.p, db->code_off.bytes);
+  f->rep.view(db->rep.p, db->rep.bytes);
+  f->compact = db->compact;
+  f->slot_code = db->slot_code;
+  if (db->compact)
+    f->slot_codes.view(db->slot_codes.p, db->slot_codes.bytes);
+  else
+    f->slot_codes.release();
+  return f;
+}
+
+uint64_t fast_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
+                      uint32_t* parent) {
+  hipStream_t s = ctx->stream;
+  const uint32_t n = db->n;
+  DevBuf valid, total;
+  valid.ensure(8ull * n);
+  total.ensure(8);
+  fill_u32(total.as<uint32_t>(), 0, 2, s);
+  const bool split = n >= kFastSplit && bands > 2 * kFastBands;
+  for (uint32_t lo = 0; lo < bands;) {
+    const uint32_t hi = split && lo == 0 ? kFastBands : bands;
+    FastRound f;
+    f.parent = parent;
+    f.bands = (hi < 64 ? (1ull << hi) - 1ull : ~0ull) & ~((1ull << lo) - 1ull);
+    f.valid = valid.as<uint64_t>();
+    f.last = hi == bands;
+    enqueue_bins(ctx, db, identity, bands, s, f);
+    d2h(ctx->pin + kPinCnt, db->counters.as<Counters>()->bin_cnt, 4 * kBins, s);
+    NGIA_HIP(hipStreamSynchronize(s));
+    uint64_t mask = 0;
+    for (int b = 0; b < kBins; b++)
+      if (((const uint32_t*)(ctx->pin + kPinCnt))[b]) mask |= 1ull << b;
+    if ((mask >> kBinPlain) & 1u) ensure_plain_bin_space(db, bands);
+    enqueue_scores(ctx, db, identity, bands, mask, false, false, s, false);
+    fast_resolve(n, db->off.as<uint64_t>(), db->pairs.as<uint2>(), db->score.as<uint32_t>(),
+                 db->keep.as<uint64_t>(), f, total.as<unsigned long long>(), s);
+    lo = hi;
+  }
+  unsigned long long t = 0;
+  d2h(&t, total.p, 8, s);
+  NGIA_HIP(hipStreamSynchronize(s));
+  return t;
 }
 
 // The database's representative rows from its signatures: one block per band
@@ -1040,14 +1120,38 @@ extern "C" int ngia_db_fast(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint3
     DevBuf parent;
     parent.ensure(4ull * std::max<uint32_t>(n, 1));
     fill_u32(parent.as<uint32_t>(), 0xFFFFFFFFu, n, ctx->stream);
-    ngia_graph_stats st{};
-    graph_plain(ctx, db, identity, bands, &st, parent.as<uint32_t>());
+    if (n == 0) {
+      if (total_pairs) *total_pairs = 0;
+      return NGIA_OK;
+    }
+    // The pair lists take 1.3 KiB per record at 64 bands; without the memory
+    // (or past 2^32 pairs) the bands run one by one.
+    bool batched = (uint64_t)n * bands < (1ull << 32);
+    uint64_t total = 0;
+    if (batched) {
+      try {
+        ensure_pair_space(fast_db(ctx, db), bands);
+      } catch (const HipError& e) {
+        if (e.code != NGIA_ERR_NOMEM) throw;
+        (void)hipGetLastError();
+        db->fast.reset();
+        batched = false;
+      }
+    }
+    db->have_bins = false;
+    if (batched) {
+      total = fast_batched(ctx, db->fast.get(), identity, bands, parent.as<uint32_t>());
+    } else {
+      ngia_graph_stats st{};
+      graph_plain(ctx, db, identity, bands, &st, parent.as<uint32_t>());
+      total = st.total_pairs;
+    }
     std::vector<uint32_t> par(n);
     d2h(par.data(), parent.p, 4ull * n, ctx->stream);
     NGIA_HIP(hipStreamSynchronize(ctx->stream));
     // fastClustering.hpp:338-347: parent[i] < i, resolve in ascending order
     for (uint32_t i = 0; i < n; i++) cluster[i] = par[i] == 0xFFFFFFFFu ? i : cluster[par[i]];
-    if (total_pairs) *total_pairs = st.total_pairs;
+    if (total_pairs) *total_pairs = total;
     return NGIA_OK;
   });
 }

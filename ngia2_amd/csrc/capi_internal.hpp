@@ -200,6 +200,8 @@ struct ngia_db {
   // this database's records, codes and signatures and its own rows and
   // round workspace
   std::unique_ptr<ngia_db> head;
+  // the fast mode's round workspace (ngia_db_fast), with views likewise
+  std::unique_ptr<ngia_db> fast;
   // (head only) its records' sketch in chunks of positions: (record, first
   // position) per chunk
   ngia::DevBuf sketch_chunks;
@@ -318,6 +320,7 @@ inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64
   validate_records(packed, n_words, word_off, lengths, n, &db->max_len);
   db->host_len.assign(lengths, lengths + n);
   db->head.reset();
+  db->fast.reset();
   db->n = n;
   db->n_words = n_words;
   hipStream_t s = ctx->stream;

@@ -212,6 +212,48 @@ void fast_apply(const uint32_t* jobs, uint32_t count, uint32_t* parent, hipStrea
   NGIA_HIP(hipGetLastError());
 }
 
+// One thread per target that has no parent yet: its kept pairs of the round in
+// band order; the first that passes gives its parent.  The reference aligns the
+// target in every band up to that one (in all of them when none passes):
+// *total counts those bands.
+__global__ __launch_bounds__(256) void k_fast_resolve(uint32_t n, const uint64_t* __restrict__ off,
+                                                      const uint2* __restrict__ pairs,
+                                                      const uint32_t* __restrict__ score,
+                                                      const uint64_t* __restrict__ keep,
+                                                      FastRound fast,
+                                                      unsigned long long* __restrict__ total) {
+  __shared__ unsigned long long sum;
+  if (threadIdx.x == 0) sum = 0;
+  __syncthreads();
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  uint32_t aligned = 0;
+  if (i < n && fast.parent[i] == 0xFFFFFFFFu) {
+    uint64_t left = keep[i];
+    const uint64_t valid = fast.valid[i];
+    bool pass = false;
+    for (uint64_t p = off[i]; left; p++, left &= left - 1) {
+      if (!score[p]) continue;
+      fast.parent[i] = pairs[p].x;
+      const uint32_t b = (uint32_t)__builtin_ctzll(left);
+      aligned = (uint32_t)__builtin_popcountll(valid & ((2ull << b) - 1ull));
+      pass = true;
+      break;
+    }
+    if (!pass && fast.last) aligned = (uint32_t)__builtin_popcountll(valid);
+  }
+  if (aligned) atomicAdd(&sum, (unsigned long long)aligned);
+  __syncthreads();
+  if (threadIdx.x == 0 && sum) atomicAdd(total, sum);
+}
+
+void fast_resolve(uint32_t n, const uint64_t* off, const uint2* pairs, const uint32_t* score,
+                  const uint64_t* keep, const FastRound& fast, unsigned long long* total,
+                  hipStream_t s) {
+  hipLaunchKernelGGL(k_fast_resolve, dim3(grid_for(n, 256)), dim3(256), 0, s, n, off, pairs, score,
+                     keep, fast, total);
+  NGIA_HIP(hipGetLastError());
+}
+
 // ------------------------------------------------------------- batched form
 // Count pass: a block takes 64 consecutive targets.  The 64 x 64 tile
 // rep[b][i0..i0+63] is read row by row (coalesced) into LDS; each wavefront
@@ -233,7 +275,7 @@ __device__ inline void load_rep_tile(const uint32_t* __restrict__ rep, uint32_t 
 __global__ __launch_bounds__(256) void k_pair_count(const uint32_t* __restrict__ rep,
                                                     const uint32_t* __restrict__ len, uint32_t n,
                                                     uint32_t t0, uint32_t bands, float thr,
-                                                    uint32_t* __restrict__ cnt,
+                                                    FastRound fast, uint32_t* __restrict__ cnt,
                                                     uint64_t* __restrict__ keep_out,
                                                     unsigned long long* __restrict__ total) {
   __shared__ uint32_t tile[64][65];
@@ -262,8 +304,10 @@ __global__ __launch_bounds__(256) void k_pair_count(const uint32_t* __restrict__
     const uint32_t i = i0 + t;
     if (i >= n) break;
     const uint32_t r = tile[lane][t];
-    // is_job: r != i and (float)len[i] >= (float)len[r] * thr
-    const bool valid = ((need >> tt) & 1u) && (float)li[tt] >= (float)lr[tt] * thr;
+    // is_job: r != i and (float)len[i] >= (float)len[r] * thr; the fast mode has
+    // no length test (fastClustering.hpp:256-258)
+    const bool valid =
+        ((need >> tt) & 1u) && (fast.parent || (float)li[tt] >= (float)lr[tt] * thr);
     const uint64_t vm = __builtin_amdgcn_ballot_w64(valid);
     uint64_t mask = vm, keep = 0;
     while (mask) {
@@ -271,6 +315,10 @@ __global__ __launch_bounds__(256) void k_pair_count(const uint32_t* __restrict__
       const uint32_t r0 = __builtin_amdgcn_readlane(r, b0);
       keep |= 1ull << b0;
       mask &= ~__builtin_amdgcn_ballot_w64(valid && r == r0);
+    }
+    if (fast.parent) {
+      keep = fast.parent[i] == 0xFFFFFFFFu ? keep & fast.bands : 0ull;
+      if (lane == 0) fast.valid[i] = vm;
     }
     if (lane == 0) {
       cnt[i] = (uint32_t)__builtin_popcountll(keep);
@@ -310,9 +358,10 @@ __global__ __launch_bounds__(256) void k_pair_emit(const uint32_t* __restrict__ 
 }
 
 void pair_count(const uint32_t* rep, const uint32_t* len, uint32_t n, uint32_t t0, uint32_t bands,
-                float thr, uint32_t* cnt, uint64_t* keep, unsigned long long* total, hipStream_t s) {
+                float thr, uint32_t* cnt, uint64_t* keep, unsigned long long* total, hipStream_t s,
+                const FastRound& fast) {
   hipLaunchKernelGGL(k_pair_count, dim3((n + 63) / 64), dim3(256), 0, s, rep, len, n, t0, bands,
-                     thr, cnt, keep, total);
+                     thr, fast, cnt, keep, total);
   NGIA_HIP(hipGetLastError());
 }
 

@@ -136,13 +136,27 @@ void jobs_to_edges(const uint32_t* jobs, uint32_t count, uint64_t* ekeys, uint32
                    unsigned long long* ecount, hipStream_t s);
 void fast_apply(const uint32_t* jobs, uint32_t count, uint32_t* parent, hipStream_t s);
 
+// A round of the batched fast mode: targets without a parent yet, the pairs
+// whose representative first appears in the bands of `bands`; valid receives
+// every band with a representative; last: no round follows.
+struct FastRound {
+  uint32_t* parent = nullptr;  // nullptr: not the fast mode
+  uint64_t bands = 0;
+  uint64_t* valid = nullptr;
+  bool last = false;
+};
+void fast_resolve(uint32_t n, const uint64_t* off, const uint2* pairs, const uint32_t* score,
+                  const uint64_t* keep, const FastRound& fast, unsigned long long* total,
+                  hipStream_t s);
+
 // Batched form.
 // Candidates: the count pass writes cnt[i] (distinct pairs of target i),
 // keep[i] (the bands whose representatives are kept) and adds the count with
 // duplicates to *total; after cnt is scanned into off, the emit pass writes
 // the pairs grouped by target, in target order.  Targets below t0 get none.
 void pair_count(const uint32_t* rep, const uint32_t* len, uint32_t n, uint32_t t0, uint32_t bands,
-                float thr, uint32_t* cnt, uint64_t* keep, unsigned long long* total, hipStream_t s);
+                float thr, uint32_t* cnt, uint64_t* keep, unsigned long long* total, hipStream_t s,
+                const FastRound& fast = FastRound());
 void pair_emit(const uint32_t* rep, uint32_t n, uint32_t bands, const uint64_t* keep,
                const uint64_t* off, uint2* pairs, hipStream_t s);
 void bin_pairs(const uint2* pairs, const uint64_t* npairs, const uint32_t* len, float thr,
