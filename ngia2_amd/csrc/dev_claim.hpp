@@ -25,10 +25,12 @@ __device__ inline bool cannot_pass(uint32_t lcs_now, uint32_t done, uint32_t R, 
 // wave still gets many claims and the queue drains evenly: count / (16
 // waves' worth), between `lo` and `hi` (lo >= the most items handed out at
 // once).  The wave starts on the slice of its XCD (kQueueSlices slices, one
-// counter each); when a claim comes back empty it reads every slice's
-// counter and moves to the next slice with items left, and with none left
-// the queue is drained.  All members are wave-uniform; take() is called by
-// the whole wave at a convergent point.
+// counter each) with the chunk of its number there, which needs no claim; the
+// counters hand out what follows the waves' first chunks, so a queue that
+// those cover is never touched.  When a slice is exhausted the wave reads the
+// counters of the slices that have more and moves to the next one with items
+// left; with none left the queue is drained.  All members are wave-uniform;
+// take() is called by the whole wave at a convergent point.
 struct WaveClaim {
   uint32_t next = 0, end = 0, chunk = 1, count, slice;
   bool drained = false;
@@ -36,6 +38,17 @@ struct WaveClaim {
     const uint32_t per = count / (gridDim.x * (blockDim.x / 64u) * 16u);
     chunk = per < lo ? lo : per > hi ? hi : per;
     slice = blockIdx.x % kQueueSlices;
+    const uint32_t s0 = slice_lo(slice), len = slice_lo(slice + 1) - s0;
+    const uint32_t first = blockIdx.x / kQueueSlices * chunk;
+    if (first < len) {
+      next = s0 + first;
+      end = s0 + (len - first < chunk ? len : first + chunk);
+    }
+  }
+  // Items of slice s that its waves take without a claim (blocks of one
+  // wavefront).
+  __device__ uint32_t slice_first(uint32_t s) const {
+    return (gridDim.x - s + kQueueSlices - 1) / kQueueSlices * chunk;
   }
   __device__ uint32_t slice_lo(uint32_t s) const {
     return (uint32_t)((uint64_t)count * s / kQueueSlices);
@@ -51,9 +64,12 @@ struct WaveClaim {
     while (given < n && !drained) {
       if (next == end) {
         const uint32_t lo = slice_lo(slice), len = slice_lo(slice + 1) - lo;
-        uint32_t b = 0;
-        if (lane == 0) b = atomicAdd(queue + slice * kQueueStride, chunk);
-        b = __builtin_amdgcn_readfirstlane(b);
+        uint32_t b = slice_first(slice);
+        if (b < len) {
+          uint32_t a = 0;
+          if (lane == 0) a = atomicAdd(queue + slice * kQueueStride, chunk);
+          b += __builtin_amdgcn_readfirstlane(a);
+        }
         if (b < len) {
           next = lo + b;
           end = lo + (len - b < chunk ? len : b + chunk);
@@ -63,9 +79,10 @@ struct WaveClaim {
           // stays so)
           bool left = false;
           if (lane < kQueueSlices) {
-            const uint32_t c = __hip_atomic_load(queue + lane * kQueueStride, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT);
-            left = c < slice_lo(lane + 1) - slice_lo(lane);
+            const uint32_t f = slice_first(lane), n = slice_lo(lane + 1) - slice_lo(lane);
+            if (f < n)
+              left = __hip_atomic_load(queue + lane * kQueueStride, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT) < n - f;
           }
           const uint32_t m = (uint32_t)__builtin_amdgcn_ballot_w64(left);
           if (m == 0) {

@@ -465,7 +465,8 @@ __global__ __launch_bounds__(64) void k_bin_offsets(uint32_t* __restrict__ bin_c
     for (int W = kWinLds + 1; W <= kLaneMax; W++) total += tiles[lane_bin(W)];
     const bool lanes_off = lane_fill == 0xFFFFFFFFu;
     auto lanes_pay = [&](uint32_t c, unsigned long long t) {
-      return !lanes_off && total * c >= (unsigned long long)lane_fill * t;
+      const unsigned long long few = (unsigned long long)kLaneTiles * c;
+      return !lanes_off && (t <= few || total * c >= (unsigned long long)lane_fill * (t - few));
     };
     // Window bins: the tuned shape; without a table, kWinLds+1..kWinMax words
     // by lanes_pay, and where it does not pay a wavefront or a segment per

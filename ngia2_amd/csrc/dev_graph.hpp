@@ -55,12 +55,19 @@ constexpr int bin_width(int b) {
 // log-normal set's 0.37M and 2.3M at -i 70 and 50 took 22% and 20% less
 // time.
 constexpr uint32_t kSeg2MinPairs = 32768;
-// One lane per pair is the cheapest form per word and character (its rate is
-// twice the segmented kernels') and the slowest for a single pair.  Without a
-// tuned table a bin takes it when the round's lane work would keep the device
-// busy for longer than one of the bin's pairs takes: total reference tiles
-// >= kLaneFill x the tiles of an average pair of the bin.
-constexpr uint32_t kLaneFill = 131072;
+// One lane per pair is the cheapest form per word and character (about twice
+// the segmented kernels' rate) and the slowest for a single pair: 14 ns per word
+// and character, while the whole device does 64 x 1,024 such steps in 9 ns.
+// Without a tuned table a bin takes it when a pair is short (at most
+// kLaneTiles reference tiles on average) or the round's lane work keeps the
+// device busy for about 2.5 times what one of the bin's pairs takes: total
+// tiles >= kLaneFill x (an average pair's tiles - kLaneTiles).  Measured, the
+// graph at kLaneFill 131,072 / 200,000 / 300,000: 10,000 proteins at -i 70 0.29
+// / 0.27 / 0.28 ms, 100,000 at -i 70 0.55 / 0.61 / 0.67, 500,000 at -i 70 2.08 /
+// 1.57 / 1.67, 300,000 at -i 60 1.50 / 1.29 / 1.36; kLaneTiles 0 / 100 at
+// 300,000: 50,000 of 50-1,000 residues at -i 60 0.59 / 0.48.
+constexpr uint32_t kLaneTiles = 80;
+constexpr uint32_t kLaneFill = 262144;
 // With a tuned table, a group of 17-40-word windows routed to several words
 // per lane takes one lane per pair from this many pairs on.
 constexpr uint32_t kLaneMinPairs = 65536;
@@ -166,10 +173,12 @@ void bin_pairs(const uint2* pairs, const uint64_t* npairs, const uint32_t* len, 
                bool compact, uint32_t grid, hipStream_t s);
 // One lane per pair over the window bins wlo..whi of a width class (0..3:
 // 2-8, 9-16, 17-24 and 25-40 words), widest first; bin_off, bin_cnt, queue
-// (kQueueWords words a bin) and tally are indexed by bin.  max_pairs bounds
-// the pairs of the launch.
+// (kQueueWords words a bin; the launch uses that of whi) and tally are
+// indexed by bin.  max_pairs bounds the pairs of the launch.
 constexpr int kLaneClasses = 4;
 constexpr int lane_class(int W) { return W <= 8 ? 0 : W <= 16 ? 1 : W <= 24 ? 2 : 3; }
+constexpr int lane_class_min(int cls) { return cls == 0 ? 2 : 8 * cls + 1; }
+constexpr int lane_class_max(int cls) { return cls == 3 ? kLaneMax : 8 * cls + 8; }
 void launch_align_lanes(int cls, const AlignArgs& a, const uint2* pairs, const uint32_t* list,
                         const uint32_t* bin_off, const uint32_t* bin_cnt, uint32_t* queue,
                         uint32_t* score, unsigned long long* tally, uint32_t wlo, uint32_t whi,

@@ -493,7 +493,8 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
   }
   for (int cls = kLaneClasses - 1; cls >= 0; cls--)
     launch_align_lanes(cls, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), dc->bin_off, dc->bin_cnt,
-                       dc->queue[0], ln.score.as<uint32_t>(), nullptr, 2, kLaneMax,
+                       dc->queue[0], ln.score.as<uint32_t>(), nullptr, lane_class_min(cls),
+                       lane_class_max(cls),
                        (uint32_t)sv->ctx->prop.multiProcessorCount, 64ull * Q, s);
   for (int W = kWinLds; W >= 2; W--)
     launch_align_win(W, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), &dc->bin_off[W],
