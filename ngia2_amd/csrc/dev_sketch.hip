@@ -504,24 +504,46 @@ __global__ __launch_bounds__(256) void k_bucket_rep_wide(const uint64_t* __restr
 
 // ------------------------------------------------ partitioned bucketing
 // Only equality of signatures within a band matters, so the full sort above
-// is replaced, for n <= kPartMaxN, by a partition and a sort in LDS:
-//  1. every (band b, record i) gets h = mix(sig), a bijection of the 32-bit
-//     signature that spreads its bits (minhash values crowd near 0), the
-//     16-bit key (b << pb | top pb bits of h) and the value (h << 32 | i);
-//  2. a stable radix sort on the key's low pb bits groups each band's
-//     elements into 2^pb partitions, each still in ascending i (the input is
-//     band-major, so the stable sort keeps each (bucket, band) group
-//     contiguous without sorting the band bits);
-//  3. one block per partition sorts it by h in LDS (stable), and every
-//     element equal to its predecessor gets rep[b][i] = that predecessor's i
-//     -- the element before it in the reference's stable (sig, i) order.
-// pb = 8 (one radix pass, partitions average n/256) up to kPart8MaxN records,
-// else pb = 10 (two passes, partitions average n/1024).  A partition larger
-// than a block's capacity (heavily repeated signatures) is counted; the host
-// then redoes the whole bucketing with the full sort.
-constexpr int kPartBlock = 512;  // threads per partition sort
-constexpr uint32_t kPart8MaxN = 1000000;  // partitions average <= 3907, capacity 8192
-constexpr uint32_t kPartMaxN = 2800000;   // partitions average <= 2735, capacity 4096
+// is replaced, for n <= kPartMaxN, by a partition and hash chains in LDS:
+//  1. k_mix_columns: h = mix(sig), a bijection of the 32-bit signature that
+//     spreads its bits (minhash values crowd near 0), band-major, and the rows
+//     of bucket heads (their own index), which most elements are: k_part_chain
+//     writes at random places, the others' rows only;
+//  2. k_part_scatter: each band's (h, i) into 2^pb partitions by the top pb bits
+//     of h, in no order.  A partition has room for kPartCap elements, twice or
+//     more its average (pb is chosen for an average of 1,024 to 2,048);
+//  3. k_part_chain: one block per partition hangs its elements into chains by
+//     the low bits of h; each element walks its chain for the largest index
+//     below its own with the same h, which is its predecessor in the
+//     reference's stable (sig, i) order.
+//  4. k_part_long: the partitions that outgrew their room (heavily repeated
+//     signatures), from the column.
+// A partition with more distinct values than it has room for is counted; the
+// host then redoes the whole bucketing with the full sort.
+// Bound: memory for the first two, 4 + 8 and 4 + 8 bytes an element; the LDS's
+// latency down the chains and the scattered 4-byte row writes for the third.
+// Bands stay on one XCD (block b takes bands of XCD b mod 8), so that the short
+// runs a partition and a row are written in meet in one L2.
+// All 64 bands, against a radix sort by partition and a block sort for each:
+//   records   20,000  50,000  100,000  300,000    1M     2M
+//   before      395     423      472      694   1434   3379 us
+//   now          47      68       95      273    861   1865 us
+// (1M: k_mix_columns 155, k_part_scatter 220, k_part_chain 450 us), and with one
+// signature set repeated 6,000 times 526 -> 196 us at 50,000 and 3950 -> 1703
+// us at 1M records.
+constexpr uint32_t kPartMaxN = 2800000;
+constexpr uint32_t kPartCap = 4096;
+constexpr uint32_t kScatterTile = 8192, kScatterThreads = 1024;
+constexpr uint32_t kPartMaxBits = 11;
+
+// Partition bits for n records.
+constexpr uint32_t part_bits(uint32_t n) {
+  uint32_t pb = 0;
+  while (pb < kPartMaxBits && (n >> pb) > kPartCap / 2) pb++;
+  return pb;
+}
+static_assert(part_bits(kPartMaxN) <= kPartMaxBits && (kPartMaxN >> part_bits(kPartMaxN)) <= kPartCap / 2,
+              "partitions too large at the largest n");
 
 __device__ inline uint32_t sig_mix(uint32_t x) {
   x *= 0x9E3779B1u;  // odd multiplier: a bijection mod 2^32
@@ -531,9 +553,9 @@ __device__ inline uint32_t sig_mix(uint32_t x) {
   return x;
 }
 
-__global__ __launch_bounds__(256) void k_part_keys(const uint32_t* __restrict__ sig, uint32_t n,
-                                                   uint32_t pb, uint16_t* __restrict__ keys,
-                                                   uint64_t* __restrict__ vals) {
+__global__ __launch_bounds__(256) void k_mix_columns(const uint32_t* __restrict__ sig, uint32_t n,
+                                                     uint32_t* __restrict__ col,
+                                                     uint32_t* __restrict__ rep) {
   // 64 records x 64 bands through LDS, as in k_bucket_keys
   __shared__ uint32_t tile[64][65];
   const uint32_t i0 = blockIdx.x * 64;
@@ -545,139 +567,312 @@ __global__ __launch_bounds__(256) void k_part_keys(const uint32_t* __restrict__ 
   __syncthreads();
   for (uint32_t e = t; e < 64 * 64; e += 256) {
     const uint32_t b = e >> 6, si = e & 63;
-    const uint32_t i = i0 + si;
-    if (i < n) {
-      const uint32_t h = sig_mix(tile[si][b]);
-      keys[(uint64_t)b * n + i] = (uint16_t)((b << pb) | (h >> (32 - pb)));
-      vals[(uint64_t)b * n + i] = ((uint64_t)h << 32) | i;
+    if (i0 + si < n) {
+      col[(uint64_t)b * n + i0 + si] = sig_mix(tile[si][b]);
+      rep[(uint64_t)b * n + i0 + si] = i0 + si;
     }
   }
 }
 
-// start[k], end[k]: the sorted range of partition k (left 0, 0 when empty).
-// Eight keys per thread from one 16-byte load (m is a multiple of 64), the
-// neighbours across the group boundary from the adjacent groups.
-__global__ __launch_bounds__(256) void k_part_bounds(const uint16_t* __restrict__ keys, uint64_t m,
-                                                     uint32_t* __restrict__ start,
-                                                     uint32_t* __restrict__ end) {
-  const uint64_t groups = m / 8;
-  for (uint64_t g = (uint64_t)blockIdx.x * 256 + threadIdx.x; g < groups;
-       g += (uint64_t)gridDim.x * 256) {
-    const uint64_t p0 = 8 * g;
-    const uint4 w = *(const uint4*)(keys + p0);
-    uint32_t k[8] = {w.x & 0xFFFFu, w.x >> 16, w.y & 0xFFFFu, w.y >> 16,
-                     w.z & 0xFFFFu, w.z >> 16, w.w & 0xFFFFu, w.w >> 16};
-    // keys are 16-bit: 0x10000 differs from every key
-    uint32_t prev = p0 ? keys[p0 - 1] : 0x10000u;
-    const uint32_t after = p0 + 8 < m ? keys[p0 + 8] : 0x10000u;
-    #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const uint32_t next = j < 7 ? k[j + 1] : after;
-      if (prev != k[j]) start[k[j]] = (uint32_t)(p0 + j);
-      if (next != k[j]) end[k[j]] = (uint32_t)(p0 + j + 1);
-      prev = k[j];
-    }
-  }
+// The band and the place within the band of a block, bands spread over the
+// XCDs: blocks of bands 8x .. 8x + 7 run on XCD x, band by band.
+__device__ inline void band_block(uint32_t per_band, uint32_t* band, uint32_t* at) {
+  const uint32_t q = blockIdx.x / 8;
+  *band = (blockIdx.x % 8) * 8 + q / per_band;
+  *at = q % per_band;
 }
 
-// One partition sorted in LDS, stably, by the low kLowBits bits of h alone
-// (ITEMS elements per thread in the blocked arrangement): elements of equal h
-// then sit in one run of equal low bits, in ascending i, possibly between
-// elements of other values with the same low bits (about one per run at the
-// partitions' sizes, since h mixes the signature's bits).  An element's
-// predecessor -- the element before it in the (h, i) order -- is the nearest
-// earlier element of its run with the same h, found by a scan backwards
-// through the sorted keys in LDS.  The partition's elements share the top pb
-// bits of h; sorting 12 of the other 32 - pb bits takes half the passes.  With
-// the scan the bucketing of a million records went from 1.44 to 1.40 ms
-// (log-normal lengths) and to 1.43 ms (heavy-tailed); the kernel's loads and
-// scattered row writes stay as they were.
-constexpr uint32_t kLowBits = 12, kLowMask = (1u << kLowBits) - 1u;
-template <int BS, int ITEMS>
-__device__ inline void part_sort_tier(const uint64_t* __restrict__ v, uint32_t cnt, uint64_t row,
-                                      uint32_t* __restrict__ rep, void* storage_raw) {
-  using Sort = rocprim::block_radix_sort<uint32_t, BS, ITEMS, uint32_t>;
-  auto& storage = *reinterpret_cast<typename Sort::storage_type*>(storage_raw);
-  const uint32_t t = threadIdx.x;
-  uint32_t key[ITEMS], val[ITEMS];
+// One tile of a band's column: counted by partition, given room by one atomic
+// per partition, ordered by partition in LDS, written as runs.
+__global__ __launch_bounds__(kScatterThreads) void k_part_scatter(const uint32_t* __restrict__ col, uint32_t n,
+                                                      uint32_t pb, uint32_t tiles,
+                                                      uint32_t* __restrict__ cursor,
+                                                      uint2* __restrict__ entries) {
+  __shared__ __align__(16) uint2 stage[kScatterTile];
+  __shared__ uint32_t cnt[1u << kPartMaxBits], base[1u << kPartMaxBits];
+  __shared__ uint32_t wsum[kScatterThreads / 64];
+  constexpr uint32_t kPer = (1u << kPartMaxBits) / kScatterThreads;  // partitions a thread
+  constexpr uint32_t kItems = kScatterTile / kScatterThreads;
+  const uint32_t t = threadIdx.x, parts = 1u << pb;
+  uint32_t band, tile;
+  band_block(tiles, &band, &tile);
+  const uint32_t i0 = tile * kScatterTile;
+  const uint32_t m = n - i0 < kScatterTile ? n - i0 : kScatterTile;
+  for (uint32_t k = t; k < parts; k += kScatterThreads) cnt[k] = 0;
+  __syncthreads();
+  uint32_t h[kItems], r[kItems];
   #pragma unroll
-  for (int j = 0; j < ITEMS; j++) {
-    const uint32_t q = t * ITEMS + j;  // blocked: input order = ascending i
-    if (q < cnt) {
-      const uint64_t x = v[q];
-      key[j] = (uint32_t)(x >> 32);
-      val[j] = (uint32_t)x;
-    } else {  // padding: the largest low bits, and after every element of them (stable)
-      key[j] = 0xFFFFFFFFu;
-      val[j] = 0xFFFFFFFFu;
-    }
+  for (uint32_t j = 0; j < kItems; j++) {
+    const uint32_t q = j * kScatterThreads + t;
+    h[j] = q < m ? col[(uint64_t)band * n + i0 + q] : 0u;
   }
-  Sort().sort(key, val, storage, 0, kLowBits);
-  __syncthreads();  // the sort's storage now holds the sorted keys and values
-  uint32_t* sk = reinterpret_cast<uint32_t*>(storage_raw);
-  uint32_t* sv = sk + BS * ITEMS;
+  // pb = 0: a shift by 32 would be none
+  auto part_of = [&](uint32_t x) { return (uint32_t)(((uint64_t)x << pb) >> 32); };
   #pragma unroll
-  for (int j = 0; j < ITEMS; j++) {
-    sk[t * ITEMS + j] = key[j];
-    sv[t * ITEMS + j] = val[j];
+  for (uint32_t j = 0; j < kItems; j++)
+    if (j * kScatterThreads + t < m) r[j] = atomicAdd(&cnt[part_of(h[j])], 1u);
+  __syncthreads();
+  // exclusive prefix over the partitions
+  const uint32_t k0 = kPer * t;
+  uint32_t c[kPer], sum = 0;
+  #pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) {
+    c[k] = k0 + k < parts ? cnt[k0 + k] : 0u;
+    sum += c[k];
+  }
+  uint32_t x = sum;
+  #pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o);
+    if ((t & 63) >= (uint32_t)o) x += y;
+  }
+  if ((t & 63) == 63) wsum[t >> 6] = x;
+  __syncthreads();
+  uint32_t run = x - sum;
+  for (uint32_t w = 0; w < t >> 6; w++) run += wsum[w];
+  #pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) {
+    if (k0 + k >= parts) break;
+    const uint32_t g = c[k] ? atomicAdd(&cursor[(band << pb) + k0 + k], c[k]) : 0u;
+    cnt[k0 + k] = run;
+    base[k0 + k] = g - run;  // place in the partition of the tile's element s: base + s
+    run += c[k];
   }
   __syncthreads();
-  // The element just before is in registers (or, for the thread's first
-  // item, the previous thread's last); only a run holding other values of
-  // the same low bits between equal ones needs the scan through LDS.
-  uint32_t pk = t ? sk[t * ITEMS - 1] : 0u, pv = t ? sv[t * ITEMS - 1] : 0u;
   #pragma unroll
-  for (int j = 0; j < ITEMS; j++) {
-    const uint32_t q = t * ITEMS + j;
-    if (q >= 1 && q < cnt && ((pk ^ key[j]) & kLowMask) == 0) {
-      if (pk == key[j]) {
-        rep[row + val[j]] = pv;
-      } else {
-        for (uint32_t r = q - 1; r-- > 0;) {
-          const uint32_t kr = sk[r];
-          if ((kr & kLowMask) != (key[j] & kLowMask)) break;
-          if (kr == key[j]) {
-            rep[row + val[j]] = sv[r];
-            break;
-          }
-        }
-      }
-    }
-    pk = key[j];
-    pv = val[j];
+  for (uint32_t j = 0; j < kItems; j++)
+    if (j * kScatterThreads + t < m) stage[cnt[part_of(h[j])] + r[j]] = make_uint2(h[j], i0 + j * kScatterThreads + t);
+  __syncthreads();
+  for (uint32_t q = t; q < m; q += kScatterThreads) {
+    const uint2 e = stage[q];
+    const uint32_t k = part_of(e.x), at = base[k] + q;
+    if (at < kPartCap) entries[(uint64_t)((band << pb) + k) * kPartCap + at] = e;
   }
 }
 
-// One block of BS threads per partition, sorted at the smallest of three
-// capacities (BS x I1, I2 or I3 items) that holds it: the sort's cost follows
-// its capacity, and most partitions sit near the average, under the largest.
-// The LDS holds the sort's storage, then the sorted keys and values.
-template <int BS, int I1, int I2, int I3>
-__global__ __launch_bounds__(BS) void k_part_local(const uint64_t* __restrict__ vals,
-                                                    const uint32_t* __restrict__ start,
-                                                    const uint32_t* __restrict__ end, uint32_t n,
+// The rows of `cnt` elements (h, i) in LDS, in any order: chained through next[]
+// by the low bits of h (a chain ends at element kPartCap, which matches
+// nothing and follows itself), a row written for every
+// element with a predecessor.  A walk takes kChainMax steps at most; past that
+// *many is set and the rows are left to the sort.
+constexpr uint32_t kChainMax = 96;
+// A thread walks the chains of all its elements in step: one after another, each
+// would wait for the longest chain of its wavefront.
+constexpr uint32_t kHeads = 2048;
+template <int BS, int kItems>
+__device__ inline void chain_rows(uint2* el, uint16_t* next, uint32_t* head, uint32_t cnt,
+                                  uint32_t* __restrict__ rep, uint32_t* many) {
+  const uint32_t t = threadIdx.x;
+  #pragma unroll
+  for (uint32_t k = 0; k < kHeads / BS; k++) head[t + k * BS] = kPartCap;
+  if (t == 0) {
+    el[kPartCap] = make_uint2(~0u, ~0u);
+    next[kPartCap] = (uint16_t)kPartCap;
+  }
+  __syncthreads();
+  uint32_t h[kItems], i[kItems], f[kItems], best[kItems];  // best: the predecessor's index + 1
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    const uint32_t e = t + j * BS;
+    const uint2 x = el[e < cnt ? e : kPartCap];
+    h[j] = x.x;
+    i[j] = x.y;
+    best[j] = 0;
+  }
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    const uint32_t e = t + j * BS;
+    if (e < cnt) next[e] = (uint16_t)atomicExch(&head[h[j] % kHeads], e);
+  }
+  __syncthreads();
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) f[j] = t + j * BS < cnt ? head[h[j] % kHeads] : kPartCap;
+  bool more = true;
+  for (uint32_t steps = 0; more && steps < kChainMax; steps++) {
+    uint2 x[kItems];
+    #pragma unroll
+    for (int j = 0; j < kItems; j++) {
+      x[j] = el[f[j]];
+      f[j] = next[f[j]];
+    }
+    more = false;
+    #pragma unroll
+    for (int j = 0; j < kItems; j++) {
+      if (x[j].x == h[j] && x[j].y < i[j] && x[j].y + 1 > best[j]) best[j] = x[j].y + 1;
+      more = more || f[j] != kPartCap;
+    }
+  }
+  if (more) *many = 1u;
+  #pragma unroll
+  for (int j = 0; j < kItems; j++)
+    if (best[j] && f[j] == kPartCap) rep[i[j]] = best[j] - 1;
+  __syncthreads();
+}
+
+template <int BS>
+constexpr size_t kSortBytes =
+    std::max(std::max(sizeof(typename rocprim::block_radix_sort<uint64_t, BS, (int)kPartCap / BS>::storage_type),
+                      (size_t)16 * BS),
+             (size_t)8 * kPartCap);
+
+// Long chains: the elements sorted by (h, i) in LDS, each row from the element
+// before it.  kKeep: leaves the last element of each value in el[] and returns
+// how many these are.  The storage overlays the elements.
+template <int BS, bool kKeep>
+__device__ inline uint32_t sort_rows(uint2* el, uint32_t cnt, uint32_t* __restrict__ rep,
+                                     void* storage_raw) {
+  constexpr int kItems = (int)kPartCap / BS;
+  using Sort = rocprim::block_radix_sort<uint64_t, BS, kItems>;
+  auto& storage = *reinterpret_cast<typename Sort::storage_type*>(storage_raw);
+  const uint32_t t = threadIdx.x;
+  uint64_t key[kItems];
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    const uint32_t q = t * kItems + j;
+    key[j] = q < cnt ? ((uint64_t)el[q].x << 32) | el[q].y : ~0ull;  // no index is all ones
+  }
+  __syncthreads();
+  Sort().sort(key, storage);
+  __syncthreads();
+  uint64_t* last = reinterpret_cast<uint64_t*>(storage_raw);
+  uint32_t* first = reinterpret_cast<uint32_t*>(last + BS);
+  uint32_t* wsum = first + BS;
+  last[t] = key[kItems - 1];
+  first[t] = (uint32_t)(key[0] >> 32);
+  __syncthreads();
+  uint64_t prev = t ? last[t - 1] : ~0ull;
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    const uint32_t q = t * kItems + j, i = (uint32_t)key[j];
+    if (q >= 1 && q < cnt && (prev >> 32) == (key[j] >> 32)) rep[i] = (uint32_t)prev;
+    prev = key[j];
+  }
+  if (!kKeep) return 0;
+  const uint32_t after = t + 1 < BS ? first[t + 1] : 0u;  // 0 for the last: q + 1 == cnt or no element
+  uint32_t keep = 0;  // bit j: key[j] is the last of its value
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    const uint32_t q = t * kItems + j, h = (uint32_t)(key[j] >> 32);
+    const uint32_t nh = j + 1 < kItems ? (uint32_t)(key[j + 1 < kItems ? j + 1 : j] >> 32) : after;
+    if (q < cnt && (q + 1 == cnt || nh != h)) keep |= 1u << j;
+  }
+  uint32_t x = __popc(keep);
+  #pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o);
+    if ((t & 63) >= (uint32_t)o) x += y;
+  }
+  if ((t & 63) == 63) wsum[t >> 6] = x;
+  __syncthreads();
+  uint32_t at = x - __popc(keep), total = 0;
+  for (uint32_t w = 0; w < BS / 64; w++) {
+    if (w < t >> 6) at += wsum[w];
+    total += wsum[w];
+  }
+  __syncthreads();  // el overlays the storage
+  #pragma unroll
+  for (int j = 0; j < kItems; j++)
+    if (keep >> j & 1) el[at++] = make_uint2((uint32_t)(key[j] >> 32), (uint32_t)key[j]);
+  __syncthreads();
+  return total;
+}
+
+// The rows of a partition of any size, from the band's whole column: its
+// elements in index order, as many at a time as the room holds, behind the
+// last element of each value so far.  False when these leave no room.
+// Bound: the latency of the column's loads, eight a thread at a time, and a sort for
+// every 4,096 elements.
+template <int BS>
+__device__ inline bool long_rows(const uint32_t* __restrict__ col, uint32_t n, uint32_t pb,
+                                 uint32_t part, uint2* el, uint32_t* __restrict__ rep,
+                                 uint32_t (*wsum)[BS / 64], void* storage_raw) {
+  constexpr uint32_t kLoads = 8;
+  const uint32_t t = threadIdx.x;
+  uint32_t cnt = 0;
+  __syncthreads();
+  for (uint32_t q0 = 0; q0 < n; q0 += kLoads * BS) {
+    uint32_t h[kLoads];
+    #pragma unroll
+    for (uint32_t k = 0; k < kLoads; k++) h[k] = q0 + k * BS + t < n ? col[q0 + k * BS + t] : 0u;
+    #pragma unroll
+    for (uint32_t k = 0; k < kLoads; k++) {
+      const uint32_t i = q0 + k * BS + t;
+      const bool take = i < n && (uint32_t)(((uint64_t)h[k] << pb) >> 32) == part;
+      const uint64_t m = __builtin_amdgcn_ballot_w64(take);
+      if ((t & 63) == 0) wsum[k & 1][t >> 6] = (uint32_t)__popcll(m);
+      __syncthreads();
+      uint32_t at = (uint32_t)__popcll(m & ((1ull << (t & 63)) - 1ull)), total = 0;
+      for (uint32_t w = 0; w < BS / 64; w++) {
+        if (w < t >> 6) at += wsum[k & 1][w];
+        total += wsum[k & 1][w];
+      }
+      if (cnt + total > kPartCap) {  // the same in every thread
+        cnt = sort_rows<BS, true>(el, cnt, rep, storage_raw);
+        if (cnt + BS > kPartCap) return false;
+      }
+      if (take) el[cnt + at] = make_uint2(h[k], i);
+      cnt += total;
+    }
+  }
+  __syncthreads();
+  sort_rows<BS, false>(el, cnt, rep, storage_raw);
+  return true;
+}
+
+// cursor: the partitions' sizes; `longer` (a count, then the partitions) takes
+// those with more elements than room or with a long chain, for k_part_long.
+__global__ __launch_bounds__(512) void k_part_chain(const uint2* __restrict__ entries,
+                                                    const uint32_t* __restrict__ cursor, uint32_t n,
                                                     uint32_t pb, uint32_t* __restrict__ rep,
-                                                    uint32_t* __restrict__ overflow) {
-  using S1 = rocprim::block_radix_sort<uint32_t, BS, I1, uint32_t>;
-  using S2 = rocprim::block_radix_sort<uint32_t, BS, I2, uint32_t>;
-  using S3 = rocprim::block_radix_sort<uint32_t, BS, I3, uint32_t>;
-  constexpr size_t kStore =
-      std::max(std::max(sizeof(typename S1::storage_type),
-                        std::max(sizeof(typename S2::storage_type), sizeof(typename S3::storage_type))),
-               (size_t)8 * BS * I3);
-  __shared__ __align__(16) unsigned char storage[kStore];
-  const uint32_t part = blockIdx.x;
-  const uint32_t s = start[part], cnt = end[part] - s;
-  if (cnt < 2) return;  // a lone element is a bucket head: its row entry stays i
-  const uint64_t row = (uint64_t)(part >> pb) * n;
-  if (cnt <= (uint32_t)BS * I1)
-    part_sort_tier<BS, I1>(vals + s, cnt, row, rep, storage);
-  else if (cnt <= (uint32_t)BS * I2)
-    part_sort_tier<BS, I2>(vals + s, cnt, row, rep, storage);
-  else if (cnt <= (uint32_t)BS * I3)
-    part_sort_tier<BS, I3>(vals + s, cnt, row, rep, storage);
-  else if (threadIdx.x == 0)
-    atomicAdd(overflow, 1u);
+                                                    uint32_t* __restrict__ longer) {
+  __shared__ __align__(16) uint2 el[kPartCap + 2];
+  __shared__ uint32_t head[kHeads], many;
+  __shared__ uint16_t next[kPartCap + 2];
+  uint32_t band, at;
+  band_block(1u << pb, &band, &at);
+  const uint32_t part = (band << pb) + at, cnt = cursor[part];
+  if (threadIdx.x == 0) many = cnt > kPartCap;
+  if (cnt <= kPartCap) {
+    const uint2* const v = entries + (uint64_t)part * kPartCap;
+    for (uint32_t e = threadIdx.x; e < cnt; e += 512) el[e] = v[e];
+    __syncthreads();
+    uint32_t* const row = rep + (uint64_t)band * n;
+    // most partitions hold half the room: four elements a thread, not eight
+    if (cnt <= kPartCap / 2)
+      chain_rows<512, (int)kPartCap / 1024>(el, next, head, cnt, row, &many);
+    else
+      chain_rows<512, (int)kPartCap / 512>(el, next, head, cnt, row, &many);
+  }
+  if (threadIdx.x == 0 && many) longer[1 + atomicAdd(longer, 1u)] = part;
+}
+
+// The partitions that k_part_chain left: sorted, or, past their room, taken
+// from the column.  A kernel of its own, since the sort's registers would cost
+// k_part_chain a third of its wavefronts (1M records: 940 us against 840).  A
+// partition with too many values is counted in `overflow`.
+__global__ __launch_bounds__(512) void k_part_long(const uint32_t* __restrict__ longer,
+                                                   const uint2* __restrict__ entries,
+                                                   const uint32_t* __restrict__ cursor,
+                                                   const uint32_t* __restrict__ col, uint32_t n,
+                                                   uint32_t pb, uint32_t* __restrict__ rep,
+                                                   uint32_t* __restrict__ overflow) {
+  __shared__ __align__(16) unsigned char mem[kSortBytes<512>];
+  __shared__ uint32_t wsum[2][8];
+  uint2* const el = (uint2*)mem;
+  const uint32_t parts = longer[0];
+  for (uint32_t p = blockIdx.x; p < parts; p += gridDim.x) {
+    const uint32_t part = longer[1 + p], cnt = cursor[part];
+    const uint64_t row = (uint64_t)(part >> pb) * n;
+    __syncthreads();
+    if (cnt <= kPartCap) {
+      const uint2* const v = entries + (uint64_t)part * kPartCap;
+      for (uint32_t e = threadIdx.x; e < cnt; e += 512) el[e] = v[e];
+      __syncthreads();
+      sort_rows<512, false>(el, cnt, rep + row, mem);
+    } else if (!long_rows<512>(col + row, n, pb, part & ((1u << pb) - 1u), el, rep + row, wsum, mem)) {
+      if (threadIdx.x == 0) atomicAdd(overflow, 1u);
+    }
+  }
 }
 
 // Bucketing of at most kBucketSmallMax records (the head of a step, and any
@@ -743,37 +938,25 @@ struct BucketLayout {
   bool wide;
   size_t keys_in, keys_out, vals_in, vals_out, temp, temp_bytes, total;
 };
-// partitioned path: 16-bit keys, 64-bit values, the partition ranges and the
-// overflow count
+// partitioned path: the band-major column of h, the partitions, their cursors,
+// the overflow count, the count and the list of the partitions past their room
 struct PartLayout {
   bool use;
   uint32_t bits;  // partition bits pb
-  int tiers;      // capacity tiers: 0 = 4096/5120/8192, 1 = 512/1024/2048, 2 = 1024/2048/4096
-  size_t keys_in, keys_out, vals_in, vals_out, start, end, overflow, temp, temp_bytes, total;
+  size_t col, entries, cursor, overflow, total;
 };
 PartLayout part_layout(uint32_t n, bool force_wide) {
   PartLayout L{};
   L.use = !force_wide && n <= kPartMaxN;
   if (!L.use) return L;
-  const uint64_t m = (uint64_t)n * 64;
-  // The largest capacity is 1.5 to 2 times the average partition, n >> pb.
-  L.bits = n <= kPart8MaxN ? 8 : 10;
-  L.tiers = n <= kPart8MaxN ? 0 : n <= 1400000u ? 1 : 2;
-  size_t temp_bytes = 0;
-  (void)rocprim::radix_sort_pairs(nullptr, temp_bytes, (uint16_t*)nullptr, (uint16_t*)nullptr,
-                                  (uint64_t*)nullptr, (uint64_t*)nullptr, (size_t)m, 0, L.bits);
+  L.bits = part_bits(n);
   auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
   const size_t parts = (size_t)64 << L.bits;
-  L.keys_in = 0;
-  L.keys_out = L.keys_in + al(2 * m);
-  L.vals_in = L.keys_out + al(2 * m);
-  L.vals_out = L.vals_in + al(8 * m);
-  L.start = L.vals_out + al(8 * m);
-  L.end = L.start + al(4 * parts);
-  L.overflow = L.end + al(4 * parts);
-  L.temp = L.overflow + 256;
-  L.temp_bytes = temp_bytes;
-  L.total = L.temp + al(temp_bytes);
+  L.col = 0;
+  L.entries = L.col + al(256ull * n);
+  L.cursor = L.entries + al(8 * parts * kPartCap);
+  L.overflow = L.cursor + al(4 * parts);
+  L.total = L.overflow + al(4 * (parts + 2));
   return L;
 }
 BucketLayout bucket_layout(uint32_t n, bool force_wide) {
@@ -809,37 +992,22 @@ namespace {
 // then holds a partial result and the caller redoes it with the full sort).
 bool bucket_partitioned(const PartLayout& L, const uint32_t* sig, uint32_t n, uint32_t* rep,
                         char* s, hipStream_t stream, uint32_t* pinned_flag) {
-  const uint64_t m = (uint64_t)n * 64;
   const uint32_t pb = L.bits, parts = 64u << pb;
-  uint16_t* keys_in = (uint16_t*)(s + L.keys_in);
-  uint16_t* keys_out = (uint16_t*)(s + L.keys_out);
-  uint64_t* vals_in = (uint64_t*)(s + L.vals_in);
-  uint64_t* vals_out = (uint64_t*)(s + L.vals_out);
-  uint32_t* start = (uint32_t*)(s + L.start);
-  uint32_t* end = (uint32_t*)(s + L.end);
+  uint32_t* col = (uint32_t*)(s + L.col);
+  uint2* entries = (uint2*)(s + L.entries);
+  uint32_t* cursor = (uint32_t*)(s + L.cursor);
   uint32_t* overflow = (uint32_t*)(s + L.overflow);
-  hipLaunchKernelGGL(k_part_keys, dim3((n + 63) / 64), dim3(256), 0, stream, sig, n, pb, keys_in,
-                     vals_in);
-  NGIA_HIP(hipGetLastError());
-  size_t tb = L.temp_bytes;
-  NGIA_HIP(rocprim::radix_sort_pairs(s + L.temp, tb, keys_in, keys_out, vals_in, vals_out, (size_t)m,
-                                     0, pb, stream));
-  fill_u32(start, 0, parts, stream);
-  fill_u32(end, 0, parts, stream);
-  fill_u32(overflow, 0, 1, stream);
-  hipLaunchKernelGGL(k_part_bounds, dim3(std::min<uint64_t>((m / 8 + 255) / 256, 16384)), dim3(256),
-                     0, stream, keys_out, m, start, end);
-  // capacity tiers around the average partition, n >> pb
-  constexpr int B = kPartBlock;
-  if (L.tiers == 0)
-    hipLaunchKernelGGL((k_part_local<B, 4096 / B, 5120 / B, 8192 / B>), dim3(parts), dim3(B), 0,
-                       stream, vals_out, start, end, n, pb, rep, overflow);
-  else if (L.tiers == 1)
-    hipLaunchKernelGGL((k_part_local<B, 512 / B, 1024 / B, 2048 / B>), dim3(parts), dim3(B), 0,
-                       stream, vals_out, start, end, n, pb, rep, overflow);
-  else  // 256 threads measured faster here than 512 (2M records: 3.9 against 4.2 ms)
-    hipLaunchKernelGGL((k_part_local<256, 4, 8, 16>), dim3(parts), dim3(256), 0, stream, vals_out,
-                       start, end, n, pb, rep, overflow);
+  uint32_t* longer = overflow + 1;
+  // the cursors and the two counts behind them
+  fill_u32(cursor, 0, (L.overflow - L.cursor) / 4 + 2, stream);
+  hipLaunchKernelGGL(k_mix_columns, dim3((n + 63) / 64), dim3(256), 0, stream, sig, n, col, rep);
+  const uint32_t tiles = (n + kScatterTile - 1) / kScatterTile;
+  hipLaunchKernelGGL(k_part_scatter, dim3(64 * tiles), dim3(kScatterThreads), 0, stream, col, n, pb, tiles, cursor,
+                     entries);
+  hipLaunchKernelGGL(k_part_chain, dim3(parts), dim3(512), 0, stream, entries, cursor, n, pb, rep,
+                     longer);
+  hipLaunchKernelGGL(k_part_long, dim3(std::min(parts, 512u)), dim3(512), 0, stream, longer, entries,
+                     cursor, col, n, pb, rep, overflow);
   NGIA_HIP(hipGetLastError());
   uint32_t local = 0;
   uint32_t* over = pinned_flag ? pinned_flag : &local;
@@ -858,15 +1026,11 @@ void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch
   uint32_t* vals_in = (uint32_t*)(s + L.vals_in);
   uint32_t* vals_out = (uint32_t*)(s + L.vals_out);
   size_t tb = L.temp_bytes;
+  const PartLayout P = part_layout(n, force_wide);
+  if (P.use && !few_values && bucket_partitioned(P, sig, n, rep, s, stream, pinned_flag)) return;
+  // the full sort (also when a partition overflowed), from the identity rows
   hipLaunchKernelGGL(k_rep_identity, dim3(grid_for(n, 256), 64), dim3(256), 0, stream, n, rep);
   NGIA_HIP(hipGetLastError());
-  const PartLayout P = part_layout(n, force_wide);
-  if (P.use && !few_values) {
-    if (bucket_partitioned(P, sig, n, rep, s, stream, pinned_flag)) return;
-    // a partition overflowed: start again from the identity rows, full sort
-    hipLaunchKernelGGL(k_rep_identity, dim3(grid_for(n, 256), 64), dim3(256), 0, stream, n, rep);
-    NGIA_HIP(hipGetLastError());
-  }
   if (!L.wide) {
     uint32_t* keys_in = (uint32_t*)(s + L.keys_in);
     uint32_t* keys_out = (uint32_t*)(s + L.keys_out);
