@@ -589,12 +589,13 @@ uint64_t fast_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t ba
   return t;
 }
 
-// The database's representative rows from its signatures: one block per band
-// (no scratch, no host synchronisation) up to kBucketSmallMax records, the
-// partitioned or full sort beyond (or always, under NGIA_BUCKET_WIDE).
+// The database's representative rows from its signatures: the small form (no
+// host synchronisation) up to kBucketSmallMax records, partitions or the full
+// sort beyond (the latter always under NGIA_BUCKET_WIDE).
 void bucket_rows(ngia_ctx* ctx, ngia_db* db, hipStream_t s) {
   if (!ctx->bucket_wide && db->n <= kBucketSmallMax)
-    launch_bucket_small(db->sig.as<uint32_t>(), db->n, db->rep.as<uint32_t>(), s);
+    launch_bucket_small(db->sig.as<uint32_t>(), db->n, db->rep.as<uint32_t>(), db->bucket_scratch.p,
+                        s);
   else
     launch_bucket(db->sig.as<uint32_t>(), db->n, db->rep.as<uint32_t>(), db->bucket_scratch.p, s,
                   ctx->bucket_wide, db->compact, (uint32_t*)(ctx->pin + kPinOverflow));
@@ -701,8 +702,8 @@ bool head_may_need_plain(const ngia_ctx* ctx, uint32_t max_len, float thr) {
 //
 // Side stream 1, with no host synchronisation: the head's signatures (one
 // wavefront per chunk of 1,024 positions: a few thousand long records, one
-// wavefront each, would leave most SIMDs idle), its rows (one block per
-// band), its candidates and its wavefront bins, longest first.  Context
+// wavefront each, would leave most SIMDs idle), its rows (the small
+// bucketing), its candidates and its wavefront bins, longest first.  Context
 // stream, beside it: the rest's sketch, then after the head's signatures the
 // full bucketing, the main round from target h on, the head's raw edges, and
 // the sort.  The head's bins are latency bound (a few long pairs, one
@@ -727,6 +728,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
   if (h) {
     ngia_db* hd = step_head(ctx, db, h);
     hd->rep.ensure(256ull * h);
+    hd->bucket_scratch.ensure(bucket_small_bytes(h));
     ensure_batched_space(hd, bands);
     uint64_t mask = 0;
     for (uint32_t k = 0; (1u << k) <= ctx->wave_kmax; k++) mask |= 1ull << (kBinWave0 + k);
@@ -745,7 +747,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
     launch_sketch_chunks(codes, coff, len, hd->sketch_chunks.as<uint2>(), hd->n_sketch_chunks,
                          kSketchChunk, sig, q);
     NGIA_HIP(hipEventRecord(ctx->head_rows, q));
-    launch_bucket_small(sig, h, hd->rep.as<uint32_t>(), q);
+    launch_bucket_small(sig, h, hd->rep.as<uint32_t>(), hd->bucket_scratch.p, q);
     enqueue_bins(ctx, hd, identity, bands, q);
     enqueue_align(ctx, hd, identity, bands, mask, false, false, q, /*serial=*/true);
     NGIA_HIP(hipEventRecord(ctx->head_done, q));
@@ -1179,7 +1181,7 @@ extern "C" int ngia_bucket(ngia_ctx* ctx, const uint32_t* sig, uint32_t n, uint3
     scratch.ensure(bucket_scratch_bytes(n, ctx->bucket_wide));
     h2d(dsig.p, sig, 256ull * n, ctx->stream);
     if (ctx->bucket_small && n <= kBucketSmallMax)
-      launch_bucket_small(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), ctx->stream);
+      launch_bucket_small(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, ctx->stream);
     else
       launch_bucket(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, ctx->stream,
                     ctx->bucket_wide);

@@ -103,7 +103,7 @@ struct ngia_ctx {
   ngia::RouteTable route{}, route_compact{};
   // NGIA_BUCKET_WIDE=1 selects the 38-bit-key bucketing that n >= 2^26 uses
   bool bucket_wide = false;
-  // NGIA_BUCKET_SMALL=1: ngia_bucket takes the one-block-per-band bucketing
+  // NGIA_BUCKET_SMALL=1: ngia_bucket takes the small bucketing
   // of a step's head whenever n <= kBucketSmallMax (a check of that path)
   bool bucket_small = false;
   // fewest head records that ngia_db_step splits off (env NGIA_HEAD_MIN),

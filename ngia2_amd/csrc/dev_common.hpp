@@ -91,10 +91,13 @@ size_t bucket_scratch_bytes(uint32_t n, bool force_wide = false);
 void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch,
                    hipStream_t stream, bool force_wide = false, bool few_values = false,
                    uint32_t* pinned_flag = nullptr);
-// The same rows for n <= kBucketSmallMax records: one block per band, no
-// scratch and no host synchronisation.
+// The same rows for n <= kBucketSmallMax records, without a host
+// synchronisation; scratch holds bucket_small_bytes(n) bytes (no more than
+// bucket_scratch_bytes(n)).
 constexpr uint32_t kBucketSmallMax = 16384;
-void launch_bucket_small(const uint32_t* sig, uint32_t n, uint32_t* rep, hipStream_t stream);
+size_t bucket_small_bytes(uint32_t n);
+void launch_bucket_small(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch,
+                         hipStream_t stream);
 // Signatures of long records in chunks of `len` window positions:
 // chunks[c] = (record, first position); sig rows set to all ones beforehand.
 void launch_sketch_chunks(const uint8_t* codes, const uint64_t* code_off, const uint32_t* lengths,

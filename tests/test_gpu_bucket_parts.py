@@ -4,6 +4,8 @@ signatures repeated past a chain's length, past a partition's room (once and
 several times over), and more distinct values in one partition than it can
 hold, which the full sort takes."""
 
+import os
+
 import numpy as np
 import pytest
 
@@ -16,6 +18,17 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(scope="module")
 def ctx():
     c = ng.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.fixture(scope="module")
+def small():
+    os.environ["NGIA_BUCKET_SMALL"] = "1"
+    try:
+        c = ng.Context(0)
+    finally:
+        del os.environ["NGIA_BUCKET_SMALL"]
     yield c
     c.close()
 
@@ -74,3 +87,33 @@ def test_crowded_partition(ctx, distinct, each):
         sig[rows, b] = unmix(h[np.arange(k) % distinct])
     print("crowded partition", distinct, each, flush=True)
     np.testing.assert_array_equal(ctx.bucket(sig), orc.bucket(sig))
+
+
+@pytest.mark.parametrize("n", [1, 2048, 2049, 8191, 8192, 8193, 8448, 12287, 12288, 12289, 16383, 16384])
+def test_small(small, n):
+    """At most 16,384 records: each block shape's ends; by wavefronts, the
+    column's tiles of 256 and 4,096, values repeated in one round and over many."""
+    sig = signatures(n, n + 7)
+    rng = np.random.default_rng(n + 8)
+    for b, values in enumerate((1, 2, 7, 30, 300, max(n // 3, 1))):
+        sig[:, b] = sig[rng.integers(0, values, n) % n, b]
+    sig[:, 8] = sig[np.arange(n) // 2, 8]  # pairs side by side
+    sig[:, 9] = sig[np.arange(n) % ((n + 1) // 2), 9]  # pairs half a column apart
+    sig[:, 10] = unmix(np.full(n, 0xFFFFFFFF, dtype=np.uint32))
+    sig[:, 11] = unmix(np.zeros(n, dtype=np.uint32))
+    print("small bucketing", n, flush=True)
+    np.testing.assert_array_equal(small.bucket(sig), orc.bucket(sig))
+
+
+@pytest.mark.parametrize("distinct", [959, 960, 961, 1023, 1024, 1025, 3000])
+def test_small_crowded_partition(small, distinct):
+    """As many values in one wavefront's table as it has slots, and more."""
+    n = 9000
+    sig = signatures(n, distinct)
+    rng = np.random.default_rng(distinct)
+    for b in (0, 9, 63):
+        h = rng.choice(1 << 20, size=distinct, replace=False).astype(np.uint32) + np.uint32(b << 24)
+        rows = rng.permutation(n)[: min(2 * distinct, n)]
+        sig[rows, b] = unmix(h[np.arange(len(rows)) % distinct])
+    print("small bucketing, crowded partition", distinct, flush=True)
+    np.testing.assert_array_equal(small.bucket(sig), orc.bucket(sig))
