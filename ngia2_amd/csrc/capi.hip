@@ -631,8 +631,6 @@ uint32_t head_records(const ngia_db* db, float thr, uint32_t min_window) {
   return h;
 }
 
-// Positions per wavefront of the head's chunked sketch.
-constexpr uint32_t kSketchChunk = 1024;
 // Fewer head records than this are not split off (NGIA_HEAD_MIN overrides
 // it, for tests on small sets): the split's own launches and waits cost about
 // 0.2 ms (50 head records of the 10,000-protein set at -i 50: 1.60 against
@@ -646,13 +644,8 @@ ngia_db* step_head(ngia_ctx* ctx, ngia_db* db, uint32_t h) {
   if (!db->head || db->head->n != h) {
     db->head = std::make_unique<ngia_db>();
     std::vector<uint2> ch;
-    for (uint32_t i = 0; i < h; i++) {
-      const uint32_t L = db->host_len[i];
-      if (L == 0) continue;  // no window: its signature stays all ones
-      const uint32_t first = L >= 8 ? 7u : L - 1;
-      for (uint32_t p = 0; p < L; p += kSketchChunk)
-        ch.push_back(make_uint2(i, std::max(p, first)));
-    }
+    for (uint32_t i = 0; i < h; i++)
+      sketch_chunks_of(i, db->host_len[i], [&](uint2 c) { ch.push_back(c); });
     ngia_db* hd = db->head.get();
     hd->sketch_chunks.ensure(8 * std::max<size_t>(ch.size(), 1));
     if (!ch.empty())

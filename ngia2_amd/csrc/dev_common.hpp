@@ -98,6 +98,15 @@ constexpr uint32_t kBucketSmallMax = 16384;
 size_t bucket_small_bytes(uint32_t n);
 void launch_bucket_small(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch,
                          hipStream_t stream);
+// Positions per wavefront of a chunked sketch.
+constexpr uint32_t kSketchChunk = 1024;
+// The chunks of record i of L residues, for launch_sketch_chunks; none at L = 0,
+// whose signature stays all ones.
+template <typename F>
+inline void sketch_chunks_of(uint32_t i, uint32_t L, F&& chunk) {
+  const uint32_t first = L >= 8 ? 7u : L ? L - 1 : 0u;
+  for (uint32_t p = 0; p < L; p += kSketchChunk) chunk(make_uint2(i, p > first ? p : first));
+}
 // Signatures of long records in chunks of `len` window positions:
 // chunks[c] = (record, first position); sig rows set to all ones beforehand.
 void launch_sketch_chunks(const uint8_t* codes, const uint64_t* code_off, const uint32_t* lengths,

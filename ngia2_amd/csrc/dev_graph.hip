@@ -535,6 +535,37 @@ __global__ __launch_bounds__(64) void k_bin_offsets(uint32_t* __restrict__ bin_c
   if (t == 0) bin_off[kBins] = off[kBins];
 }
 
+uint64_t reachable_bins(uint32_t wlo, uint32_t whi, uint64_t pairs, uint32_t kmax,
+                        const RouteTable& route) {
+  uint64_t m = 0;
+  auto add = [&](int b) { m |= 1ull << b; };
+  for (uint32_t W = std::max(wlo, 2u); W <= std::min(whi, 60u); W++) {
+    if (W <= (uint32_t)kWinMax) {
+      if (W > (uint32_t)kWinLds || pairs >= kLowLanePairs) add((int)W);
+      add(lane_bin((int)W));
+      add(kBinWave0);
+      add(kBinSeg8x2);
+      add(kBinSeg32);
+      if (route.class_size[0]) add(kBinSeg16);
+    } else if (W <= 31) {
+      add(lane_bin((int)W));
+      add(W <= 21 ? kBinSeg8x3 : kBinSeg16x2);
+      add(kBinSeg32);
+    } else {
+      if (W <= (uint32_t)kLaneMax) add(lane_bin((int)W));
+      add(W <= 45 ? kBinSeg16x3 : kBinSeg16x4);
+      add(kBinWave0);
+    }
+  }
+  uint32_t from = 61;  // the narrowest window of the next bin
+  for (uint32_t k = 0, K = 1; K <= kmax; k++, K <<= 1) {
+    if (whi >= from && wlo <= 64 * K - K + 1) add(kBinWave0 + (int)k);
+    from = 64 * K - K + 2;
+  }
+  if (whi >= from) add(kBinPlain);
+  return m;
+}
+
 // Scatter pair indices into their bin's segment.  A block takes tiles of
 // 4096 pairs: slots are counted in LDS, reserved with one global atomic per
 // (tile, bin), then written.

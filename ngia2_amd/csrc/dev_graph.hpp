@@ -129,6 +129,13 @@ __host__ __device__ inline uint32_t route_window_bin(const RouteTable& rt, uint3
   }
 }
 
+// The bins (bit b: bin b) that pairs with windows of wlo..whi words, at most
+// `pairs` of them and not of a compact alphabet, can be aligned in after any
+// routing of k_bin_offsets; for callers that launch the bins' kernels without
+// having read the counts.
+uint64_t reachable_bins(uint32_t wlo, uint32_t whi, uint64_t pairs, uint32_t kmax,
+                        const RouteTable& route);
+
 void fill_u32(uint32_t* p, uint32_t v, uint64_t count, hipStream_t s);
 uint64_t scan_scratch_words(uint32_t n);
 // out[0..n] = exclusive prefix sums of in[0..n), out[n] = total (n >= 1).

@@ -11,8 +11,8 @@
 // order of insertion within a batch).  The length-binned alignment kernels of
 // the batched graph run unchanged on snapshot pairs.
 //
-// One batch on one lane stream: copy the packed queries into their snapshot
-// slots, byte codes, sketch; insert the batch's signatures (after the
+// One batch on one lane stream: the packed queries into their snapshot slots,
+// byte codes, sketch; insert the batch's signatures (after the
 // previous batch's insertion, whatever lane it ran on); per query the heads
 // of its 64 signatures that lie before it (one wavefront per query, lane =
 // band, distinct heads kept, longer sequence as rep, the isJob length test);
@@ -36,6 +36,47 @@ constexpr unsigned long long kEmpty = ~0ull;
 
 __device__ __host__ inline uint32_t slot_of_sig(uint32_t sig, uint32_t cap_log2) {
   return (uint32_t)((sig * 0x9E3779B1u) >> (32 - cap_log2));  // Fibonacci hashing
+}
+
+// A batch from the lane's staging (pinned host memory, read in place) to its
+// snapshot slots, and its buffers cleared: one launch where a batch of 16
+// queries spent more on five copies and three fills than on its sketch.
+struct Placement {
+  const uint32_t* h_packed;
+  const uint64_t *h_word_off, *h_code_off, *h_qid;
+  const uint32_t* h_len;
+  uint32_t* packed;
+  uint64_t *word_off, *code_off, *qid;
+  uint32_t* len;
+  uint64_t words;
+  uint32_t count;
+  unsigned long long* best;  // count, zero
+  uint32_t* done;            // count, zero
+  uint32_t* counters;        // counter_words, zero
+  uint32_t counter_words;
+  uint32_t* sig;  // 64 count, all ones; null: left as it is
+};
+__global__ __launch_bounds__(256) void k_serve_place(Placement a) {
+  const uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x, step = (uint64_t)gridDim.x * 256;
+  for (uint64_t i = t; i < a.words; i += 4 * step) {
+    uint32_t w[4];
+    #pragma unroll
+    for (int k = 0; k < 4; k++) w[k] = i + k * step < a.words ? a.h_packed[i + k * step] : 0u;
+    #pragma unroll
+    for (int k = 0; k < 4; k++)
+      if (i + k * step < a.words) a.packed[i + k * step] = w[k];
+  }
+  for (uint64_t i = t; i < a.count; i += step) {
+    a.word_off[i] = a.h_word_off[i];
+    a.code_off[i] = a.h_code_off[i];
+    a.qid[i] = a.h_qid[i];
+    a.len[i] = a.h_len[i];
+    a.best[i] = 0;
+    a.done[i] = 0;
+  }
+  for (uint64_t i = t; i < a.counter_words; i += step) a.counters[i] = 0;
+  if (a.sig)
+    for (uint64_t i = t; i < 64ull * a.count; i += step) a.sig[i] = 0xFFFFFFFFu;
 }
 
 // Insert (sig, index0 + i) for i < count and every band (signatures
@@ -212,30 +253,34 @@ struct Seg {
 };
 
 struct Lane {
-  hipStream_t stream = nullptr;
+  hipStream_t stream = nullptr, side = nullptr;
   hipEvent_t t0 = nullptr, t1 = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;  // the long windows, on `side`
   hipEvent_t inserted = nullptr, resolved = nullptr;  // ordering marks for the next batch
-  // pinned host staging: packed words, then per-query word_off, code_off, lengths, qid
+  // pinned host staging: packed words, per-query word_off, code_off, lengths, qid,
+  // the chunks of the sketch; and the results
   uint32_t* h_packed = nullptr;
   uint64_t* h_word_off = nullptr;
   uint64_t* h_code_off = nullptr;
   uint32_t* h_len = nullptr;
   uint64_t* h_qid = nullptr;
+  uint2* h_chunks = nullptr;
   ngia_assignment* h_out = nullptr;
   // device buffers of qcap queries (grown at admission, by free HBM)
   uint32_t qcap = 0;
-  DevBuf sig, pairs, score, bin_of, list, counters, best, ncand, qid, out, done, plain_jobs,
+  DevBuf sig, pairs, score, bin_of, list, counters, best, ncand, qid, done, plain_jobs,
       plain_scratch;
   std::vector<Seg> segs;
   uint32_t count = 0;
   bool busy = false;
   ~Lane() {
     for (void* p : {(void*)h_packed, (void*)h_word_off, (void*)h_code_off, (void*)h_len,
-                    (void*)h_qid, (void*)h_out})
+                    (void*)h_qid, (void*)h_chunks, (void*)h_out})
       if (p) (void)hipHostFree(p);
-    for (hipEvent_t e : {t0, t1, inserted, resolved})
+    for (hipEvent_t e : {t0, t1, fork, join, inserted, resolved})
       if (e) (void)hipEventDestroy(e);
-    if (stream) (void)hipStreamDestroy(stream);
+    for (hipStream_t q : {stream, side})
+      if (q) (void)hipStreamDestroy(q);
   }
 };
 
@@ -274,7 +319,7 @@ constexpr uint32_t kServePlainBlocks = 64;
 // Device bytes of a lane's buffers for q queries (at most one pair per band
 // per query).
 uint64_t lane_bytes(uint32_t q) {
-  return (uint64_t)q * (256 + 64 * (8 + 4 + 4 + 4 + 12) + 8 + 4 + 8 + sizeof(ngia_assignment) + 4);
+  return (uint64_t)q * (256 + 64 * (8 + 4 + 4 + 4 + 12) + 8 + 4 + 8 + 4);
 }
 
 void lane_alloc(Lane& ln, uint32_t q) {
@@ -287,7 +332,6 @@ void lane_alloc(Lane& ln, uint32_t q) {
   ln.best.ensure(8ull * q);
   ln.ncand.ensure(4ull * q);
   ln.qid.ensure(8ull * q);
-  ln.out.ensure(sizeof(ngia_assignment) * q);
   ln.done.ensure(4ull * q);
   ln.plain_jobs.ensure(12 * pcap);
   ln.qcap = q;
@@ -369,6 +413,9 @@ void serve_setup(ngia_serve* sv, ngia_db* db, const uint32_t* cluster_of,
   for (uint32_t k = 0; k < sv->lanes; k++) {
     auto ln = std::make_unique<Lane>();
     NGIA_HIP(hipStreamCreateWithFlags(&ln->stream, hipStreamNonBlocking));
+    NGIA_HIP(hipStreamCreateWithFlags(&ln->side, hipStreamNonBlocking));
+    NGIA_HIP(hipEventCreateWithFlags(&ln->fork, hipEventDisableTiming));
+    NGIA_HIP(hipEventCreateWithFlags(&ln->join, hipEventDisableTiming));
     NGIA_HIP(hipEventCreate(&ln->t0));
     NGIA_HIP(hipEventCreate(&ln->t1));
     NGIA_HIP(hipEventCreateWithFlags(&ln->inserted, hipEventDisableTiming));
@@ -378,6 +425,7 @@ void serve_setup(ngia_serve* sv, ngia_db* db, const uint32_t* cluster_of,
     NGIA_HIP(hipHostMalloc((void**)&ln->h_code_off, 8ull * sv->qmax, 0));
     NGIA_HIP(hipHostMalloc((void**)&ln->h_len, 4ull * sv->qmax, 0));
     NGIA_HIP(hipHostMalloc((void**)&ln->h_qid, 8ull * sv->qmax, 0));
+    NGIA_HIP(hipHostMalloc((void**)&ln->h_chunks, 8 * (sv->qmax + sv->wmax * 8 / kSketchChunk + 1), 0));
     NGIA_HIP(hipHostMalloc((void**)&ln->h_out, sizeof(ngia_assignment) * sv->qmax, 0));
     ln->counters.ensure(sizeof(Counters));
     ln->plain_scratch.ensure(4 * align_plain_scratch_words(sv->nw_cap, kServePlainBlocks));
@@ -413,6 +461,7 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
   const uint64_t wbase = sv->res_words + sv->wcur;
   const uint64_t cbase = sv->res_codes + sv->ccur;
   uint64_t w = 0, c = 0;
+  uint32_t shortest = 0xFFFFFFFFu, longest = 0, chunks = 0;  // of the queries that align at all
   for (const Seg& sg : ln.segs) {
     for (uint32_t j = 0; j < sg.count; j++) {
       const uint32_t q = sg.first + j, slot = sg.slot + j;
@@ -423,8 +472,17 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
       ln.h_qid[slot] = qid0 + q;
       w += rec_words(Lq);
       c += 32ull * ((Lq + 31) / 32);
+      if (Lq) shortest = std::min(shortest, Lq);
+      longest = std::max(longest, Lq);
     }
   }
+  // One wavefront sketches a position in about 55 ns: past two chunks the
+  // longest query would keep the batch waiting (1.1 ms for 8,192 log-normal
+  // queries, 20,000 residues the longest).
+  const bool in_chunks = longest > 2 * kSketchChunk;
+  if (in_chunks)
+    for (uint32_t q = 0; q < Q; q++)
+      sketch_chunks_of(q, ln.h_len[q], [&](uint2 ch) { ln.h_chunks[chunks++] = ch; });
   sv->pos += Q;  // capacity checked at admission
   sv->wcur += w;
   sv->ccur += c;
@@ -434,15 +492,38 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
                  ln.h_packed);
   hipStream_t s = ln.stream;
   NGIA_HIP(hipEventRecord(ln.t0, s));
-  NGIA_HIP(hipMemcpyAsync(sv->packed.as<uint32_t>() + wbase, ln.h_packed, 4 * w, hipMemcpyHostToDevice, s));
-  NGIA_HIP(hipMemcpyAsync(sv->word_off.as<uint64_t>() + base, ln.h_word_off, 8ull * Q, hipMemcpyHostToDevice, s));
-  NGIA_HIP(hipMemcpyAsync(sv->code_off.as<uint64_t>() + base, ln.h_code_off, 8ull * Q, hipMemcpyHostToDevice, s));
-  NGIA_HIP(hipMemcpyAsync(sv->lengths.as<uint32_t>() + base, ln.h_len, 4ull * Q, hipMemcpyHostToDevice, s));
-  NGIA_HIP(hipMemcpyAsync(ln.qid.p, ln.h_qid, 8ull * Q, hipMemcpyHostToDevice, s));
+  Counters* dc = ln.counters.as<Counters>();
+  Placement pl;
+  pl.h_packed = ln.h_packed;
+  pl.h_word_off = ln.h_word_off;
+  pl.h_code_off = ln.h_code_off;
+  pl.h_qid = ln.h_qid;
+  pl.h_len = ln.h_len;
+  pl.packed = sv->packed.as<uint32_t>() + wbase;
+  pl.word_off = sv->word_off.as<uint64_t>() + base;
+  pl.code_off = sv->code_off.as<uint64_t>() + base;
+  pl.qid = ln.qid.as<uint64_t>();
+  pl.len = sv->lengths.as<uint32_t>() + base;
+  pl.words = w;
+  pl.count = Q;
+  pl.best = ln.best.as<unsigned long long>();
+  pl.done = ln.done.as<uint32_t>();
+  pl.counters = ln.counters.as<uint32_t>();
+  pl.counter_words = sizeof(Counters) / 4;
+  pl.sig = in_chunks ? ln.sig.as<uint32_t>() : nullptr;
+  const uint64_t most = std::max<uint64_t>(w, pl.counter_words);
+  hipLaunchKernelGGL(k_serve_place, dim3((uint32_t)std::min<uint64_t>((most + 1023) / 1024, 1024)),
+                     dim3(256), 0, s, pl);
+  NGIA_HIP(hipGetLastError());
   launch_codes(sv->packed.as<uint32_t>(), sv->word_off.as<uint64_t>() + base,
                sv->code_off.as<uint64_t>() + base, Q, sv->codes.as<uint8_t>(), s);
-  launch_sketch(sv->codes.as<uint8_t>(), sv->code_off.as<uint64_t>() + base,
-                sv->lengths.as<uint32_t>() + base, Q, ln.sig.as<uint32_t>(), s);
+  if (in_chunks)
+    launch_sketch_chunks(sv->codes.as<uint8_t>(), sv->code_off.as<uint64_t>() + base,
+                         sv->lengths.as<uint32_t>() + base, ln.h_chunks, chunks, kSketchChunk,
+                         ln.sig.as<uint32_t>(), s);
+  else
+    launch_sketch(sv->codes.as<uint8_t>(), sv->code_off.as<uint64_t>() + base,
+                  sv->lengths.as<uint32_t>() + base, Q, ln.sig.as<uint32_t>(), s);
   // The batch's signatures join the tables after the previous batch's (its
   // records and codes are in place by then), so every lookup below sees all
   // earlier queries of the session.
@@ -453,21 +534,29 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
   NGIA_HIP(hipGetLastError());
   NGIA_HIP(hipEventRecord(ln.inserted, s));
   sv->last_inserted = ln.inserted;
-  Counters* dc = ln.counters.as<Counters>();
-  fill_u32(ln.counters.as<uint32_t>(), 0, sizeof(Counters) / 4, s);
-  fill_u32(ln.best.as<uint32_t>(), 0, 2ull * Q, s);
-  fill_u32(ln.done.as<uint32_t>(), 0, Q, s);
   hipLaunchKernelGGL(k_serve_lookup, dim3(Q), dim3(64), 0, s, ln.sig.as<uint32_t>(), Q, base,
                      sv->tables.as<unsigned long long>(), sv->cap_log2, sv->lengths.as<uint32_t>(),
                      sv->thr, ln.pairs.as<uint2>(), &dc->total_cand, ln.ncand.as<uint32_t>());
   NGIA_HIP(hipGetLastError());
-  // The length bins, one after another on the lane stream (the snapshot's
-  // window kernels use the 16-code table, so its routing applies).
+  // The length bins (the snapshot's window kernels use the 16-code table, so its
+  // routing applies).
   const uint64_t* np = (const uint64_t*)&dc->total_cand;
   bin_pairs(ln.pairs.as<uint2>(), np, sv->lengths.as<uint32_t>(), sv->thr, ln.bin_of.as<uint32_t>(),
             dc->bin_cnt, dc->bin_off, dc->cursor, ln.list.as<uint32_t>(), dc->bin_tiles,
             ln.score.as<uint32_t>(), sv->ctx->wave_kmax, dc->remap, sv->ctx->route,
             sv->ctx->seg2_min, sv->ctx->lane_fill, false, grid, s);
+  // Nothing is read back, so the kernels launched are those of every bin that a
+  // pair with one of these queries could be in: 28 launches for any, 5 for 16
+  // queries of the usual lengths.  A pair's target has T >= R thr residues of
+  // its rep's R, and one of the two is a query: its window, lsft / 32 +
+  // ceil(rsft / 32) words of band_edges, has lsft + rsft between 2 T (1 - thr)
+  // and T (1 - thr) + R - T thr plus 64 for the roundings; two words of slack
+  // on either side for these and for thr's.
+  const double thr = sv->thr, least = shortest * thr, widest = longest / thr;
+  const uint32_t wlo = (uint32_t)std::max(2.0, std::floor(2 * least * (1 - thr) / 32) - 2);
+  const uint32_t whi = longest ? (uint32_t)((longest * (1 - thr) + widest - longest * thr + 64) / 32) + 4 : 0u;
+  const uint64_t bins = reachable_bins(wlo, whi, 64ull * Q, sv->ctx->wave_kmax, sv->ctx->route);
+  auto reached = [&](int b) { return (bins >> b & 1) != 0; };
   AlignArgs aa;
   aa.packed = sv->packed.as<uint32_t>();
   aa.word_off = sv->word_off.as<uint64_t>();
@@ -475,15 +564,27 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
   aa.code_off = sv->code_off.as<uint64_t>();
   aa.lengths = sv->lengths.as<uint32_t>();
   aa.thr = sv->thr;
-  for (int kk = 5; kk >= 0; kk--) {
-    if ((1u << kk) > sv->ctx->wave_kmax) continue;
+  auto wave = [&](int kk, hipStream_t q) {
     const int bin = kBinWave0 + kk;
+    if ((1u << kk) > sv->ctx->wave_kmax || !reached(bin)) return;
     launch_align_wave(1 << kk, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), &dc->bin_off[bin],
                       &dc->bin_cnt[bin], dc->queue[bin], ln.score.as<uint32_t>(),
-                      std::min<uint32_t>(Q * 64, persistent_blocks(sv->ctx, wave_lds_bytes(1 << kk))), s);
+                      std::min<uint32_t>(Q * 64, persistent_blocks(sv->ctx, wave_lds_bytes(1 << kk))), q);
+  };
+  // Windows past 64 words are few and long, a wavefront each for a millisecond
+  // and more: beside the other bins (8,192 log-normal queries at 90%: 1.7 + 0.4
+  // ms beside 0.8 of the rest).
+  const bool beside = (bins >> (kBinWave0 + 1) & 31) != 0;
+  if (beside) {
+    NGIA_HIP(hipEventRecord(ln.fork, s));
+    NGIA_HIP(hipStreamWaitEvent(ln.side, ln.fork, 0));
+    for (int kk = 5; kk >= 1; kk--) wave(kk, ln.side);
+    NGIA_HIP(hipEventRecord(ln.join, ln.side));
   }
+  wave(0, s);
   for (const int bin :
        {kBinSeg16x4, kBinSeg16x3, kBinSeg8x3, kBinSeg16x2, kBinSeg32, kBinSeg16, kBinSeg8x2}) {
+    if (!reached(bin)) continue;
     const int G = seg_lanes(bin), K = seg_words(bin);
     launch_align_seg(G, K, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), &dc->bin_off[bin],
                      &dc->bin_cnt[bin], dc->queue[bin], ln.score.as<uint32_t>(),
@@ -491,22 +592,29 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
                                         sv->ctx->prop.multiProcessorCount * seg_blocks_per_cu(G, K)),
                      s);
   }
-  for (int cls = kLaneClasses - 1; cls >= 0; cls--)
-    launch_align_lanes(cls, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), dc->bin_off, dc->bin_cnt,
-                       dc->queue[0], ln.score.as<uint32_t>(), nullptr, lane_class_min(cls),
-                       lane_class_max(cls),
-                       (uint32_t)sv->ctx->prop.multiProcessorCount, 64ull * Q, s);
+  for (int cls = kLaneClasses - 1; cls >= 0; cls--) {
+    bool any = false;
+    for (int W = lane_class_min(cls); W <= lane_class_max(cls); W++) any = any || reached(lane_bin(W));
+    if (any)
+      launch_align_lanes(cls, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), dc->bin_off, dc->bin_cnt,
+                         dc->queue[0], ln.score.as<uint32_t>(), nullptr, lane_class_min(cls),
+                         lane_class_max(cls), (uint32_t)sv->ctx->prop.multiProcessorCount, 64ull * Q, s);
+  }
   for (int W = kWinLds; W >= 2; W--)
-    launch_align_win(W, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), &dc->bin_off[W],
-                     &dc->bin_cnt[W], dc->queue[W], ln.score.as<uint32_t>(),
-                     std::min<uint32_t>(Q, persistent_blocks(sv->ctx, win_lds_bytes(W))), s);
-  plain_bin_jobs(ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), dc->bin_off, dc->bin_cnt,
-                 ln.plain_jobs.as<uint32_t>(), s);
-  launch_align_plain(aa, ln.plain_jobs.as<uint32_t>(), kServePlainBlocks * 64, sv->nw_cap,
-                     ln.plain_scratch.as<uint32_t>(), ln.plain_scratch.bytes / 4, s,
-                     &dc->bin_cnt[kBinPlain], kServePlainBlocks);
-  plain_bin_scores(ln.list.as<uint32_t>(), dc->bin_off, dc->bin_cnt, ln.plain_jobs.as<uint32_t>(),
-                   ln.score.as<uint32_t>(), s);
+    if (reached(W))
+      launch_align_win(W, aa, ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), &dc->bin_off[W],
+                       &dc->bin_cnt[W], dc->queue[W], ln.score.as<uint32_t>(),
+                       std::min<uint32_t>(Q, persistent_blocks(sv->ctx, win_lds_bytes(W))), s);
+  if (reached(kBinPlain)) {
+    plain_bin_jobs(ln.pairs.as<uint2>(), ln.list.as<uint32_t>(), dc->bin_off, dc->bin_cnt,
+                   ln.plain_jobs.as<uint32_t>(), s);
+    launch_align_plain(aa, ln.plain_jobs.as<uint32_t>(), kServePlainBlocks * 64, sv->nw_cap,
+                       ln.plain_scratch.as<uint32_t>(), ln.plain_scratch.bytes / 4, s,
+                       &dc->bin_cnt[kBinPlain], kServePlainBlocks);
+    plain_bin_scores(ln.list.as<uint32_t>(), dc->bin_off, dc->bin_cnt, ln.plain_jobs.as<uint32_t>(),
+                     ln.score.as<uint32_t>(), s);
+  }
+  if (beside) NGIA_HIP(hipStreamWaitEvent(s, ln.join, 0));
   hipLaunchKernelGGL(k_serve_best, dim3(grid), dim3(256), 0, s, ln.pairs.as<uint2>(),
                      (const unsigned long long*)np, ln.score.as<uint32_t>(), base,
                      ln.best.as<unsigned long long>());
@@ -515,11 +623,10 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
   hipLaunchKernelGGL(k_serve_result, dim3(1), dim3(1024), 0, s, ln.best.as<unsigned long long>(),
                      ln.ncand.as<uint32_t>(), Q, sv->n, pos0, sv->cluster_of.as<uint32_t>(),
                      sv->qcluster.as<uint32_t>(), ln.done.as<uint32_t>(), ln.qid.as<uint64_t>(),
-                     sv->new_base, ln.out.as<ngia_assignment>());
+                     sv->new_base, ln.h_out);
   NGIA_HIP(hipGetLastError());
   NGIA_HIP(hipEventRecord(ln.resolved, s));
   sv->last_resolved = ln.resolved;
-  NGIA_HIP(hipMemcpyAsync(ln.h_out, ln.out.p, sizeof(ngia_assignment) * Q, hipMemcpyDeviceToHost, s));
   NGIA_HIP(hipEventRecord(ln.t1, s));
   ln.busy = true;
 }
@@ -661,7 +768,8 @@ int run_stream(ngia_serve* sv, const uint8_t* res, const uint64_t* res_off, cons
 // Wait for every lane (after a failed call some may still run).
 void drain(ngia_serve* sv) {
   for (auto& ln : sv->L)
-    if (ln->stream) (void)hipStreamSynchronize(ln->stream);
+    for (hipStream_t q : {ln->stream, ln->side})
+      if (q) (void)hipStreamSynchronize(q);
 }
 
 }  // namespace

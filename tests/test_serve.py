@@ -315,3 +315,33 @@ def test_handles_outlive_their_context(served):
         sv.assign(queries)
     sv.close()
     db.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("identity", [20, 50, 90, 99])
+@pytest.mark.parametrize("length", [1, 9, 150, 700, 2047, 2049, 4000, 9000])
+def test_serve_batch_of_one_length(ctx, identity, length):
+    """Batches whose queries have about one length, against residents as long
+    and shorter and longer by up to the identity: only the bins these can reach
+    are launched, and past 2,048 residues the sketch is cut into chunks."""
+    rng = np.random.default_rng(identity * 10007 + length)
+    anc = bytes(AMINO[i] for i in rng.integers(20, size=min(2 * length, 12000) + 40))
+    cuts = sorted({max(1, min(len(anc), int(length * f)))
+                   for f in (0.02, 0.2, identity / 100, identity / 100 + 0.02, 0.97, 1.0, 1.02,
+                             min(2.0, 100 / identity - 0.02), min(2.0, 100 / identity), 2.0)},
+                  reverse=True)
+    seqs = [anc[:c] for c in cuts]
+    packed, off = orc.pack_many(seqs)
+    lengths = np.array([len(s) for s in seqs], dtype=np.uint32)
+    sig = orc.sketch_all(packed, off)
+    cluster_of = np.arange(len(seqs), dtype=np.uint32) + 3
+    qs = [anc[:length], mutate(rng, anc[:length], 0.02, 0.01), anc[2:length + 2], b""]
+    want = orc.serve_assign(packed, off, sig, cluster_of, qs, identity, 10 ** 6)
+    print("[case] serve batch of one length", identity, length, flush=True)
+    db = ng.Database(ctx, packed, off, lengths)
+    db.sketch()
+    sv = ng.Serve(db, cluster_of, identity, 10 ** 6)
+    got, _ = sv.assign(ng.Queries.from_strings(qs))
+    np.testing.assert_array_equal(as_rows(got), want)
+    sv.close()
+    db.close()
