@@ -157,7 +157,7 @@ void enqueue_bins(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
   const uint32_t* len = db->lengths.as<uint32_t>();
   fill_u32(db->counters.as<uint32_t>(), 0, sizeof(Counters) / 4, s);
   pair_count(db->rep.as<uint32_t>(), len, n, db->t0, bands, thr, db->cnt.as<uint32_t>(),
-             db->keep.as<uint64_t>(), &dc->total_cand, s, fast);
+             db->keep.as<uint64_t>(), db->degree.as<uint32_t>(), &dc->total_cand, s, fast);
   scan_u32(db->cnt.as<uint32_t>(), n, db->off.as<uint64_t>(), db->sums.as<uint64_t>(), s);
   pair_emit(db->rep.as<uint32_t>(), n, bands, db->keep.as<uint64_t>(), db->off.as<uint64_t>(),
             db->pairs.as<uint2>(), s);
@@ -289,13 +289,25 @@ void enqueue_scores(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t band
   }
 }
 
-// Part 2 of a graph round: the scores, then the passing pairs as raw edges.
+// Blocks of a kernel over a round's pairs, 1,024 a block at least.
+uint32_t pair_grid(ngia_ctx* ctx, const ngia_db* db, uint32_t bands) {
+  return (uint32_t)std::min<uint64_t>(persistent_blocks(ctx, 0) * 4, ((uint64_t)db->n * bands + 1023) / 1024);
+}
+
+// The passing pairs of round `of` into the edge counts of `db` (the same, or
+// `of` its head round).
+void enqueue_edge_count(ngia_ctx* ctx, ngia_db* db, ngia_db* of, uint32_t bands, hipStream_t s) {
+  Counters* dc = db->counters.as<Counters>();
+  edge_count(of->pairs.as<uint2>(), of->off.as<uint64_t>() + of->n, of->score.as<uint32_t>(),
+             db->degree.as<uint32_t>(), of->bin_of.as<uint32_t>(), &dc->ecount, &dc->max_degree,
+             pair_grid(ctx, of, bands), s);
+}
+
+// Part 2 of a graph round: the scores, then the passing pairs counted.
 void enqueue_align(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, uint64_t mask,
-                   bool time_align, bool tally, hipStream_t s, bool serial = false) {
-  enqueue_scores(ctx, db, identity, bands, mask, time_align, tally, s, serial);
-  pairs_to_edges(db->pairs.as<uint2>(), db->off.as<uint64_t>() + db->n, db->score.as<uint32_t>(),
-                 db->ekeys.as<uint64_t>(), db->escores.as<uint32_t>(),
-                 &db->counters.as<Counters>()->ecount, persistent_blocks(ctx, 0) * 4, s);
+                   bool time_align, bool tally, hipStream_t s) {
+  enqueue_scores(ctx, db, identity, bands, mask, time_align, tally, s, /*serial=*/false);
+  enqueue_edge_count(ctx, db, db, bands, s);
 }
 
 // Capture what fn enqueues on stream s into an instantiated graph.
@@ -337,6 +349,8 @@ void ensure_pair_space(ngia_db* db, uint32_t bands) {
 // The same with the edge list.
 void ensure_batched_space(ngia_db* db, uint32_t bands) {
   ensure_pair_space(db, bands);
+  db->degree.ensure(4ull * db->n);
+  db->edge_off.ensure(8ull * (db->n + 1));
   ensure_edge_space(db, std::max<uint64_t>((uint64_t)db->n * bands, 1));
 }
 
@@ -354,8 +368,8 @@ bool ensure_plain_bin_space(ngia_db* db, uint32_t bands) {
   return db->plain_jobs.p != j0 || db->plain_scratch.p != s0;
 }
 
-// The head round of a step (ngia_db_step), whose raw edges join the main
-// round's before the sort: its database and the event recorded after them.
+// The head round of a step (ngia_db_step), whose edges join the main round's:
+// its database and the event recorded after its scores.
 struct HeadRound {
   ngia_db* db = nullptr;
   hipEvent_t done = nullptr;
@@ -364,8 +378,7 @@ struct HeadRound {
 // The batched round: its first part captured once per (identity, bands), its
 // second once per set of bins that hold pairs, both replayed (or launched
 // eagerly, with the alignment phase timed).  With a head round, the main
-// round's targets start at db->t0 and the head's raw edges are appended
-// before the sort.
+// round's targets start at db->t0 and the head's edges join it in the list.
 void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
                    ngia_graph_stats* st, bool eager, bool tally, const HeadRound* head = nullptr) {
   hipStream_t s = ctx->stream;
@@ -376,7 +389,7 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
   std::vector<uintptr_t> key;
   for (const DevBuf* b : {&db->packed, &db->word_off, &db->lengths, &db->codes, &db->code_off,
                           &db->rep, &db->counters, &db->cnt, &db->keep, &db->off, &db->sums, &db->pairs,
-                          &db->score, &db->bin_of, &db->list, &db->ekeys, &db->escores})
+                          &db->score, &db->bin_of, &db->list, &db->degree})
     key.push_back((uintptr_t)b->p);
   {
     const ngia::RouteTable& rt = db->compact ? ctx->route_compact : ctx->route;
@@ -440,35 +453,53 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
     NGIA_HIP(hipGraphLaunch(g2, s));
   }
   NGIA_HIP(hipEventRecord(ctx->ev[1], s));
+  // the sorted edge list, with the head's pairs (targets below db->t0, disjoint
+  // from the main round's)
+  Counters* dc = db->counters.as<Counters>();
+  ngia_db* const hd = head ? head->db : nullptr;
+  if (hd) NGIA_HIP(hipStreamWaitEvent(s, head->done, 0));
+  NGIA_HIP(hipEventRecord(ctx->ev[4], s));
+  if (hd) enqueue_edge_count(ctx, db, hd, bands, s);
+  scan_u32(db->degree.as<uint32_t>(), n, db->edge_off.as<uint64_t>(), db->sums.as<uint64_t>(), s);
+  for (ngia_db* of : {db, hd})
+    if (of)
+      edge_scatter(of->pairs.as<uint2>(), of->off.as<uint64_t>() + of->n, of->score.as<uint32_t>(),
+                   db->edge_off.as<uint64_t>(), of->bin_of.as<uint32_t>(), &dc->max_degree,
+                   db->ekeys_tmp.as<uint64_t>(), db->escores_tmp.as<uint32_t>(),
+                   pair_grid(ctx, of, bands), s);
+  edge_rank(db->edge_off.as<uint64_t>(), n, &dc->max_degree, db->ekeys_tmp.as<uint64_t>(),
+            db->escores_tmp.as<uint32_t>(), db->ekeys.as<uint64_t>(), db->escores.as<uint32_t>(),
+            pair_grid(ctx, db, bands), s);
+  NGIA_HIP(hipEventRecord(ctx->ev[5], s));
   Counters hc, hh{};
   uint64_t npairs = 0, hpairs = 0;
   d2h(ctx->pin + kPinCounters, db->counters.p, kCounterStats, s);
   d2h(ctx->pin + kPinPairs, db->off.as<uint64_t>() + n, 8, s);
-  if (head) {
-    NGIA_HIP(hipStreamWaitEvent(s, head->done, 0));
-    d2h(ctx->pin + kPinHeadCounters, head->db->counters.p, kCounterStats, s);
-    d2h(ctx->pin + kPinHeadPairs, head->db->off.as<uint64_t>() + head->db->n, 8, s);
+  if (hd) {
+    d2h(ctx->pin + kPinHeadCounters, hd->counters.p, kCounterStats, s);
+    d2h(ctx->pin + kPinHeadPairs, hd->off.as<uint64_t>() + hd->n, 8, s);
   }
   NGIA_HIP(hipStreamSynchronize(s));
   std::memcpy(&hc, ctx->pin + kPinCounters, kCounterStats);
   std::memcpy(&npairs, ctx->pin + kPinPairs, 8);
-  if (head) {
+  if (hd) {
     std::memcpy(&hh, ctx->pin + kPinHeadCounters, kCounterStats);
     std::memcpy(&hpairs, ctx->pin + kPinHeadPairs, 8);
   }
   db->n_pairs = npairs;
-  NGIA_HIP(hipEventRecord(ctx->ev[4], s));
-  if (hh.ecount) {
-    // the head's pairs (targets below db->t0) are disjoint from the main
-    // round's; their raw edges follow the main round's
-    NGIA_HIP(hipMemcpyAsync(db->ekeys.as<uint64_t>() + hc.ecount, head->db->ekeys.p, 8 * hh.ecount,
-                            hipMemcpyDeviceToDevice, s));
-    NGIA_HIP(hipMemcpyAsync(db->escores.as<uint32_t>() + hc.ecount, head->db->escores.p,
-                            4 * hh.ecount, hipMemcpyDeviceToDevice, s));
+  db->n_edges = hc.ecount;
+  const bool sorted = hc.max_degree > kMaxDegree;
+  if (sorted) {  // a u with too many edges to rank: compacted and sorted
+    fill_u32((uint32_t*)&dc->ecount, 0, 2, s);
+    for (ngia_db* of : {db, hd})
+      if (of)
+        pairs_to_edges(of->pairs.as<uint2>(), of->off.as<uint64_t>() + of->n,
+                       of->score.as<uint32_t>(), db->ekeys.as<uint64_t>(),
+                       db->escores.as<uint32_t>(), &dc->ecount, persistent_blocks(ctx, 0) * 4, s);
+    finalize(ctx, db, hc.ecount);
+    NGIA_HIP(hipEventRecord(ctx->ev[5], s));
+    NGIA_HIP(hipEventSynchronize(ctx->ev[5]));
   }
-  finalize(ctx, db, hc.ecount + hh.ecount);
-  NGIA_HIP(hipEventRecord(ctx->ev[5], s));
-  NGIA_HIP(hipEventSynchronize(ctx->ev[5]));
   ctx->timing.graph_ms = event_ms(ctx->ev[0], ctx->ev[1]);
   ctx->timing.finalize_ms = event_ms(ctx->ev[4], ctx->ev[5]);
   ctx->timing.align_ms = eager ? event_ms(ctx->ev[2], ctx->ev[3]) : 0.0;
@@ -494,7 +525,7 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
     st->ms_align = event_ms(ctx->ev[0], ctx->ev[1]);
     st->ms_edges = event_ms(ctx->ev[4], ctx->ev[5]);
     st->align_launches = launches;
-    st->host_syncs = 3;
+    st->host_syncs = sorted ? 3 : 2;
   }
 }
 
@@ -698,8 +729,8 @@ bool head_may_need_plain(const ngia_ctx* ctx, uint32_t max_len, float thr) {
 // wavefront each, would leave most SIMDs idle), its rows (the small
 // bucketing), its candidates and its wavefront bins, longest first.  Context
 // stream, beside it: the rest's sketch, then after the head's signatures the
-// full bucketing, the main round from target h on, the head's raw edges, and
-// the sort.  The head's bins are latency bound (a few long pairs, one
+// full bucketing, the main round from target h on, and the sorted edge list of
+// both.  The head's bins are latency bound (a few long pairs, one
 // wavefront each) and run on the SIMDs the VALU-bound sketch leaves between
 // its instructions.
 void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, bool split,
@@ -722,7 +753,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
     ngia_db* hd = step_head(ctx, db, h);
     hd->rep.ensure(256ull * h);
     hd->bucket_scratch.ensure(bucket_small_bytes(h));
-    ensure_batched_space(hd, bands);
+    ensure_pair_space(hd, bands);
     uint64_t mask = 0;
     for (uint32_t k = 0; (1u << k) <= ctx->wave_kmax; k++) mask |= 1ull << (kBinWave0 + k);
     // a head window below 61 words lets head pairs into the 3- and 4-word bins
@@ -742,7 +773,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
     NGIA_HIP(hipEventRecord(ctx->head_rows, q));
     launch_bucket_small(sig, h, hd->rep.as<uint32_t>(), hd->bucket_scratch.p, q);
     enqueue_bins(ctx, hd, identity, bands, q);
-    enqueue_align(ctx, hd, identity, bands, mask, false, false, q, /*serial=*/true);
+    enqueue_scores(ctx, hd, identity, bands, mask, false, false, q, /*serial=*/true);
     NGIA_HIP(hipEventRecord(ctx->head_done, q));
     hr.db = hd;
     hr.done = ctx->head_done;

@@ -65,6 +65,7 @@ struct Counters {
   unsigned long long total_cand;  // candidates with duplicates
   unsigned long long ecount;      // raw edges
   unsigned long long unique;      // edges after unique
+  unsigned long long max_degree;  // a u's edges, when above kMaxDegree
   unsigned long long bin_tiles[kBins];  // reference tiles of the pairs in each bin
   unsigned long long run_tiles[kBins];  // tally: reference tiles of the blocks run
   uint32_t bin_cnt[kBins];
@@ -176,7 +177,7 @@ struct ngia_db {
   // four-letter sketch: sym_code of launch_sketch_walk (0: off)
   uint32_t walk_code = 0;
   // graph workspace
-  ngia::DevBuf flags, pos, sums, jobs, ekeys, escores, ekeys_tmp, escores_tmp, fin_temp;
+  ngia::DevBuf flags, pos, sums, jobs, degree, edge_off, ekeys, escores, ekeys_tmp, escores_tmp, fin_temp;
   ngia::DevBuf counters, cnt, keep, off, pairs, score, bin_of, list, plain_scratch, plain_jobs,
       bucket_scratch;
   uint64_t n_edges = 0, n_pairs = 0;

@@ -277,10 +277,12 @@ __global__ __launch_bounds__(256) void k_pair_count(const uint32_t* __restrict__
                                                     uint32_t t0, uint32_t bands, float thr,
                                                     FastRound fast, uint32_t* __restrict__ cnt,
                                                     uint64_t* __restrict__ keep_out,
+                                                    uint32_t* __restrict__ degree,
                                                     unsigned long long* __restrict__ total) {
   __shared__ uint32_t tile[64][65];
   __shared__ unsigned long long btotal;
   const uint32_t i0 = blockIdx.x * 64;
+  if (degree && threadIdx.x < 64 && i0 + threadIdx.x < n) degree[i0 + threadIdx.x] = 0;
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (threadIdx.x == 0) btotal = 0;
@@ -358,10 +360,10 @@ __global__ __launch_bounds__(256) void k_pair_emit(const uint32_t* __restrict__ 
 }
 
 void pair_count(const uint32_t* rep, const uint32_t* len, uint32_t n, uint32_t t0, uint32_t bands,
-                float thr, uint32_t* cnt, uint64_t* keep, unsigned long long* total, hipStream_t s,
-                const FastRound& fast) {
+                float thr, uint32_t* cnt, uint64_t* keep, uint32_t* degree,
+                unsigned long long* total, hipStream_t s, const FastRound& fast) {
   hipLaunchKernelGGL(k_pair_count, dim3((n + 63) / 64), dim3(256), 0, s, rep, len, n, t0, bands,
-                     thr, fast, cnt, keep, total);
+                     thr, fast, cnt, keep, degree, total);
   NGIA_HIP(hipGetLastError());
 }
 
@@ -707,6 +709,131 @@ void pairs_to_edges(const uint2* pairs, const uint64_t* npairs, const uint32_t* 
                     hipStream_t s) {
   hipLaunchKernelGGL(k_pairs_to_edges, dim3(grid), dim3(256), 0, s, pairs, npairs, score, ekeys,
                      escores, ecount);
+  NGIA_HIP(hipGetLastError());
+}
+
+// ------------------------------------------------------------- edge list
+// The sorted edge list of a batched round, whose pairs are distinct: a counting
+// sort by u, then each edge's place among its u's by the number of smaller v.
+//  1. k_edge_count: a passing pair takes the next slot of its u (kept in
+//     slot[p]) in degree[], zero beforehand (k_pair_count);
+//  2. off = prefix sums of degree;
+//  3. k_edge_scatter: its key and score to off[u] + slot;
+//  4. k_edge_rank: from there to off[u] + its rank.
+// The host reads no count in between.  A round with a u of more than kMaxDegree
+// edges (max_degree says so; steps 3 and 4 return at once) is sorted by
+// pairs_to_edges and finalize_edges instead, since a rank costs its u's degree.
+// Rows of the bucketing give a u at most one edge per band; only a caller's own
+// rows pass kMaxDegree.
+// Bound: latency of a few dependent passes, and for the counting the atomics' round
+// trip (16 in flight a thread: 200,000 16S reads, 6 million pairs, 80 us with
+// four, 32 so).  Before: compaction, a host synchronisation, a radix or merge
+// sort of the 64-bit keys and a unique pass with nothing to drop.  Kernels from
+// the last score to the list: 10,000 proteins at -i 70 20 us in 6 (130 in 13
+// with the gaps), 1 million at -i 50 180 us (430).
+__global__ __launch_bounds__(256) void k_edge_count(const uint2* __restrict__ pairs,
+                                                    const uint64_t* __restrict__ npairs,
+                                                    const uint32_t* __restrict__ score,
+                                                    uint32_t* __restrict__ degree,
+                                                    uint32_t* __restrict__ slot,
+                                                    unsigned long long* __restrict__ ecount,
+                                                    unsigned long long* __restrict__ max_degree) {
+  __shared__ uint32_t edges, over;
+  if (threadIdx.x == 0) edges = over = 0;
+  __syncthreads();
+  const uint64_t P = *npairs;
+  uint32_t mine = 0, most = 0;
+  constexpr int kPer = 16;  // pairs a thread at a time; one at a time waits on memory for each
+  for (uint64_t base = (uint64_t)blockIdx.x * 256 * kPer; base < P;
+       base += (uint64_t)gridDim.x * 256 * kPer) {
+    uint32_t u[kPer], on = 0;
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      const uint64_t p = base + (uint64_t)k * 256 + threadIdx.x;
+      on |= (uint32_t)(p < P && score[p] != 0u) << k;
+    }
+    #pragma unroll
+    for (int k = 0; k < kPer; k++)
+      if (on >> k & 1) u[k] = pairs[base + (uint64_t)k * 256 + threadIdx.x].x;
+    #pragma unroll
+    for (int k = 0; k < kPer; k++)
+      if (on >> k & 1) u[k] = atomicAdd(&degree[u[k]], 1u);
+    #pragma unroll
+    for (int k = 0; k < kPer; k++) {
+      if (!(on >> k & 1)) continue;
+      slot[base + (uint64_t)k * 256 + threadIdx.x] = u[k];
+      most = u[k] + 1 > most ? u[k] + 1 : most;
+    }
+    mine += __popc(on);
+  }
+  for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o);
+  if ((threadIdx.x & 63) == 0 && mine) atomicAdd(&edges, mine);
+  if (most > kMaxDegree) atomicMax(&over, most);
+  __syncthreads();
+  if (threadIdx.x == 0 && edges) atomicAdd(ecount, (unsigned long long)edges);
+  if (threadIdx.x == 0 && over) atomicMax(max_degree, (unsigned long long)over);
+}
+
+__global__ __launch_bounds__(256) void k_edge_scatter(const uint2* __restrict__ pairs,
+                                                      const uint64_t* __restrict__ npairs,
+                                                      const uint32_t* __restrict__ score,
+                                                      const uint64_t* __restrict__ off,
+                                                      const uint32_t* __restrict__ slot,
+                                                      const unsigned long long* __restrict__ max_degree,
+                                                      uint64_t* __restrict__ keys,
+                                                      uint32_t* __restrict__ scores) {
+  if (*max_degree > kMaxDegree) return;
+  const uint64_t P = *npairs;
+  for (uint64_t p = (uint64_t)blockIdx.x * 256 + threadIdx.x; p < P; p += (uint64_t)gridDim.x * 256) {
+    const uint32_t sc = score[p];
+    if (sc == 0) continue;
+    const uint2 pr = pairs[p];
+    const uint64_t at = off[pr.x] + slot[p];
+    keys[at] = ((uint64_t)pr.x << 32) | pr.y;
+    scores[at] = sc;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_edge_rank(const uint64_t* __restrict__ off, uint32_t n,
+                                                   const unsigned long long* __restrict__ max_degree,
+                                                   const uint64_t* __restrict__ keys_in,
+                                                   const uint32_t* __restrict__ scores_in,
+                                                   uint64_t* __restrict__ keys,
+                                                   uint32_t* __restrict__ scores) {
+  if (*max_degree > kMaxDegree) return;
+  const uint64_t m = off[n];
+  for (uint64_t e = (uint64_t)blockIdx.x * 256 + threadIdx.x; e < m; e += (uint64_t)gridDim.x * 256) {
+    const uint64_t key = keys_in[e];
+    const uint32_t sc = scores_in[e], u = (uint32_t)(key >> 32);
+    const uint64_t first = off[u], end = off[u + 1];
+    uint64_t at = first;
+    for (uint64_t j = first; j < end; j++) at += keys_in[j] < key;
+    keys[at] = key;
+    scores[at] = sc;
+  }
+}
+
+void edge_count(const uint2* pairs, const uint64_t* npairs, const uint32_t* score, uint32_t* degree,
+                uint32_t* slot, unsigned long long* ecount, unsigned long long* max_degree,
+                uint32_t grid, hipStream_t s) {
+  hipLaunchKernelGGL(k_edge_count, dim3(grid), dim3(256), 0, s, pairs, npairs, score, degree, slot,
+                     ecount, max_degree);
+  NGIA_HIP(hipGetLastError());
+}
+
+void edge_scatter(const uint2* pairs, const uint64_t* npairs, const uint32_t* score,
+                  const uint64_t* off, const uint32_t* slot, const unsigned long long* max_degree,
+                  uint64_t* keys, uint32_t* scores, uint32_t grid, hipStream_t s) {
+  hipLaunchKernelGGL(k_edge_scatter, dim3(grid), dim3(256), 0, s, pairs, npairs, score, off, slot,
+                     max_degree, keys, scores);
+  NGIA_HIP(hipGetLastError());
+}
+
+void edge_rank(const uint64_t* off, uint32_t n, const unsigned long long* max_degree,
+               const uint64_t* keys_in, const uint32_t* scores_in, uint64_t* keys, uint32_t* scores,
+               uint32_t grid, hipStream_t s) {
+  hipLaunchKernelGGL(k_edge_rank, dim3(grid), dim3(256), 0, s, off, n, max_degree, keys_in, scores_in,
+                     keys, scores);
   NGIA_HIP(hipGetLastError());
 }
 

@@ -168,9 +168,10 @@ void fast_resolve(uint32_t n, const uint64_t* off, const uint2* pairs, const uin
 // keep[i] (the bands whose representatives are kept) and adds the count with
 // duplicates to *total; after cnt is scanned into off, the emit pass writes
 // the pairs grouped by target, in target order.  Targets below t0 get none.
+// degree, when not null: n words cleared for edge_count.
 void pair_count(const uint32_t* rep, const uint32_t* len, uint32_t n, uint32_t t0, uint32_t bands,
-                float thr, uint32_t* cnt, uint64_t* keep, unsigned long long* total, hipStream_t s,
-                const FastRound& fast = FastRound());
+                float thr, uint32_t* cnt, uint64_t* keep, uint32_t* degree,
+                unsigned long long* total, hipStream_t s, const FastRound& fast = FastRound());
 void pair_emit(const uint32_t* rep, uint32_t n, uint32_t bands, const uint64_t* keep,
                const uint64_t* off, uint2* pairs, hipStream_t s);
 void bin_pairs(const uint2* pairs, const uint64_t* npairs, const uint32_t* len, float thr,
@@ -197,6 +198,20 @@ void plain_bin_scores(const uint32_t* list, const uint32_t* bin_off, const uint3
 void pairs_to_edges(const uint2* pairs, const uint64_t* npairs, const uint32_t* score,
                     uint64_t* ekeys, uint32_t* escores, unsigned long long* ecount, uint32_t grid,
                     hipStream_t s);
+
+// The sorted edge list of distinct pairs without a sort (dev_graph.hip); off =
+// prefix sums of degree (scan_u32), keys_in / scores_in what edge_scatter wrote.
+// More edges of one u than this: max_degree tells, and nothing is written.
+constexpr uint32_t kMaxDegree = 1024;
+void edge_count(const uint2* pairs, const uint64_t* npairs, const uint32_t* score, uint32_t* degree,
+                uint32_t* slot, unsigned long long* ecount, unsigned long long* max_degree,
+                uint32_t grid, hipStream_t s);
+void edge_scatter(const uint2* pairs, const uint64_t* npairs, const uint32_t* score,
+                  const uint64_t* off, const uint32_t* slot, const unsigned long long* max_degree,
+                  uint64_t* keys, uint32_t* scores, uint32_t grid, hipStream_t s);
+void edge_rank(const uint64_t* off, uint32_t n, const unsigned long long* max_degree,
+               const uint64_t* keys_in, const uint32_t* scores_in, uint64_t* keys, uint32_t* scores,
+               uint32_t grid, hipStream_t s);
 
 // Sort + unique of m raw edges in place (keys/scores); *d_unique = count.
 // The keys are u << 32 | v with u, v < n: the sort skips the bits above

@@ -1,0 +1,54 @@
+"""The sorted edge list of a batched round, against the oracle: no edges, one
+edge, many per record, and a record with as many edges as the ranking takes,
+one more and many more (rows given by the caller: every record below a star's
+head), which the sort takes."""
+import numpy as np
+import pytest
+
+import ngia2_amd as ng
+import oracle_lib as orc
+from conftest import AMINO, mutate
+
+pytestmark = pytest.mark.gpu
+
+
+def database(n, seed, length=60):
+    """Close copies of one ancestor, longest first."""
+    rng = np.random.default_rng(seed)
+    anc = bytes(AMINO[i] for i in rng.integers(20, size=length))
+    seqs = sorted((mutate(rng, anc, 0.03, 0.005) for _ in range(n)), key=len, reverse=True)
+    packed, off = orc.pack_many(seqs)
+    return packed, off, np.array([len(s) for s in seqs], dtype=np.uint32)
+
+
+@pytest.mark.parametrize("edges", [0, 1, 63, 64, 1023, 1024, 1025, 1026, 5000])
+def test_star(ctx, edges):
+    n = edges + 40
+    packed, off, lengths = database(n, edges + 1)
+    rep = np.tile(np.arange(n, dtype=np.uint32), (64, 1))
+    rng = np.random.default_rng(edges)
+    tars = rng.permutation(np.arange(1, n))[:edges]
+    rep[rng.integers(0, 64, edges), tars] = 0  # the star's rays, each in some band
+    rep[5, n - 20:] = n - 30 + (np.arange(20, dtype=np.uint32) // 4)  # and a few more heads
+    want, tot = orc.build_graph(packed, off, lengths, rep, 64, 50)
+    print("star of", edges, len(want), flush=True)
+    db = ng.Database(ctx, packed, off, lengths)
+    db.set_reps(rep, 64)
+    for mode in (ng.GRAPH_BATCHED, ng.GRAPH_BATCHED, ng.GRAPH_BATCHED_EAGER):
+        st = db.graph(50, 64, mode)
+        np.testing.assert_array_equal(db.edges(), want)
+        assert st["n_edges"] == len(want) and st["total_pairs"] == tot
+    db.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 1023, 1024, 1025, 4100])
+def test_sizes(ctx, n):
+    """Rows of the bucketing itself: every record has up to 64 edges."""
+    packed, off, lengths = database(n, n)
+    print("edge list", n, flush=True)
+    rep = orc.bucket(orc.sketch_all(packed, off))
+    want, _ = orc.build_graph(packed, off, lengths, rep, 64, 80)
+    db = ng.Database(ctx, packed, off, lengths)
+    db.step(80, 64)
+    np.testing.assert_array_equal(db.edges(), want)
+    db.close()
