@@ -30,95 +30,119 @@ void fill_u32(uint32_t* p, uint32_t v, uint64_t count, hipStream_t s) {
 }
 
 // ------------------------------------------------------------------ scan
-// Exclusive scan of n uint32 into n+1 uint64 (out[n] = total), three passes
-// of 4096-element tiles.
+// Exclusive scan of n uint32 into n+1 uint64 (out[n] = total), both at 16-byte
+// aligned addresses, over tiles of 4,096.  A tile's block adds up what lies before it: the sums of the tiles
+// (k_scan_reduce), or, up to kScanDirect elements, the elements themselves, in
+// one launch.  A pass of its own for the tiles' prefix, which a single block
+// took, cost a step two more launches: 10,000 elements 17 us in three, 1 million
+// 23; now
 constexpr uint32_t kScanTile = 4096;
+constexpr uint32_t kScanDirect = 4 * kScanTile;
+
+__device__ inline uint64_t wave_sum(uint64_t x) {
+  #pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+  return x;
+}
 
 __global__ __launch_bounds__(256) void k_scan_reduce(const uint32_t* __restrict__ in, uint32_t n,
                                                      uint64_t* __restrict__ sums) {
-  __shared__ uint64_t red[256];
+  __shared__ uint64_t red[4];
   const uint64_t base = (uint64_t)blockIdx.x * kScanTile;
   uint64_t s = 0;
-  for (uint32_t k = threadIdx.x; k < kScanTile; k += 256)
-    if (base + k < n) s += in[base + k];
-  red[threadIdx.x] = s;
+  #pragma unroll
+  for (uint32_t k = 0; k < kScanTile / 256; k++) {
+    const uint64_t i = base + 256 * k + threadIdx.x;
+    if (i < n) s += in[i];
+  }
+  s = wave_sum(s);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
   __syncthreads();
-  for (uint32_t w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) sums[blockIdx.x] = red[0];
-}
-
-// Single block of four wavefronts (a block that needs a whole CU's wave
-// slots waits behind any concurrent kernel that fills the CUs): exclusive
-// scan of nb block sums in chunks of 256.
-__global__ __launch_bounds__(256) void k_scan_sums(uint64_t* __restrict__ sums, uint32_t nb) {
-  __shared__ uint64_t sh[256];
-  uint64_t carry = 0;
-  for (uint32_t c0 = 0; c0 < nb; c0 += 256) {
-    const uint32_t i = c0 + threadIdx.x;
-    const uint64_t v = i < nb ? sums[i] : 0;
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (uint32_t off = 1; off < 256; off <<= 1) {
-      const uint64_t t = threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-      __syncthreads();
-      sh[threadIdx.x] += t;
-      __syncthreads();
-    }
-    if (i < nb) sums[i] = carry + sh[threadIdx.x] - v;
-    const uint64_t tot = sh[255];
-    __syncthreads();
-    carry += tot;
-  }
-  if (threadIdx.x == 0) sums[nb] = carry;
+  if (threadIdx.x == 0) sums[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
 __global__ __launch_bounds__(256) void k_scan_apply(const uint32_t* __restrict__ in, uint32_t n,
                                                     const uint64_t* __restrict__ sums,
-                                                    uint64_t* __restrict__ out, uint32_t nb) {
-  __shared__ uint64_t sh[256];
+                                                    uint64_t* __restrict__ out) {
+  __shared__ uint64_t red[4], sh[4];
+  const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const uint64_t base = (uint64_t)blockIdx.x * kScanTile;
   // each thread owns 16 consecutive elements
-  const uint64_t mine = base + (uint64_t)threadIdx.x * 16;
+  const uint64_t mine = base + (uint64_t)t * 16;
   uint32_t v[16];
+  const bool full = mine + 16 <= n;
+  if (full) {
+    #pragma unroll
+    for (int k = 0; k < 4; k++) {
+      const uint4 q = ((const uint4*)(in + mine))[k];
+      v[4 * k] = q.x;
+      v[4 * k + 1] = q.y;
+      v[4 * k + 2] = q.z;
+      v[4 * k + 3] = q.w;
+    }
+  } else {
+    #pragma unroll
+    for (int k = 0; k < 16; k++) {
+      const uint32_t q = n ? in[mine + k < n ? mine + k : n - 1] : 0u;
+      v[k] = mine + k < n ? q : 0u;
+    }
+  }
+  uint64_t before = 0;
+  if (sums) {
+    for (uint32_t k = t; k < blockIdx.x; k += 256) before += sums[k];
+  } else {  // every load before the first sum: each waits for another XCD's write
+    uint32_t b[kScanDirect / kScanTile - 1][kScanTile / 256];
+    #pragma unroll
+    for (uint32_t tile = 0; tile < kScanDirect / kScanTile - 1; tile++)
+      #pragma unroll
+      for (uint32_t k = 0; k < kScanTile / 256; k++)
+        b[tile][k] = tile < blockIdx.x ? in[tile * kScanTile + 256 * k + t] : 0u;
+    #pragma unroll
+    for (uint32_t tile = 0; tile < kScanDirect / kScanTile - 1; tile++)
+      #pragma unroll
+      for (uint32_t k = 0; k < kScanTile / 256; k++) before += b[tile][k];
+  }
+  before = wave_sum(before);
   uint64_t s = 0;
   #pragma unroll
-  for (int k = 0; k < 16; k++) {
-    v[k] = (mine + k < n) ? in[mine + k] : 0u;
-    s += v[k];
+  for (int k = 0; k < 16; k++) s += v[k];
+  uint64_t x = s;  // inclusive prefix over the wavefront
+  #pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint64_t y = __shfl_up(x, o);
+    if (lane >= (uint32_t)o) x += y;
   }
-  sh[threadIdx.x] = s;
+  if (lane == 0) red[wave] = before;
+  if (lane == 63) sh[wave] = x;
   __syncthreads();
-  for (uint32_t off = 1; off < 256; off <<= 1) {
-    const uint64_t t = threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-    __syncthreads();
-    sh[threadIdx.x] += t;
-    __syncthreads();
-  }
-  uint64_t run = sums[blockIdx.x] + sh[threadIdx.x] - s;
+  uint64_t run = red[0] + red[1] + red[2] + red[3] + x - s;
+  for (uint32_t w = 0; w < wave; w++) run += sh[w];
+  uint64_t o[16];
   #pragma unroll
   for (int k = 0; k < 16; k++) {
-    if (mine + k < n) out[mine + k] = run;
+    o[k] = run;
     run += v[k];
   }
-  if (blockIdx.x == nb - 1 && threadIdx.x == 0) out[n] = sums[nb];
+  if (full) {
+    #pragma unroll
+    for (int k = 0; k < 8; k++)
+      ((ulonglong2*)(out + mine))[k] = make_ulonglong2(o[2 * k], o[2 * k + 1]);
+  } else {
+    #pragma unroll
+    for (int k = 0; k < 16; k++)
+      if (mine + k < n) out[mine + k] = o[k];
+  }
+  if (blockIdx.x == gridDim.x - 1 && t == 255) out[n] = run;
 }
 
 uint64_t scan_scratch_words(uint32_t n) { return (n + kScanTile - 1) / kScanTile + 2; }
 
 void scan_u32(const uint32_t* in, uint32_t n, uint64_t* out, uint64_t* sums, hipStream_t s) {
-  const uint32_t nb = (n + kScanTile - 1) / kScanTile;
-  if (nb == 0) {
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(256), 0, s, sums, 0u);
-    // out[0] = 0 via a one-element copy of sums[0] (= 0 after k_scan_sums)
-    NGIA_HIP(hipMemcpyAsync(out, sums, 8, hipMemcpyDeviceToDevice, s));
-    return;
-  }
-  hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, s, in, n, sums);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(256), 0, s, sums, nb);
-  hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, s, in, n, sums, out, nb);
+  const uint32_t nb = n ? (n + kScanTile - 1) / kScanTile : 1u;
+  const bool direct = n <= kScanDirect;
+  if (!direct) hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(256), 0, s, in, n, sums);
+  hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(256), 0, s, in, n,
+                     direct ? (const uint64_t*)nullptr : sums, out);
   NGIA_HIP(hipGetLastError());
 }
 

@@ -41,9 +41,10 @@ def test_star(ctx, edges):
     db.close()
 
 
-@pytest.mark.parametrize("n", [1, 2, 255, 1023, 1024, 1025, 4100])
+@pytest.mark.parametrize("n", [1, 2, 255, 1023, 1024, 1025, 4095, 4096, 4097, 16384, 16385, 16390])
 def test_sizes(ctx, n):
-    """Rows of the bucketing itself: every record has up to 64 edges."""
+    """Rows of the bucketing itself: every record has up to 64 edges; the prefix
+    sums' tiles of 4,096 and their forms on either side of 16,384."""
     packed, off, lengths = database(n, n)
     print("edge list", n, flush=True)
     rep = orc.bucket(orc.sketch_all(packed, off))
