@@ -840,6 +840,7 @@ extern "C" int ngia_open(int device, ngia_ctx** out) {
     for (auto& e : ctx->ev) NGIA_HIP(hipEventCreate(&e));
     for (auto& q : ctx->side) NGIA_HIP(hipStreamCreateWithFlags(&q, hipStreamNonBlocking));
     NGIA_HIP(hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming));
+    for (auto& e : ctx->stage_ev) NGIA_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     for (auto& e : ctx->join) NGIA_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     for (auto& e : ctx->bin_ev) NGIA_HIP(hipEventCreate(&e));
     NGIA_HIP(hipEventCreateWithFlags(&ctx->head_rows, hipEventDisableTiming));
@@ -960,11 +961,11 @@ extern "C" int ngia_db_set_reps(ngia_ctx* ctx, ngia_db* db, const uint32_t* rep_
   if (!ctx || !db || !rep_rows) return fail(ctx, NGIA_ERR_ARG, "null argument");
   if (bands < 1 || bands > NGIA_BANDS) return fail(ctx, NGIA_ERR_ARG, "bands should be 1-64");
   const uint64_t m = (uint64_t)bands * db->n;
-  for (uint64_t k = 0; k < m; k++)
-    if (rep_rows[k] >= db->n) return fail(ctx, NGIA_ERR_ARG, "representative index out of range");
+  if (!all_below(rep_rows, m, db->n))
+    return fail(ctx, NGIA_ERR_ARG, "representative index out of range");
   return guarded(ctx, [&] {
     db->rep.ensure(256ull * std::max<uint32_t>(db->n, 1));
-    h2d(db->rep.p, rep_rows, 4 * m, ctx->stream);
+    to_device(ctx, db->rep.p, rep_rows, 4 * m);
     NGIA_HIP(hipStreamSynchronize(ctx->stream));
     db->rep_bands = bands;
     drop_graphs(db);
@@ -976,8 +977,7 @@ extern "C" int ngia_db_get_sigs(ngia_ctx* ctx, ngia_db* db, uint32_t* sig) {
   if (!ctx || !db || !sig) return fail(ctx, NGIA_ERR_ARG, "null argument");
   if (!db->have_sig) return fail(ctx, NGIA_ERR_STATE, "no signatures");
   return guarded(ctx, [&] {
-    d2h(sig, db->sig.p, 256ull * db->n, ctx->stream);
-    NGIA_HIP(hipStreamSynchronize(ctx->stream));
+    to_host(ctx, sig, db->sig.p, 256ull * db->n);
     return NGIA_OK;
   });
 }
@@ -986,8 +986,7 @@ extern "C" int ngia_db_get_reps(ngia_ctx* ctx, ngia_db* db, uint32_t* rep) {
   if (!ctx || !db || !rep) return fail(ctx, NGIA_ERR_ARG, "null argument");
   if (!db->rep_bands) return fail(ctx, NGIA_ERR_STATE, "no representative rows");
   return guarded(ctx, [&] {
-    d2h(rep, db->rep.p, 4ull * db->rep_bands * db->n, ctx->stream);
-    NGIA_HIP(hipStreamSynchronize(ctx->stream));
+    to_host(ctx, rep, db->rep.p, 4ull * db->rep_bands * db->n);
     return NGIA_OK;
   });
 }
@@ -1062,9 +1061,8 @@ extern "C" int ngia_db_get_edges(ngia_ctx* ctx, ngia_db* db, ngia_edge* out, uin
     const uint64_t m = db->n_edges;
     std::vector<uint64_t> k(m);
     std::vector<uint32_t> sc(m);
-    d2h(k.data(), db->ekeys.p, 8 * m, ctx->stream);
-    d2h(sc.data(), db->escores.p, 4 * m, ctx->stream);
-    NGIA_HIP(hipStreamSynchronize(ctx->stream));
+    to_host(ctx, k.data(), db->ekeys.p, 8 * m);
+    to_host(ctx, sc.data(), db->escores.p, 4 * m);
     for (uint64_t e = 0; e < m; e++) {
       out[e].u = (int32_t)(uint32_t)(k[e] >> 32);
       out[e].v = (int32_t)(uint32_t)k[e];
@@ -1203,14 +1201,13 @@ extern "C" int ngia_bucket(ngia_ctx* ctx, const uint32_t* sig, uint32_t n, uint3
     dsig.ensure(256ull * n);
     drep.ensure(256ull * n);
     scratch.ensure(bucket_scratch_bytes(n, ctx->bucket_wide));
-    h2d(dsig.p, sig, 256ull * n, ctx->stream);
+    to_device(ctx, dsig.p, sig, 256ull * n);
     if (ctx->bucket_small && n <= kBucketSmallMax)
       launch_bucket_small(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, ctx->stream);
     else
       launch_bucket(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, ctx->stream,
                     ctx->bucket_wide);
-    d2h(rep, drep.p, 256ull * n, ctx->stream);
-    NGIA_HIP(hipStreamSynchronize(ctx->stream));
+    to_host(ctx, rep, drep.p, 256ull * n);
     return NGIA_OK;
   });
 }

@@ -51,4 +51,9 @@ void pack_records(const uint8_t* res, const uint64_t* res_off, const uint32_t* r
                   uint32_t first, uint32_t count, const uint64_t* word_pos, uint64_t word_base,
                   uint32_t* dst);
 
+// memcpy by several threads, for copies of hundreds of kilobytes and more.
+void copy_parallel(void* dst, const void* src, size_t bytes);
+// Whether all of v[0..m) are below limit.
+bool all_below(const uint32_t* v, uint64_t m, uint32_t limit);
+
 }  // namespace ngia

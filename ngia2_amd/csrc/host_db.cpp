@@ -64,6 +64,23 @@ void pack_records(const uint8_t* res, const uint64_t* res_off, const uint32_t* r
   }
 }
 
+void copy_parallel(void* dst, const void* src, size_t bytes) {
+  constexpr size_t kPart = 128 << 10;
+  const int64_t parts = (int64_t)((bytes + kPart - 1) / kPart);
+  #pragma omp parallel for schedule(static) if (parts > 1)
+  for (int64_t p = 0; p < parts; p++) {
+    const size_t at = (size_t)p * kPart;
+    std::memcpy((char*)dst + at, (const char*)src + at, std::min(kPart, bytes - at));
+  }
+}
+
+bool all_below(const uint32_t* v, uint64_t m, uint32_t limit) {
+  int over = 0;
+  #pragma omp parallel for schedule(static) reduction(| : over) if (m > 100000)
+  for (int64_t k = 0; k < (int64_t)m; k++) over |= v[k] >= limit;
+  return !over;
+}
+
 namespace {
 struct MappedFile {
   const uint8_t* data = nullptr;
