@@ -1058,15 +1058,21 @@ extern "C" int ngia_db_get_edges(ngia_ctx* ctx, ngia_db* db, ngia_edge* out, uin
   if (!out) return NGIA_OK;
   if (cap < db->n_edges) return fail(ctx, NGIA_ERR_ARG, "edge buffer too small");
   return guarded(ctx, [&] {
-    const uint64_t m = db->n_edges;
-    std::vector<uint64_t> k(m);
-    std::vector<uint32_t> sc(m);
-    to_host(ctx, k.data(), db->ekeys.p, 8 * m);
-    to_host(ctx, sc.data(), db->escores.p, 4 * m);
-    for (uint64_t e = 0; e < m; e++) {
-      out[e].u = (int32_t)(uint32_t)(k[e] >> 32);
-      out[e].v = (int32_t)(uint32_t)k[e];
-      out[e].w = (float)sc[e] / 100.0f;  // buildGraph.hpp:346
+    // made on the device, in the list's scratch when it is large enough
+    const uint64_t m = db->n_edges, bytes = sizeof(ngia_edge) * m;
+    static_assert(sizeof(ngia_edge) == 12, "three words an edge");
+    DevBuf own;
+    if (db->ekeys_tmp.bytes < bytes) own.ensure(bytes);
+    uint32_t* rec = db->ekeys_tmp.bytes < bytes ? own.as<uint32_t>() : db->ekeys_tmp.as<uint32_t>();
+    // a short list straight to pinned memory, without a copy command
+    const bool direct = bytes <= kPinEdgeBytes;
+    if (direct) rec = (uint32_t*)(ctx->pin + kPinEdges);
+    edge_records(db->ekeys.as<uint64_t>(), db->escores.as<uint32_t>(), m, rec, ctx->stream);
+    if (direct) {
+      NGIA_HIP(hipStreamSynchronize(ctx->stream));
+      if (bytes) std::memcpy(out, rec, bytes);
+    } else {
+      to_host(ctx, out, rec, bytes);
     }
     return NGIA_OK;
   });

@@ -81,7 +81,8 @@ constexpr size_t kCounterStats = offsetof(Counters, queue);
 // Offsets into ngia_ctx::pin.
 constexpr size_t kPinOverflow = 0, kPinUnique = 8, kPinPairs = 16, kPinHeadPairs = 24,
                  kPinCnt = 64, kPinCounters = 512, kPinHeadCounters = kPinCounters + kCounterStats,
-                 kPinBytes = kPinHeadCounters + kCounterStats;
+                 kPinEdges = (kPinHeadCounters + kCounterStats + 63) / 64 * 64,
+                 kPinEdgeBytes = 64 << 10, kPinBytes = kPinEdges + kPinEdgeBytes;
 static_assert(kPinCnt + 4 * kBins <= kPinCounters, "pinned slots overlap");
 
 }  // namespace ngia

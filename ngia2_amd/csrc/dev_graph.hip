@@ -861,6 +861,27 @@ void edge_rank(const uint64_t* off, uint32_t n, const unsigned long long* max_de
   NGIA_HIP(hipGetLastError());
 }
 
+// Edges as the caller gets them, 12 bytes each, a word a thread.
+__global__ __launch_bounds__(256) void k_edge_records(const uint64_t* __restrict__ keys,
+                                                      const uint32_t* __restrict__ scores,
+                                                      uint64_t m, uint32_t* __restrict__ out) {
+  for (uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x; t < 3 * m; t += (uint64_t)gridDim.x * 256) {
+    const uint64_t e = t / 3;
+    const uint32_t k = (uint32_t)(t - 3 * e);
+    out[t] = k == 0   ? (uint32_t)(keys[e] >> 32)
+             : k == 1 ? (uint32_t)keys[e]
+                      : __float_as_uint((float)scores[e] / 100.0f);  // buildGraph.hpp:346
+  }
+}
+
+void edge_records(const uint64_t* keys, const uint32_t* scores, uint64_t m, uint32_t* out,
+                  hipStream_t s) {
+  if (m == 0) return;
+  hipLaunchKernelGGL(k_edge_records, dim3((uint32_t)std::min<uint64_t>((3 * m + 255) / 256, 16384)),
+                     dim3(256), 0, s, keys, scores, m, out);
+  NGIA_HIP(hipGetLastError());
+}
+
 // ------------------------------------------------------------- finalize
 // Sort the raw edges by (u,v) and drop duplicates (buildGraph.hpp:355-362):
 // the score is a function of (u,v), so unique by key equals the reference's

@@ -213,6 +213,10 @@ void edge_rank(const uint64_t* off, uint32_t n, const unsigned long long* max_de
                const uint64_t* keys_in, const uint32_t* scores_in, uint64_t* keys, uint32_t* scores,
                uint32_t grid, hipStream_t s);
 
+// m edges as (u, v, (float)score / 100) records of three words.
+void edge_records(const uint64_t* keys, const uint32_t* scores, uint64_t m, uint32_t* out,
+                  hipStream_t s);
+
 // Sort + unique of m raw edges in place (keys/scores); *d_unique = count.
 // The keys are u << 32 | v with u, v < n: the sort skips the bits above
 // 32 + bits(n - 1).
