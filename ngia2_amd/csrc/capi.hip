@@ -629,7 +629,8 @@ void bucket_rows(ngia_ctx* ctx, ngia_db* db, hipStream_t s) {
                         s);
   else
     launch_bucket(db->sig.as<uint32_t>(), db->n, db->rep.as<uint32_t>(), db->bucket_scratch.p, s,
-                  ctx->bucket_wide, db->compact, (uint32_t*)(ctx->pin + kPinOverflow));
+                  ctx->bucket_wide, db->compact ? dna_values(db->n, db->mean_len) : Values::kMany,
+                  (uint32_t*)(ctx->pin + kPinOverflow));
 }
 
 // The head of a step: the leading run of records whose own band window (the
@@ -822,6 +823,8 @@ extern "C" int ngia_open(int device, ngia_ctx** out) {
     if (ctx->head_min < 1) ctx->head_min = 1;
     const char* bs = std::getenv("NGIA_BUCKET_SMALL");
     ctx->bucket_small = bs && bs[0] == '1';
+    const char* bf = std::getenv("NGIA_BUCKET_FEW");
+    ctx->bucket_few = bf && bf[0] == '1';
     const char* s2 = std::getenv("NGIA_SEG2_MIN");
     ctx->seg2_min = s2 ? (uint32_t)std::strtoul(s2, nullptr, 10) : kSeg2MinPairs;
     const char* lf = std::getenv("NGIA_LANE_FILL");
@@ -1212,7 +1215,7 @@ extern "C" int ngia_bucket(ngia_ctx* ctx, const uint32_t* sig, uint32_t n, uint3
       launch_bucket_small(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, ctx->stream);
     else
       launch_bucket(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, ctx->stream,
-                    ctx->bucket_wide);
+                    ctx->bucket_wide, ctx->bucket_few ? Values::kTable : Values::kMany);
     to_host(ctx, rep, drep.p, 256ull * n);
     return NGIA_OK;
   });

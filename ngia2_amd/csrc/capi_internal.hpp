@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <functional>
 #include <memory>
+#include <numeric>
 #include <cstddef>
 #include <cstdlib>
 #include <cstring>
@@ -109,6 +110,9 @@ struct ngia_ctx {
   // NGIA_BUCKET_SMALL=1: ngia_bucket takes the small bucketing
   // of a step's head whenever n <= kBucketSmallMax (a check of that path)
   bool bucket_small = false;
+  // NGIA_BUCKET_FEW=1: ngia_bucket first tries the bucketing of few values, as
+  // databases of a compact alphabet do
+  bool bucket_few = false;
   // fewest head records that ngia_db_step splits off (env NGIA_HEAD_MIN),
   // and the narrowest own band window of a head record, in words (env
   // NGIA_HEAD_WINDOW, at least 32: every head pair must go to a wavefront bin)
@@ -174,6 +178,7 @@ struct ngia_db {
   uint32_t n = 0;
   uint64_t n_words = 0;
   uint32_t max_len = 0;
+  double mean_len = 0;
   uint32_t rep_bands = 0;
   bool have_sig = false;
   ngia::DevBuf packed, word_off, lengths, codes, code_off, sig, rep;
@@ -384,6 +389,7 @@ inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64
   }
   validate_records(packed, n_words, word_off, lengths, n, &db->max_len);
   db->host_len.assign(lengths, lengths + n);
+  db->mean_len = n ? std::accumulate(lengths, lengths + n, 0.0) / n : 0.0;
   db->head.reset();
   db->fast.reset();
   db->n = n;

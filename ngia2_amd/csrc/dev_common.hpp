@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 #include <string>
 
@@ -80,16 +81,27 @@ __host__ __device__ inline uint32_t lcs_score(uint32_t lcs, uint32_t R, uint32_t
 // scratch holds bucket_scratch_bytes(n, force_wide) bytes; force_wide selects
 // the 38-bit-key full sort that large n needs anyway.  Below that, n up to
 // 2.8M takes the partitioned form, which synchronises the stream once (to
-// learn whether a partition overflowed and the full sort must run instead).
-// few_values skips the partitioned form: signatures that take few distinct
-// values per band (8-mers of an alphabet of at most five letters, DNA among
-// them, have at most 5^8 values and their minima crowd near the smallest
-// hashes) make long runs of equal signatures that overflow any partition.
+// learn whether a partition had too many values and the full sort must run).
+// 8-mers of an alphabet of at most five letters, DNA among them, have at most
+// 5^8 values, their minima crowd near the smallest hashes, and the long runs of
+// equal signatures outgrow any partition: kFew takes the full sort, kTable
+// tries tables of each band's values first, with a synchronisation of its own.
+enum class Values { kMany, kFew, kTable };
+// kTable or kFew for n records of mean_len residues of four letters.  A band's
+// values are the minima of the 4^8 hashes' ranks over a record's 8-mers, about
+// 4^8 / L ln(n L / 4^8) of them (counted with 20,000 to 1 million random reads of
+// 64 to 1,000 residues: 0.9 to 1.25 of that; related records have fewer).
+// Within the tables: 200,000 16S reads 684 -> 242 us, 2 million 7.3 -> 1.8 ms;
+// past them finding out costs 50 us before a sort of 170 (20,000) to 710.
+inline Values dna_values(uint32_t n, double mean_len) {
+  const double L = mean_len > 1 ? mean_len : 1, kmers = 65536.0;
+  return 1.25 * kmers / L * std::log(1 + n * L / kmers) <= 1400 ? Values::kTable : Values::kFew;
+}
 size_t bucket_scratch_bytes(uint32_t n, bool force_wide = false);
 // pinned_flag (optional): 4 bytes of pinned host memory that receive the
 // overflow flag of the partitioned form.
 void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch,
-                   hipStream_t stream, bool force_wide = false, bool few_values = false,
+                   hipStream_t stream, bool force_wide = false, Values values = Values::kMany,
                    uint32_t* pinned_flag = nullptr);
 // The same rows for n <= kBucketSmallMax records, without a host
 // synchronisation; scratch holds bucket_small_bytes(n) bytes (no more than

@@ -1074,6 +1074,176 @@ void launch_bucket_small(const uint32_t* sig, uint32_t n, uint32_t* rep, void* s
   NGIA_HIP(hipGetLastError());
 }
 
+// ------------------------------------------------ bucketing of few values
+// Signatures of four letters repeat: 200,000 16S reads have about 400 values in
+// a band, 4,500 records the most frequent.  Then a table of a band's values
+// fits LDS, and a record's predecessor is the last record before it with its
+// value's slot:
+//  1. k_mix_columns;
+//  2. k_value_slots: a tile of a band's column through a table in LDS, then its
+//     values into the band's table; each record's slot and each slot's last
+//     record in the tile;
+//  3. k_value_prefix: each slot's last record before each tile;
+//  4. k_value_rows: the records of a tile in order, a wavefront for each 1,024
+//     with a table of its own, as in k_col_map; a record that is its value's
+//     first there takes the last of the wavefronts before, or before the tile.
+// More values than a table holds are noticed, and the full sort takes over.
+// Bound: LDS round trips, one chain of them for every 64 records of a wavefront.
+constexpr uint32_t kValueSlots = 2048, kValueTile = 8192, kValueThreads = 512;
+constexpr uint32_t kValueProbes = 64;
+constexpr uint32_t kValuePer = kValueTile / kValueThreads;
+
+// The slot of h in a table of ~h (0: free; the last slot is h = all ones'), or
+// kValueSlots when it has no room for it.
+__device__ inline uint32_t value_slot(uint32_t* table, uint32_t h) {
+  if (h == 0xFFFFFFFFu) return kValueSlots - 1;
+  uint32_t s = h % (kValueSlots - 1);
+  for (uint32_t probe = 0; probe < kValueProbes; probe++) {
+    uint32_t was = __hip_atomic_load(&table[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (was == 0) was = atomicCAS(&table[s], 0u, ~h);
+    if (was == 0 || was == ~h) return s;
+    s = s + 1 == kValueSlots - 1 ? 0 : s + 1;
+  }
+  return kValueSlots;
+}
+
+__global__ __launch_bounds__(kValueThreads) void k_value_slots(const uint32_t* __restrict__ col,
+                                                               uint32_t n, uint32_t tiles,
+                                                               uint32_t* __restrict__ tables,
+                                                               uint32_t* __restrict__ tile_last,
+                                                               uint16_t* __restrict__ slots,
+                                                               uint32_t* __restrict__ overflow) {
+  __shared__ uint32_t table[kValueSlots], last[kValueSlots], over;
+  __shared__ uint16_t slot_of[kValueTile], to_band[kValueSlots];
+  const uint32_t t = threadIdx.x;
+  uint32_t band, tile;
+  band_block(tiles, &band, &tile);
+  const uint32_t i0 = tile * kValueTile;
+  const uint32_t* const c = col + (uint64_t)band * n;
+  for (uint32_t s = t; s < kValueSlots; s += kValueThreads) table[s] = last[s] = 0;
+  if (t == 0) over = __hip_atomic_load(overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (over) return;  // another tile's: the rows come from elsewhere
+  uint32_t h[kValuePer];
+  #pragma unroll
+  for (uint32_t k = 0; k < kValuePer; k++) {
+    const uint32_t i = i0 + k * kValueThreads + t;
+    h[k] = c[i < n ? i : n - 1];
+  }
+  __syncthreads();
+  #pragma unroll
+  for (uint32_t k = 0; k < kValuePer; k++) {
+    const uint32_t i = i0 + k * kValueThreads + t;
+    if (i >= n) continue;
+    const uint32_t s = value_slot(table, h[k]);
+    if (s == kValueSlots) {
+      over = 1;
+    } else {
+      atomicMax(&last[s], i + 1);
+      slot_of[k * kValueThreads + t] = (uint16_t)s;
+    }
+  }
+  __syncthreads();
+  for (uint32_t s = t; s < kValueSlots && !over; s += kValueThreads) {
+    if (!last[s]) continue;
+    const uint32_t b = value_slot(tables + band * kValueSlots, s == kValueSlots - 1 ? 0xFFFFFFFFu : ~table[s]);
+    if (b == kValueSlots) {
+      over = 1;
+    } else {
+      to_band[s] = (uint16_t)b;
+      tile_last[((uint64_t)band * tiles + tile) * kValueSlots + b] = last[s];
+    }
+  }
+  __syncthreads();
+  if (over) {
+    if (t == 0) atomicOr(overflow, 1u);
+    return;
+  }
+  #pragma unroll
+  for (uint32_t k = 0; k < kValuePer; k++) {
+    const uint32_t q = k * kValueThreads + t;
+    if (i0 + q < n) slots[(uint64_t)band * n + i0 + q] = to_band[slot_of[q]];
+  }
+}
+
+// tile_last[band][tile][slot] -> the same over the tiles before.
+__global__ __launch_bounds__(256) void k_value_prefix(uint32_t tiles, uint32_t* __restrict__ tile_last) {
+  uint32_t* p = tile_last + (uint64_t)blockIdx.y * tiles * kValueSlots + blockIdx.x * 256 + threadIdx.x;
+  uint32_t run = 0;
+  for (uint32_t t0 = 0; t0 < tiles; t0 += 16) {
+    uint32_t v[16];
+    #pragma unroll
+    for (uint32_t k = 0; k < 16; k++) v[k] = t0 + k < tiles ? p[(uint64_t)(t0 + k) * kValueSlots] : 0u;
+    #pragma unroll
+    for (uint32_t k = 0; k < 16; k++) {
+      if (t0 + k >= tiles) break;
+      p[(uint64_t)(t0 + k) * kValueSlots] = run;
+      run = v[k] ? v[k] : run;  // later tiles hold larger indices
+    }
+  }
+}
+
+__global__ __launch_bounds__(kValueThreads) void k_value_rows(const uint16_t* __restrict__ slots,
+                                                              uint32_t n, uint32_t tiles,
+                                                              const uint32_t* __restrict__ before,
+                                                              const uint32_t* __restrict__ overflow,
+                                                              uint32_t* __restrict__ rep) {
+  constexpr uint32_t kWaves = kValueThreads / 64, kSpan = kValueTile / kWaves;
+  __shared__ uint32_t lasts[kWaves][kValueSlots];  // a wavefront's last record of each slot, plus one
+  if (*overflow) return;
+  const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  uint32_t band, tile;
+  band_block(tiles, &band, &tile);
+  const uint32_t i0 = tile * kValueTile;
+  const uint64_t row = (uint64_t)band * n;
+  uint32_t* const last = lasts[w];
+  for (uint32_t s = lane; s < kValueSlots; s += 64) last[s] = 0;
+  uint32_t slot[kValuePer], prev[kValuePer];
+  #pragma unroll
+  for (uint32_t r = 0; r < kValuePer; r++) {
+    const uint32_t i = i0 + w * kSpan + 64 * r + lane;
+    slot[r] = slots[row + (i < n ? i : n - 1)];
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  #pragma unroll
+  for (uint32_t r = 0; r < kValuePer; r++) {
+    const uint32_t q = w * kSpan + 64 * r + lane;
+    const bool on = i0 + q < n;
+    uint32_t now = 0;
+    prev[r] = 0;
+    if (on) {
+      prev[r] = __hip_atomic_load(&last[slot[r]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      atomicMax(&last[slot[r]], q + 1);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      now = __hip_atomic_load(&last[slot[r]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    uint64_t again = __builtin_amdgcn_ballot_w64(on && now != q + 1);
+    while (again) {  // as in k_col_map
+      const uint32_t s = __builtin_amdgcn_readlane(slot[r], __ffsll((unsigned long long)again) - 1);
+      const uint64_t same = __builtin_amdgcn_ballot_w64(on && slot[r] == s);
+      const uint64_t lower = same & ((1ull << lane) - 1ull);
+      if (on && slot[r] == s && lower) prev[r] = w * kSpan + 64 * r + 64 - __clzll(lower);
+      again &= ~same;
+    }
+  }
+  __syncthreads();
+  const uint32_t* const earlier = before + ((uint64_t)band * tiles + tile) * kValueSlots;
+  #pragma unroll
+  for (uint32_t r = 0; r < kValuePer; r++) {
+    const uint32_t i = i0 + w * kSpan + 64 * r + lane;
+    if (i >= n) continue;
+    uint32_t p = prev[r];
+    for (uint32_t v = w; p == 0 && v-- > 0;) p = lasts[v][slot[r]];
+    if (p) {
+      p += i0;
+    } else {
+      p = earlier[slot[r]];
+    }
+    rep[row + i] = p ? p - 1 : i;
+  }
+}
+
 namespace {
 struct BucketLayout {
   bool wide;
@@ -1098,6 +1268,23 @@ PartLayout part_layout(uint32_t n, bool force_wide) {
   L.cursor = L.entries + al(8 * parts * kPartCap);
   L.overflow = L.cursor + al(4 * parts);
   L.total = L.overflow + al(4 * (parts + 2));
+  return L;
+}
+// few values: the column, the slots, and, cleared together, the bands' tables,
+// the overflow flag and the last records by tile
+struct ValueLayout {
+  uint32_t tiles;
+  size_t col, slots, tables, overflow, tile_last, total;
+};
+ValueLayout value_layout(uint32_t n) {
+  auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+  ValueLayout L{};
+  L.tiles = (n + kValueTile - 1) / kValueTile;
+  L.slots = al(256ull * n);
+  L.tables = L.slots + al(128ull * n);
+  L.overflow = L.tables + 4ull * 64 * kValueSlots;
+  L.tile_last = L.overflow + 256;
+  L.total = L.tile_last + 4ull * 64 * kValueSlots * L.tiles;
   return L;
 }
 BucketLayout bucket_layout(uint32_t n, bool force_wide) {
@@ -1125,10 +1312,37 @@ BucketLayout bucket_layout(uint32_t n, bool force_wide) {
 }  // namespace
 
 size_t bucket_scratch_bytes(uint32_t n, bool force_wide) {
-  return std::max(bucket_layout(n, force_wide).total, part_layout(n, force_wide).total);
+  const size_t sorted = std::max(bucket_layout(n, force_wide).total, part_layout(n, force_wide).total);
+  return !force_wide && n <= kPartMaxN ? std::max(sorted, value_layout(n).total) : sorted;
 }
 
 namespace {
+// The bucketing of few values; returns false when there were too many (rep then
+// holds no result).
+bool bucket_values(const uint32_t* sig, uint32_t n, uint32_t* rep, char* s, hipStream_t stream,
+                   uint32_t* pinned_flag) {
+  const ValueLayout L = value_layout(n);
+  uint32_t* col = (uint32_t*)(s + L.col);
+  uint16_t* slots = (uint16_t*)(s + L.slots);
+  uint32_t* tables = (uint32_t*)(s + L.tables);
+  uint32_t* overflow = (uint32_t*)(s + L.overflow);
+  uint32_t* tile_last = (uint32_t*)(s + L.tile_last);
+  fill_u32(tables, 0, (L.total - L.tables) / 4, stream);
+  hipLaunchKernelGGL(k_mix_columns, dim3((n + 63) / 64), dim3(256), 0, stream, sig, n, col, rep);
+  hipLaunchKernelGGL(k_value_slots, dim3(64 * L.tiles), dim3(kValueThreads), 0, stream, col, n, L.tiles,
+                     tables, tile_last, slots, overflow);
+  hipLaunchKernelGGL(k_value_prefix, dim3(kValueSlots / 256, 64), dim3(256), 0, stream, L.tiles,
+                     tile_last);
+  hipLaunchKernelGGL(k_value_rows, dim3(64 * L.tiles), dim3(kValueThreads), 0, stream, slots, n, L.tiles,
+                     tile_last, overflow, rep);
+  NGIA_HIP(hipGetLastError());
+  uint32_t local = 0;
+  uint32_t* over = pinned_flag ? pinned_flag : &local;
+  NGIA_HIP(hipMemcpyAsync(over, overflow, 4, hipMemcpyDeviceToHost, stream));
+  NGIA_HIP(hipStreamSynchronize(stream));
+  return *over == 0;
+}
+
 // The partitioned bucketing; returns false when a partition overflowed (rep
 // then holds a partial result and the caller redoes it with the full sort).
 bool bucket_partitioned(const PartLayout& L, const uint32_t* sig, uint32_t n, uint32_t* rep,
@@ -1159,7 +1373,7 @@ bool bucket_partitioned(const PartLayout& L, const uint32_t* sig, uint32_t n, ui
 }  // namespace
 
 void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch,
-                   hipStream_t stream, bool force_wide, bool few_values, uint32_t* pinned_flag) {
+                   hipStream_t stream, bool force_wide, Values values, uint32_t* pinned_flag) {
   if (n == 0) return;
   const BucketLayout L = bucket_layout(n, force_wide);
   char* s = (char*)scratch;
@@ -1168,7 +1382,9 @@ void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch
   uint32_t* vals_out = (uint32_t*)(s + L.vals_out);
   size_t tb = L.temp_bytes;
   const PartLayout P = part_layout(n, force_wide);
-  if (P.use && !few_values && bucket_partitioned(P, sig, n, rep, s, stream, pinned_flag)) return;
+  if (P.use && values == Values::kTable && bucket_values(sig, n, rep, s, stream, pinned_flag)) return;
+  if (P.use && values == Values::kMany && bucket_partitioned(P, sig, n, rep, s, stream, pinned_flag))
+    return;
   // the full sort (also when a partition overflowed), from the identity rows
   hipLaunchKernelGGL(k_rep_identity, dim3(grid_for(n, 256), 64), dim3(256), 0, stream, n, rep);
   NGIA_HIP(hipGetLastError());

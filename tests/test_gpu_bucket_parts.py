@@ -33,6 +33,17 @@ def small():
     c.close()
 
 
+@pytest.fixture(scope="module")
+def few():
+    os.environ["NGIA_BUCKET_FEW"] = "1"
+    try:
+        c = ng.Context(0)
+    finally:
+        del os.environ["NGIA_BUCKET_FEW"]
+    yield c
+    c.close()
+
+
 def unmix(h):
     """The signature whose mixed value is h: the inverse of the kernel's two
     odd products and two xors with a shift of itself."""
@@ -117,3 +128,31 @@ def test_small_crowded_partition(small, distinct):
         sig[rows, b] = unmix(h[np.arange(len(rows)) % distinct])
     print("small bucketing, crowded partition", distinct, flush=True)
     np.testing.assert_array_equal(small.bucket(sig), orc.bucket(sig))
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 1023, 1024, 1025, 8191, 8192, 8193, 9216, 16385, 139264, 139265])
+def test_few_values(few, n):
+    """The tables of few values: tiles of 8,192, wavefronts of 1,024, rows of
+    64 and, past 16 tiles, the prefix's second round."""
+    rng = np.random.default_rng(n)
+    values = np.array([1, 2, 3, 30, 400, 1000] * 11)[:64]
+    sig = np.empty((n, 64), dtype=np.uint32)
+    for b in range(64):
+        pool = rng.integers(0, 1 << 32, size=values[b], dtype=np.uint64).astype(np.uint32)
+        pool[0] = unmix(np.array([0xFFFFFFFF if b % 2 else 0], dtype=np.uint32))[0]
+        sig[:, b] = pool[(rng.random(n) ** 2 * values[b]).astype(np.int64)]
+    sig[:, 7] = sig[np.arange(n) // 3, 7]
+    print("few values", n, flush=True)
+    np.testing.assert_array_equal(few.bucket(sig), orc.bucket(sig))
+
+
+@pytest.mark.parametrize("values", [1400, 1700, 2046, 2047, 2048, 3000, 20000])
+def test_too_many_values(few, values):
+    """More values than a table takes, in one band or over its tiles."""
+    n = 30000
+    rng = np.random.default_rng(values)
+    sig = rng.integers(0, 300, size=(n, 64)).astype(np.uint32)
+    sig[:, 40] = rng.integers(0, values, n)
+    sig[:, 63] = np.arange(n) // (n // values + 1)  # few in a tile
+    print("too many values", values, flush=True)
+    np.testing.assert_array_equal(few.bucket(sig), orc.bucket(sig))
