@@ -465,15 +465,36 @@ __global__ __launch_bounds__(64) void k_bin_offsets(uint32_t* __restrict__ bin_c
                                                     unsigned long long* __restrict__ bin_tiles,
                                                     RouteTable route, uint32_t seg2_min,
                                                     uint32_t lane_fill, bool compact) {
-  __shared__ uint32_t cnt[kBins], to_bin[kBins], off[kBins + 1];
+  __shared__ uint32_t cnt[kBins], to_bin[kBins], off[64];
   __shared__ unsigned long long tiles[kBins];
-  static_assert(kBins <= 64, "one thread per bin");
+  static_assert(kBins < 64, "one thread per bin, and one for the end");
   const uint32_t t = threadIdx.x;
   if (t < (uint32_t)kBins) {
     cnt[t] = bin_cnt[t];
     tiles[t] = bin_tiles[t];
     to_bin[t] = t;
     cursor[t] = 0;
+  }
+  const bool lanes_off = lane_fill == 0xFFFFFFFFu;
+  // the tiles of the bins that a lane per pair could take past kWinLds words
+  const uint64_t total = wave_sum(bin_width((int)t) > kWinLds && t < (uint32_t)kBins ? bin_tiles[t] : 0ull);
+  if (route.class_size[0] == 0 && !compact && lane_fill != 0 && !lanes_off) {
+    // Few pairs in all: a wavefront each (kWaveAllPairs).
+    const uint32_t c = t > 0 && t < (uint32_t)kBins ? bin_cnt[t] : 0u;
+    const bool narrow = bin_width((int)t) > kWaveAllMin || is_seg_bin((int)t);
+    const uint64_t all = wave_sum(narrow || bin_width((int)t) >= 2 || !c ? c : kWaveAllPairs + 1);
+    if (all <= kWaveAllPairs) {
+      const uint64_t n1 = wave_sum(narrow ? c : 0u), t1 = wave_sum(narrow && c ? bin_tiles[t] : 0ull);
+      if (narrow && c) {
+        to_bin[t] = (uint32_t)kBinWave0;
+        cnt[t] = 0;
+        tiles[t] = 0;
+      }
+      if (t == (uint32_t)kBinWave0) {
+        cnt[t] += (uint32_t)n1;
+        tiles[t] += t1;
+      }
+    }
   }
   __syncthreads();
   if (t == 0) {
@@ -487,9 +508,6 @@ __global__ __launch_bounds__(64) void k_bin_offsets(uint32_t* __restrict__ bin_c
     };
     const bool tuned = route.class_size[0] != 0;
     // Whether one lane per pair pays for `c` pairs of `t` tiles in all.
-    unsigned long long total = 0;
-    for (int W = kWinLds + 1; W <= kLaneMax; W++) total += tiles[lane_bin(W)];
-    const bool lanes_off = lane_fill == 0xFFFFFFFFu;
     auto lanes_pay = [&](uint32_t c, unsigned long long t) {
       const unsigned long long few = (unsigned long long)kLaneTiles * c;
       return !lanes_off && (t <= few || total * c >= (unsigned long long)lane_fill * (t - few));
@@ -544,32 +562,39 @@ __global__ __launch_bounds__(64) void k_bin_offsets(uint32_t* __restrict__ bin_c
     group(31, 31, -1, kBinSeg32, kBinSeg32, -1);
     group(32, kLaneMax, kBinSeg16x3, kBinSeg16x3, kBinWave0, 2);
     group(1, 0, kBinSeg16x4, kBinSeg16x4, kBinWave0, 3);
-    uint32_t s = 0;
-    for (int b = 0; b < kBins; b++) {
-      off[b] = s;
-      s += cnt[b];
-    }
-    off[kBins] = s;
   }
   __syncthreads();
+  const uint32_t c = t < (uint32_t)kBins ? cnt[t] : 0u;
+  uint32_t x = c;
+  #pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(x, o);
+    if (t >= (uint32_t)o) x += y;
+  }
+  off[t] = x - c;
   if (t < (uint32_t)kBins) {
     bin_cnt[t] = cnt[t];
     bin_tiles[t] = tiles[t];
     remap[t] = to_bin[t];
     bin_off[t] = off[t];
   }
-  if (t == 0) bin_off[kBins] = off[kBins];
+  if (t == (uint32_t)kBins) bin_off[t] = off[t];
 }
 
 uint64_t reachable_bins(uint32_t wlo, uint32_t whi, uint64_t pairs, uint32_t kmax,
-                        const RouteTable& route) {
+                        const RouteTable& route, uint32_t lane_fill) {
   uint64_t m = 0;
   auto add = [&](int b) { m |= 1ull << b; };
-  for (uint32_t W = std::max(wlo, 2u); W <= std::min(whi, 60u); W++) {
+  const bool each = !route.class_size[0] && lane_fill != 0 && lane_fill != 0xFFFFFFFFu &&
+                    pairs <= kWaveAllPairs && whi <= 60;  // a wavefront per pair
+  if (each && whi >= 2) add(kBinWave0);
+  for (uint32_t W = std::max(wlo, 2u); each && W <= std::min(whi, (uint32_t)kWaveAllMin); W++)
+    add(lane_bin((int)W));
+  for (uint32_t W = std::max(wlo, 2u); !each && W <= std::min(whi, 60u); W++) {
+    add(kBinWave0);
     if (W <= (uint32_t)kWinMax) {
       if (W > (uint32_t)kWinLds || pairs >= kLowLanePairs) add((int)W);
       add(lane_bin((int)W));
-      add(kBinWave0);
       add(kBinSeg8x2);
       add(kBinSeg32);
       if (route.class_size[0]) add(kBinSeg16);
@@ -580,7 +605,6 @@ uint64_t reachable_bins(uint32_t wlo, uint32_t whi, uint64_t pairs, uint32_t kma
     } else {
       if (W <= (uint32_t)kLaneMax) add(lane_bin((int)W));
       add(W <= 45 ? kBinSeg16x3 : kBinSeg16x4);
-      add(kBinWave0);
     }
   }
   uint32_t from = 61;  // the narrowest window of the next bin

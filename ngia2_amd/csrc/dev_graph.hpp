@@ -77,6 +77,14 @@ constexpr uint32_t kLowLanePairs = 16384;
 // this many pairs among them a wavefront per pair, else the segmented
 // kernels.
 constexpr uint32_t kWavePairs = 2048;
+// At most this many pairs, none of more than 60 words (no tuned table, not a
+// compact alphabet): a wavefront each, past kWaveAllMin words, where a lane takes
+// no longer (3 words 17 us, 5 words 24, a wavefront 20).  The device runs
+// so many at once, and a wavefront ends a pair sooner than anything else.  The
+// step with its pairs, other shapes against this: 500 records, 1,561 pairs 239 / 211
+// us; 500, 2,172 236 / 210; 1,000, 2,289 252 / 241; 1,000, 4,448 253 / 282.
+constexpr uint32_t kWaveAllPairs = 3072;
+constexpr int kWaveAllMin = 4;
 // The segmented bins and their (lanes per pair, words per lane).
 constexpr bool is_seg_bin(int b) { return b >= kBinSeg16 && b <= kBinSeg8x2; }
 constexpr int seg_lanes(int b) {
@@ -134,7 +142,7 @@ __host__ __device__ inline uint32_t route_window_bin(const RouteTable& rt, uint3
 // routing of k_bin_offsets; for callers that launch the bins' kernels without
 // having read the counts.
 uint64_t reachable_bins(uint32_t wlo, uint32_t whi, uint64_t pairs, uint32_t kmax,
-                        const RouteTable& route);
+                        const RouteTable& route, uint32_t lane_fill);
 
 void fill_u32(uint32_t* p, uint32_t v, uint64_t count, hipStream_t s);
 uint64_t scan_scratch_words(uint32_t n);

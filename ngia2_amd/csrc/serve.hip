@@ -546,7 +546,7 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
             ln.score.as<uint32_t>(), sv->ctx->wave_kmax, dc->remap, sv->ctx->route,
             sv->ctx->seg2_min, sv->ctx->lane_fill, false, grid, s);
   // Nothing is read back, so the kernels launched are those of every bin that a
-  // pair with one of these queries could be in: 28 launches for any, 5 for 16
+  // pair with one of these queries could be in: 28 launches for any, two for 16
   // queries of the usual lengths.  A pair's target has T >= R thr residues of
   // its rep's R, and one of the two is a query: its window, lsft / 32 +
   // ceil(rsft / 32) words of band_edges, has lsft + rsft between 2 T (1 - thr)
@@ -555,7 +555,8 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
   const double thr = sv->thr, least = shortest * thr, widest = longest / thr;
   const uint32_t wlo = (uint32_t)std::max(2.0, std::floor(2 * least * (1 - thr) / 32) - 2);
   const uint32_t whi = longest ? (uint32_t)((longest * (1 - thr) + widest - longest * thr + 64) / 32) + 4 : 0u;
-  const uint64_t bins = reachable_bins(wlo, whi, 64ull * Q, sv->ctx->wave_kmax, sv->ctx->route);
+  const uint64_t bins = reachable_bins(wlo, whi, 64ull * Q, sv->ctx->wave_kmax, sv->ctx->route,
+                                       sv->ctx->lane_fill);
   auto reached = [&](int b) { return (bins >> b & 1) != 0; };
   AlignArgs aa;
   aa.packed = sv->packed.as<uint32_t>();
