@@ -477,12 +477,14 @@ __global__ __launch_bounds__(64) void k_bin_offsets(uint32_t* __restrict__ bin_c
   }
   const bool lanes_off = lane_fill == 0xFFFFFFFFu;
   // the tiles of the bins that a lane per pair could take past kWinLds words
-  const uint64_t total = wave_sum(bin_width((int)t) > kWinLds && t < (uint32_t)kBins ? bin_tiles[t] : 0ull);
+  const int width = t < (uint32_t)kBins ? bin_width((int)t) : 0;
+  const uint64_t total = wave_sum(width > kWinLds ? bin_tiles[t] : 0ull);
   if (route.class_size[0] == 0 && !compact && lane_fill != 0 && !lanes_off) {
     // Few pairs in all: a wavefront each (kWaveAllPairs).
     const uint32_t c = t > 0 && t < (uint32_t)kBins ? bin_cnt[t] : 0u;
-    const bool narrow = bin_width((int)t) > kWaveAllMin || is_seg_bin((int)t);
-    const uint64_t all = wave_sum(narrow || bin_width((int)t) >= 2 || !c ? c : kWaveAllPairs + 1);
+    const bool narrow = width > kWaveAllMin || is_seg_bin((int)t);
+    const uint64_t wider = __builtin_amdgcn_ballot_w64(c != 0 && width < 2 && !narrow);
+    const uint64_t all = wider ? ~0ull : wave_sum(c);
     if (all <= kWaveAllPairs) {
       const uint64_t n1 = wave_sum(narrow ? c : 0u), t1 = wave_sum(narrow && c ? bin_tiles[t] : 0ull);
       if (narrow && c) {

@@ -53,3 +53,24 @@ def test_sizes(ctx, n):
     db.step(80, 64)
     np.testing.assert_array_equal(db.edges(), want)
     db.close()
+
+
+@pytest.mark.parametrize("n", [3, 60, 76, 77, 90])
+@pytest.mark.parametrize("length", [60, 300])
+def test_few_pairs(n, length):
+    """Rounds on both sides of 3,072 pairs (rows that pair each record with up to
+    64 before it): a wavefront each, or the usual shapes."""
+    packed, off, lengths = database(n, n, length)
+    rep = np.array([[max(i - 1 - b, 0) for i in range(n)] for b in range(64)], dtype=np.uint32)
+    want, tot = orc.build_graph(packed, off, lengths, rep, 64, 60)
+    print("few pairs", n, length, flush=True)
+    c = ng.Context(0)
+    db = ng.Database(c, packed, off, lengths)
+    db.set_reps(rep, 64)
+    st = db.graph(60, 64)
+    np.testing.assert_array_equal(db.edges(), want)
+    kinds = {b["kind"] for b in db.bin_stats() if b["pairs"]}
+    few = st["distinct_pairs"] <= 3072 and length == 300
+    assert ("wave" in kinds) == few
+    db.close()
+    c.close()

@@ -320,10 +320,14 @@ def test_handles_outlive_their_context(served):
 @pytest.mark.gpu
 @pytest.mark.parametrize("identity", [20, 50, 90, 99])
 @pytest.mark.parametrize("length", [1, 9, 150, 700, 2047, 2049, 4000, 9000])
-def test_serve_batch_of_one_length(ctx, identity, length):
+@pytest.mark.parametrize("tuned", [False, True])
+def test_serve_batch_of_one_length(ctx, identity, length, tuned):
     """Batches whose queries have about one length, against residents as long
     and shorter and longer by up to the identity: only the bins these can reach
-    are launched, and past 2,048 residues the sketch is cut into chunks."""
+    are launched, and past 2,048 residues the sketch is cut into chunks.  A
+    context of its own has no routing table; the shared one may."""
+    if not tuned:
+        ctx = ng.Context(0)
     rng = np.random.default_rng(identity * 10007 + length)
     anc = bytes(AMINO[i] for i in rng.integers(20, size=min(2 * length, 12000) + 40))
     cuts = sorted({max(1, min(len(anc), int(length * f)))
@@ -345,3 +349,5 @@ def test_serve_batch_of_one_length(ctx, identity, length):
     np.testing.assert_array_equal(as_rows(got), want)
     sv.close()
     db.close()
+    if not tuned:
+        ctx.close()
