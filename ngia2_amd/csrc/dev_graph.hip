@@ -669,6 +669,30 @@ void bin_pairs(const uint2* pairs, const uint64_t* npairs, const uint32_t* len, 
   NGIA_HIP(hipGetLastError());
 }
 
+// Job triplets as pairs, and the scores back.
+__global__ __launch_bounds__(256) void k_jobs_to_pairs(const uint32_t* __restrict__ jobs, uint32_t count,
+                                                       uint2* __restrict__ pairs,
+                                                       unsigned long long* __restrict__ npairs) {
+  const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+  if (j == 0) *npairs = count;
+  if (j < count) pairs[j] = make_uint2(jobs[3ull * j], jobs[3ull * j + 1]);
+}
+__global__ __launch_bounds__(256) void k_scores_to_jobs(const uint32_t* __restrict__ score,
+                                                        uint32_t count, uint32_t* __restrict__ jobs) {
+  const uint32_t j = blockIdx.x * 256 + threadIdx.x;
+  if (j < count) jobs[3ull * j + 2] = score[j];
+}
+void jobs_to_pairs(const uint32_t* jobs, uint32_t count, uint2* pairs, unsigned long long* npairs,
+                   hipStream_t s) {
+  hipLaunchKernelGGL(k_jobs_to_pairs, dim3(grid_for(count, 256)), dim3(256), 0, s, jobs, count, pairs,
+                     npairs);
+  NGIA_HIP(hipGetLastError());
+}
+void scores_to_jobs(const uint32_t* score, uint32_t count, uint32_t* jobs, hipStream_t s) {
+  hipLaunchKernelGGL(k_scores_to_jobs, dim3(grid_for(count, 256)), dim3(256), 0, s, score, count, jobs);
+  NGIA_HIP(hipGetLastError());
+}
+
 // Pairs of the plain-kernel bin as job triplets, scores copied back after.
 __global__ void k_bin_to_jobs(const uint2* __restrict__ pairs, const uint32_t* __restrict__ list,
                               const uint32_t* __restrict__ bin_off, const uint32_t* __restrict__ bin_cnt,

@@ -203,6 +203,11 @@ void plain_bin_jobs(const uint2* pairs, const uint32_t* list, const uint32_t* bi
                     const uint32_t* bin_cnt, uint32_t* jobs, hipStream_t s);
 void plain_bin_scores(const uint32_t* list, const uint32_t* bin_off, const uint32_t* bin_cnt,
                       const uint32_t* jobs, uint32_t* score, hipStream_t s);
+// count job triplets (rep, tar, score) as pairs, their number to *npairs; scores
+// back into the triplets.
+void jobs_to_pairs(const uint32_t* jobs, uint32_t count, uint2* pairs, unsigned long long* npairs,
+                   hipStream_t s);
+void scores_to_jobs(const uint32_t* score, uint32_t count, uint32_t* jobs, hipStream_t s);
 void pairs_to_edges(const uint2* pairs, const uint64_t* npairs, const uint32_t* score,
                     uint64_t* ekeys, uint32_t* escores, unsigned long long* ecount, uint32_t grid,
                     hipStream_t s);
