@@ -290,10 +290,17 @@ void fast_resolve(uint32_t n, const uint64_t* off, const uint2* pairs, const uin
 // count with duplicates.
 __device__ inline void load_rep_tile(const uint32_t* __restrict__ rep, uint32_t n, uint32_t bands,
                                      uint32_t i0, uint32_t (&tile)[64][65]) {
-  for (uint32_t e = threadIdx.x; e < 64 * 64; e += 256) {
-    const uint32_t b = e >> 6, t = e & 63;
-    tile[b][t] = (b < bands && i0 + t < n) ? rep[(uint64_t)b * n + i0 + t] : 0u;
+  // all 16 loads of a thread before the first store (unconditional, index 0 where
+  // there is nothing to load): one at a time they took 16 us of a small round
+  const uint32_t t = threadIdx.x & 63u, b0 = threadIdx.x >> 6;
+  uint32_t v[16];
+  #pragma unroll
+  for (uint32_t k = 0; k < 16; k++) {
+    const uint32_t b = b0 + 4 * k;
+    v[k] = rep[b < bands && i0 + t < n ? (uint64_t)b * n + i0 + t : 0u];
   }
+  #pragma unroll
+  for (uint32_t k = 0; k < 16; k++) tile[b0 + 4 * k][t] = v[k];
 }
 
 __global__ __launch_bounds__(256) void k_pair_count(const uint32_t* __restrict__ rep,

@@ -560,10 +560,14 @@ __global__ __launch_bounds__(256) void k_mix_columns(const uint32_t* __restrict_
   __shared__ uint32_t tile[64][65];
   const uint32_t i0 = blockIdx.x * 64;
   const uint32_t t = threadIdx.x;
-  for (uint32_t e = t; e < 64 * 64; e += 256) {
-    const uint32_t si = e >> 6, b = e & 63;
-    tile[si][b] = (i0 + si < n) ? sig[(uint64_t)(i0 + si) * 64 + b] : 0u;
+  uint32_t v[16];  // all loads in flight before the first store
+  #pragma unroll
+  for (uint32_t k = 0; k < 16; k++) {
+    const uint32_t e = t + 256 * k;
+    v[k] = sig[i0 + (e >> 6) < n ? (uint64_t)(i0 + (e >> 6)) * 64 + (e & 63) : 0u];
   }
+  #pragma unroll
+  for (uint32_t k = 0; k < 16; k++) tile[(t + 256 * k) >> 6][t & 63] = v[k];
   __syncthreads();
   for (uint32_t e = t; e < 64 * 64; e += 256) {
     const uint32_t b = e >> 6, si = e & 63;
