@@ -95,7 +95,7 @@ typedef struct {
   double sketch_ms;   /* k_sketch of the last ngia_db_sketch */
   double bucket_ms;   /* transpose + radix sort + predecessor of the last ngia_db_bucket */
   double graph_ms;    /* candidates .. raw edges of the last ngia_db_graph */
-  double finalize_ms; /* sort + unique of the last ngia_db_graph */
+  double finalize_ms; /* the sorted edge list of the last ngia_db_graph */
   double align_ms;    /* alignment bins alone (NGIA_GRAPH_BATCHED_EAGER only, else 0) */
   double step_ms;     /* the whole of the last ngia_db_step */
   uint32_t step_head; /* records in the head round of the last ngia_db_step (0: none) */
