@@ -150,7 +150,7 @@ void graph_plain(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
 // Part 1: candidates and bins (capturable: fixed grids, device-side counts),
 // on stream s; targets from db->t0 on.
 void enqueue_bins(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, hipStream_t s,
-                  const FastRound& fast = FastRound()) {
+                  const FastRound& fast = FastRound(), bool tell = true) {
   const uint32_t n = db->n;
   const float thr = (float)identity / 100.0f;
   Counters* dc = db->counters.as<Counters>();
@@ -166,7 +166,8 @@ void enqueue_bins(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
   bin_pairs(db->pairs.as<uint2>(), npairs, len, thr, db->bin_of.as<uint32_t>(), dc->bin_cnt,
             dc->bin_off, dc->cursor, db->list.as<uint32_t>(), dc->bin_tiles, db->score.as<uint32_t>(),
             ctx->wave_kmax, dc->remap, db->compact ? ctx->route_compact : ctx->route, ctx->seg2_min,
-            ctx->lane_fill, db->compact, grid, s);
+            ctx->lane_fill, db->compact, grid, s,
+            tell ? (uint32_t*)(ctx->pin + kPinCnt) : nullptr);
 }
 
 // Part 2: the alignment kernels of the bins in `mask` (bit b: bin b holds
@@ -417,7 +418,6 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
     NGIA_HIP(hipGraphLaunch(db->gexec, s));
   // the bins that hold pairs pick the second part
   uint32_t cnt[kBins];
-  d2h(ctx->pin + kPinCnt, db->counters.as<Counters>()->bin_cnt, sizeof(cnt), s);
   NGIA_HIP(hipStreamSynchronize(s));
   std::memcpy(cnt, ctx->pin + kPinCnt, sizeof(cnt));
   uint64_t mask = 0;
@@ -466,18 +466,23 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
                    db->edge_off.as<uint64_t>(), of->bin_of.as<uint32_t>(), &dc->max_degree,
                    db->ekeys_tmp.as<uint64_t>(), db->escores_tmp.as<uint32_t>(),
                    pair_grid(ctx, of, bands), s);
-  edge_rank(db->edge_off.as<uint64_t>(), n, &dc->max_degree, db->ekeys_tmp.as<uint64_t>(),
+  auto report = [&](ngia_db* of, size_t counters, size_t pairs) {
+    RoundReport r;
+    if (!of) return r;
+    r.counters = of->counters.as<uint32_t>();
+    r.words = kCounterStats / 4;
+    r.pairs = of->off.as<uint64_t>() + of->n;
+    r.host = (uint32_t*)(ctx->pin + counters);
+    r.host_pairs = (uint64_t*)(ctx->pin + pairs);
+    return r;
+  };
+  edge_rank(report(db, kPinCounters, kPinPairs), report(hd, kPinHeadCounters, kPinHeadPairs),
+            db->edge_off.as<uint64_t>(), n, &dc->max_degree, db->ekeys_tmp.as<uint64_t>(),
             db->escores_tmp.as<uint32_t>(), db->ekeys.as<uint64_t>(), db->escores.as<uint32_t>(),
             pair_grid(ctx, db, bands), s);
   NGIA_HIP(hipEventRecord(ctx->ev[5], s));
   Counters hc, hh{};
   uint64_t npairs = 0, hpairs = 0;
-  d2h(ctx->pin + kPinCounters, db->counters.p, kCounterStats, s);
-  d2h(ctx->pin + kPinPairs, db->off.as<uint64_t>() + n, 8, s);
-  if (hd) {
-    d2h(ctx->pin + kPinHeadCounters, hd->counters.p, kCounterStats, s);
-    d2h(ctx->pin + kPinHeadPairs, hd->off.as<uint64_t>() + hd->n, 8, s);
-  }
   NGIA_HIP(hipStreamSynchronize(s));
   std::memcpy(&hc, ctx->pin + kPinCounters, kCounterStats);
   std::memcpy(&npairs, ctx->pin + kPinPairs, 8);
@@ -602,7 +607,6 @@ uint64_t fast_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t ba
     f.valid = valid.as<uint64_t>();
     f.last = hi == bands;
     enqueue_bins(ctx, db, identity, bands, s, f);
-    d2h(ctx->pin + kPinCnt, db->counters.as<Counters>()->bin_cnt, 4 * kBins, s);
     NGIA_HIP(hipStreamSynchronize(s));
     uint64_t mask = 0;
     for (int b = 0; b < kBins; b++)
@@ -654,8 +658,8 @@ bool align_binned(ngia_ctx* ctx, ngia_db* db, uint32_t* jobs, uint32_t count, fl
             db->bin_of.as<uint32_t>(), dc->bin_cnt, dc->bin_off, dc->cursor, db->list.as<uint32_t>(),
             dc->bin_tiles, db->score.as<uint32_t>(), ctx->wave_kmax, dc->remap,
             db->compact ? ctx->route_compact : ctx->route, ctx->seg2_min, ctx->lane_fill, db->compact,
-            (uint32_t)std::min<uint64_t>(persistent_blocks(ctx, 0) * 4, (c + 255) / 256), s);
-  d2h(ctx->pin + kPinCnt, dc->bin_cnt, 4 * kBins, s);
+            (uint32_t)std::min<uint64_t>(persistent_blocks(ctx, 0) * 4, (c + 255) / 256), s,
+            (uint32_t*)(ctx->pin + kPinCnt));
   NGIA_HIP(hipStreamSynchronize(s));
   uint64_t mask = 0;
   for (int b = 0; b < kBins; b++)
@@ -829,7 +833,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
                          kSketchChunk, sig, q);
     NGIA_HIP(hipEventRecord(ctx->head_rows, q));
     launch_bucket_small(sig, h, hd->rep.as<uint32_t>(), hd->bucket_scratch.p, q);
-    enqueue_bins(ctx, hd, identity, bands, q);
+    enqueue_bins(ctx, hd, identity, bands, q, FastRound(), /*tell=*/false);
     enqueue_scores(ctx, hd, thr, (uint64_t)h * bands, mask, false, false, q, /*serial=*/true);
     NGIA_HIP(hipEventRecord(ctx->head_done, q));
     hr.db = hd;

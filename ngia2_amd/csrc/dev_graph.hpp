@@ -182,11 +182,12 @@ void pair_count(const uint32_t* rep, const uint32_t* len, uint32_t n, uint32_t t
                 unsigned long long* total, hipStream_t s, const FastRound& fast = FastRound());
 void pair_emit(const uint32_t* rep, uint32_t n, uint32_t bands, const uint64_t* keep,
                const uint64_t* off, uint2* pairs, hipStream_t s);
+// bin_pairs: host_cnt, when not null: pinned memory that gets the bin counts.
 void bin_pairs(const uint2* pairs, const uint64_t* npairs, const uint32_t* len, float thr,
                uint32_t* bin_of, uint32_t* bin_cnt, uint32_t* bin_off, uint32_t* cursor,
                uint32_t* list, unsigned long long* bin_tiles, uint32_t* score, uint32_t kmax,
                uint32_t* remap, const RouteTable& route, uint32_t seg2_min, uint32_t lane_fill,
-               bool compact, uint32_t grid, hipStream_t s);
+               bool compact, uint32_t grid, hipStream_t s, uint32_t* host_cnt = nullptr);
 // One lane per pair over the window bins wlo..whi of a width class (0..3:
 // 2-8, 9-16, 17-24 and 25-40 words), widest first; bin_off, bin_cnt, queue
 // (kQueueWords words a bin; the launch uses that of whi) and tally are
@@ -222,9 +223,19 @@ void edge_count(const uint2* pairs, const uint64_t* npairs, const uint32_t* scor
 void edge_scatter(const uint2* pairs, const uint64_t* npairs, const uint32_t* score,
                   const uint64_t* off, const uint32_t* slot, const unsigned long long* max_degree,
                   uint64_t* keys, uint32_t* scores, uint32_t grid, hipStream_t s);
-void edge_rank(const uint64_t* off, uint32_t n, const unsigned long long* max_degree,
-               const uint64_t* keys_in, const uint32_t* scores_in, uint64_t* keys, uint32_t* scores,
-               uint32_t grid, hipStream_t s);
+// What a round's end tells the host, in pinned memory: `words` of its counters and
+// its number of pairs (host null: nothing).
+struct RoundReport {
+  const uint32_t* counters = nullptr;
+  uint32_t words = 0;
+  const uint64_t* pairs = nullptr;
+  uint32_t* host = nullptr;
+  uint64_t* host_pairs = nullptr;
+};
+void edge_rank(const RoundReport& main, const RoundReport& head, const uint64_t* off, uint32_t n,
+               const unsigned long long* max_degree, const uint64_t* keys_in,
+               const uint32_t* scores_in, uint64_t* keys, uint32_t* scores, uint32_t grid,
+               hipStream_t s);
 
 // m edges as (u, v, (float)score / 100) records of three words.
 void edge_records(const uint64_t* keys, const uint32_t* scores, uint64_t m, uint32_t* out,
