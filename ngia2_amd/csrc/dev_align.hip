@@ -182,7 +182,11 @@ __device__ inline void plain_job(const AlignArgs& A, uint32_t* __restrict__ jobs
   const uint32_t* rr = A.packed + A.word_off[rep];
   const uint32_t* tr = A.packed + A.word_off[tar];
   const uint32_t T = tr[0];
-  if (length_rejects(R, T, A.thr)) return;  // score keeps its initial 0
+  if (length_rejects(R, T, A.thr)) {
+    // ngia_align scores it 0; ngia_align_noalloc leaves the caller's value
+    if (!kPlanes) jobs[3 * job + 2] = 0;
+    return;
+  }
   const uint32_t nw = (R + 31) / 32;
   for (uint32_t w = 0; w < nw; w++) rows[(uint64_t)w * stride] = 0xFFFFFFFFu;
   const Band bd = band_edges(R, T, A.thr);

@@ -65,3 +65,20 @@ def test_other_thresholds(ctx, thr):
     print("align threshold", thr, flush=True)
     np.testing.assert_array_equal(ctx.align(packed, off, jobs, thr),
                                   orc.align_jobs(packed, off, jobs, thr))
+
+
+@pytest.mark.parametrize("count", [1, 15, 16, 17, 400])
+@pytest.mark.parametrize("thr", [0.0, 0.7, 1.0, 1.25])
+def test_score_column_is_overwritten(ctx, count, thr):
+    """Whatever the third column holds, a job that the length filter rejects
+    scores 0, like any other that does not pass."""
+    seqs = records(9, AMINO, 8, 400, 80)
+    packed, off = orc.pack_many(seqs)
+    rng = np.random.default_rng(count)
+    jobs = np.zeros((count, 3), dtype=np.uint32)
+    jobs[:, :2] = rng.integers(0, len(seqs), (count, 2))
+    jobs[0, :2] = 0, len(seqs) - 1  # a single residue
+    want = orc.align_jobs(packed, off, jobs, thr)
+    jobs[:, 2] = 77
+    print("align with an old score column", count, thr, flush=True)
+    np.testing.assert_array_equal(ctx.align(packed, off, jobs, thr), want)
