@@ -640,6 +640,7 @@ bool align_binned(ngia_ctx* ctx, ngia_db* db, uint32_t* jobs, uint32_t count, fl
                  at_list = at_bin + al(4 * c), at_cnt = at_list + al(4 * c);
   DevBuf work;
   try {
+    SpareSpace spare(ctx);
     work.ensure(at_cnt + sizeof(Counters));
   } catch (const HipError& e) {
     if (e.code != NGIA_ERR_NOMEM) throw;
@@ -664,19 +665,24 @@ bool align_binned(ngia_ctx* ctx, ngia_db* db, uint32_t* jobs, uint32_t count, fl
   uint64_t mask = 0;
   for (int b = 0; b < kBins; b++)
     if (((const uint32_t*)(ctx->pin + kPinCnt))[b]) mask |= 1ull << b;
+  auto drop_work = [&] {
+    for (DevBuf* b : {&db->pairs, &db->score, &db->bin_of, &db->list, &db->counters}) b->release();
+  };
   try {
+    SpareSpace spare(ctx);
     if ((mask >> kBinPlain) & 1u) {
       db->plain_jobs.ensure(12 * c);
       db->plain_scratch.ensure(4 * align_plain_scratch_words((db->max_len + 31) / 32, kPlainBinBlocks));
     }
   } catch (const HipError& e) {
     if (e.code != NGIA_ERR_NOMEM) throw;
+    drop_work();
     return false;
   }
   enqueue_scores(ctx, db, thr, c, mask, false, false, s, /*serial=*/false);
   scores_to_jobs(db->score.as<uint32_t>(), count, jobs, s);
   NGIA_HIP(hipStreamSynchronize(s));  // the workspace goes
-  for (DevBuf* b : {&db->pairs, &db->score, &db->bin_of, &db->list, &db->counters}) b->release();
+  drop_work();
   return true;
 }
 
@@ -897,6 +903,8 @@ extern "C" int ngia_open(int device, ngia_ctx** out) {
     ctx->raw_lcs = rl && rl[0] == '1';
     const char* fa = std::getenv("NGIA_FULL_ALPHABET");
     ctx->full_alphabet = fa && fa[0] == '1';
+    const char* sl = std::getenv("NGIA_SPARE_LIMIT");
+    if (sl) ctx->spare_limit = (size_t)std::strtoull(sl, nullptr, 10);
     NGIA_HIP(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     NGIA_HIP(hipHostMalloc((void**)&ctx->pin, kPinBytes, hipHostMallocDefault));
     std::memset(ctx->pin, 0, kPinBytes);
@@ -1226,7 +1234,6 @@ extern "C" int ngia_db_fast(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint3
         ensure_pair_space(fast_db(ctx, db), bands);
       } catch (const HipError& e) {
         if (e.code != NGIA_ERR_NOMEM) throw;
-        (void)hipGetLastError();
         db->fast.reset();
         batched = false;
       }

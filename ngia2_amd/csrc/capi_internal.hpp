@@ -22,6 +22,10 @@ namespace ngia {
 
 constexpr int kSideStreams = 4;
 
+// Largest allocation, in bytes, that the running call's spare workspaces may
+// make on this thread (SpareSpace).
+inline thread_local size_t spare_limit = ~(size_t)0;
+
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
@@ -49,9 +53,14 @@ struct DevBuf {
     if (!owned) throw HipError{NGIA_ERR_ARG, "a view buffer cannot grow"};
     release();
     size_t want = b < 256 ? 256 : (b + 255) & ~(size_t)255;
+    // past the limit: more than any device has, which the runtime refuses
+    if (want > spare_limit) want = (size_t)1 << 60;
     hipError_t e = hipMalloc(&p, want);
     if (e != hipSuccess) {
       p = nullptr;
+      // A caller may go on without the memory: the runtime keeps the error, and the
+      // check after the next launch would report it.
+      (void)hipGetLastError();
       throw HipError{NGIA_ERR_NOMEM, "hipMalloc(" + std::to_string(want) + " bytes) failed: " +
                                          hipGetErrorString(e)};
     }
@@ -132,6 +141,9 @@ struct ngia_ctx {
   // env NGIA_FULL_ALPHABET=1: the window kernels keep the 16-code table even
   // for a compact alphabet
   bool full_alphabet = false;
+  // largest allocation of a workspace that a call can do without (env
+  // NGIA_SPARE_LIMIT, bytes: a check of the forms that need less memory)
+  size_t spare_limit = ~(size_t)0;
   // the 8-mer lists of the four-letter sketch (k_walk_table), for the letters
   // of walk_code (0: none yet); used on the context stream only
   ngia::DevBuf walk_table;
@@ -172,6 +184,18 @@ struct ngia_ctx {
     if (stage) (void)hipHostFree(stage);
   }
 };
+
+namespace ngia {
+// While one lives, this thread allocates workspace that the call has a form
+// without.
+struct SpareSpace {
+  const size_t was = spare_limit;
+  explicit SpareSpace(const ngia_ctx* ctx) { spare_limit = ctx->spare_limit; }
+  ~SpareSpace() { spare_limit = was; }
+  SpareSpace(const SpareSpace&) = delete;
+  SpareSpace& operator=(const SpareSpace&) = delete;
+};
+}  // namespace ngia
 
 struct ngia_db {
   ngia_ctx* ctx = nullptr;
