@@ -1225,23 +1225,27 @@ extern "C" int ngia_db_fast(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint3
       if (total_pairs) *total_pairs = 0;
       return NGIA_OK;
     }
-    // The pair lists take 1.3 KiB per record at 64 bands; without the memory
-    // (or past 2^32 pairs) the bands run one by one.
+    // The pair lists take 1.3 KiB per record at 64 bands, the job list of pairs
+    // with the widest windows 0.8; without the memory (or past 2^32 pairs) the
+    // bands run one by one.
     bool batched = (uint64_t)n * bands < (1ull << 32);
     uint64_t total = 0;
+    db->have_bins = false;
     if (batched) {
       try {
+        SpareSpace spare(ctx);
         ensure_pair_space(fast_db(ctx, db), bands);
+        total = fast_batched(ctx, db->fast.get(), identity, bands, parent.as<uint32_t>());
       } catch (const HipError& e) {
         if (e.code != NGIA_ERR_NOMEM) throw;
+        // a round may have run: its kernels end, and its parents go
+        NGIA_HIP(hipStreamSynchronize(ctx->stream));
         db->fast.reset();
+        fill_u32(parent.as<uint32_t>(), 0xFFFFFFFFu, n, ctx->stream);
         batched = false;
       }
     }
-    db->have_bins = false;
-    if (batched) {
-      total = fast_batched(ctx, db->fast.get(), identity, bands, parent.as<uint32_t>());
-    } else {
+    if (!batched) {
       ngia_graph_stats st{};
       graph_plain(ctx, db, identity, bands, &st, parent.as<uint32_t>());
       total = st.total_pairs;

@@ -43,3 +43,35 @@ def test_align(limit):
         for _ in range(2):
             np.testing.assert_array_equal(c.align(packed, off, jobs, 0.1), want)
 
+
+def plain_fast(c, packed, off, lengths, rep, bands, identity):
+    db = ng.Database(c, packed, off, lengths)
+    db.set_reps(rep, 64)
+    got, tot = db.fast(identity, bands)
+    again, tot2 = db.fast(identity, bands)
+    db.close()
+    want, wtot = orc.fast_cluster(packed, off, lengths, rep, bands, identity)
+    assert tot == tot2 == wtot
+    np.testing.assert_array_equal(got, want)
+    np.testing.assert_array_equal(again, want)
+    return want
+
+
+@pytest.mark.parametrize("cfg,scale,identity,bands", [(1, 0.1, 50, 64), (1, 0.1, 95, 64), (2, 0.052, 85, 17),
+                                                      (4, 0.005, 90, 64), (3, 0.002, 97, 64), (1, 0.1, 70, 1)])
+def test_fast_band_by_band(cfg, scale, identity, bands):
+    d = ng.gen_packed(ng.gen_config(cfg, scale, 5))
+    rep = orc.bucket(orc.sketch_all(d.packed, d.word_off))
+    say("fast mode band by band, config", cfg, scale, "identity", identity, "bands", bands)
+    with limited(0) as c:
+        plain_fast(c, d.packed, d.word_off, d.lengths, rep, bands, identity)
+
+
+@pytest.mark.parametrize("limit", [0, 1 << 20])
+def test_fast_long(limit):
+    packed, off, lengths = long_set()
+    rep = np.tile(np.maximum(np.arange(4, dtype=np.int64) - 1, 0).astype(np.uint32), (64, 1))
+    say("fast mode without its workspace", limit)
+    with limited(limit) as c:
+        want = plain_fast(c, packed, off, lengths, rep, 8, 10)
+    assert (want == 0).all()
