@@ -567,10 +567,9 @@ constexpr uint32_t kFastBands = 8;
 constexpr uint32_t kFastSplit = 50000;
 // The database of the fast mode: db's records and rows (views) with a round
 // workspace of its own, since the pairs and scores of db's last graph stay
-// readable.
-ngia_db* fast_db(ngia_ctx* ctx, ngia_db* db) {
-  if (!db->fast) db->fast = std::make_unique<ngia_db>();
-  ngia_db* f = db->fast.get();
+// readable.  What the last fast call left (`kept`) is used again.
+std::unique_ptr<ngia_db> fast_db(ngia_ctx* ctx, ngia_db* db, std::unique_ptr<ngia_db> kept) {
+  std::unique_ptr<ngia_db> f = kept ? std::move(kept) : std::make_unique<ngia_db>();
   f->ctx = ctx;
   f->n = db->n;
   f->n_words = db->n_words;
@@ -954,6 +953,13 @@ extern "C" int ngia_device_query(ngia_ctx* ctx, ngia_device_info* info) {
   });
 }
 
+namespace ngia {
+void give_back_kept(ngia_ctx* ctx) {
+  const CallScope call(ctx);
+  (void)give_back();
+}
+}  // namespace ngia
+
 extern "C" int ngia_get_timing(ngia_ctx* ctx, ngia_timing* out) {
   if (!ctx || !out) return fail(ctx, NGIA_ERR_ARG, "null argument");
   *out = ctx->timing;
@@ -1234,13 +1240,14 @@ extern "C" int ngia_db_fast(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint3
     if (batched) {
       try {
         SpareSpace spare(ctx);
-        ensure_pair_space(fast_db(ctx, db), bands);
-        total = fast_batched(ctx, db->fast.get(), identity, bands, parent.as<uint32_t>());
+        std::unique_ptr<ngia_db> f = fast_db(ctx, db, std::move(db->fast));
+        ensure_pair_space(f.get(), bands);
+        total = fast_batched(ctx, f.get(), identity, bands, parent.as<uint32_t>());
+        db->fast = std::move(f);
       } catch (const HipError& e) {
         if (e.code != NGIA_ERR_NOMEM) throw;
         // a round may have run: its kernels end, and its parents go
         NGIA_HIP(hipStreamSynchronize(ctx->stream));
-        db->fast.reset();
         fill_u32(parent.as<uint32_t>(), 0xFFFFFFFFu, n, ctx->stream);
         batched = false;
       }

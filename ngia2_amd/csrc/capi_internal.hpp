@@ -26,6 +26,10 @@ constexpr int kSideStreams = 4;
 // make on this thread (SpareSpace).
 inline thread_local size_t spare_limit = ~(size_t)0;
 
+// Frees workspaces that the running call's context only keeps for a later call;
+// whether there were any.
+inline bool give_back();
+
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
@@ -56,6 +60,7 @@ struct DevBuf {
     // past the limit: more than any device has, which the runtime refuses
     if (want > spare_limit) want = (size_t)1 << 60;
     hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess && give_back()) e = hipMalloc(&p, want);
     if (e != hipSuccess) {
       p = nullptr;
       // A caller may go on without the memory: the runtime keeps the error, and the
@@ -238,7 +243,8 @@ struct ngia_db {
   // this database's records, codes and signatures and its own rows and
   // round workspace
   std::unique_ptr<ngia_db> head;
-  // the fast mode's round workspace (ngia_db_fast), with views likewise
+  // the fast mode's round workspace (ngia_db_fast), with views likewise; null
+  // while a fast call uses it
   std::unique_ptr<ngia_db> fast;
   // (head only) its records' sketch in chunks of positions: (record, first
   // position) per chunk
@@ -257,6 +263,29 @@ inline void drop_graphs(ngia_db* db) {
   for (auto& e : db->gexec2) (void)hipGraphExecDestroy(e.second);
   db->gexec2.clear();
 }
+
+namespace ngia {
+// The context of the call this thread runs.
+inline thread_local ngia_ctx* call_ctx = nullptr;
+struct CallScope {
+  ngia_ctx* const was = call_ctx;
+  explicit CallScope(ngia_ctx* ctx) { call_ctx = ctx; }
+  ~CallScope() { call_ctx = was; }
+  CallScope(const CallScope&) = delete;
+  CallScope& operator=(const CallScope&) = delete;
+};
+
+inline bool give_back() {
+  bool any = false;
+  if (call_ctx)
+    for (ngia_db* db : call_ctx->dbs)
+      if (db->fast) {
+        db->fast.reset();
+        any = true;
+      }
+  return any;
+}
+}  // namespace ngia
 
 // Called by ngia_close for each live serving handle (serve.hip).
 void serve_detach(ngia_serve* sv);
@@ -277,6 +306,7 @@ inline int fail(ngia_ctx* ctx, int code, const std::string& msg) {
 
 template <class F>
 inline int guarded(ngia_ctx* ctx, F&& f) {
+  const CallScope call(ctx);
   try {
     return f();
   } catch (const HipError& e) {

@@ -85,6 +85,7 @@ extern "C" int ngia_build_graph_chunked(ngia_ctx* ctx, const uint32_t* packed, u
   uint32_t brec = 0;
   if (bw == 0) {
     ngia_device_info info;
+    give_back_kept(ctx);
     int rc = ngia_device_query(ctx, &info);
     if (rc != NGIA_OK) return rc;
     const uint64_t budget = info.hbm_free / 4;  // per block

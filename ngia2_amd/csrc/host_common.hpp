@@ -51,6 +51,10 @@ void pack_records(const uint8_t* res, const uint64_t* res_off, const uint32_t* r
                   uint32_t first, uint32_t count, const uint64_t* word_pos, uint64_t word_base,
                   uint32_t* dst);
 
+// Frees device workspaces that ctx only keeps for a later call, before its free
+// memory is asked for.
+void give_back_kept(ngia_ctx* ctx);
+
 // memcpy by several threads, for copies of hundreds of kilobytes and more.
 void copy_parallel(void* dst, const void* src, size_t bytes);
 // Whether all of v[0..m) are below limit.

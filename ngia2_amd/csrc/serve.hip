@@ -381,6 +381,7 @@ void serve_setup(ngia_serve* sv, ngia_db* db, const uint32_t* cluster_of,
   NGIA_HIP(hipMemGetInfo(&free_b, &total_b));
   const uint64_t need = 4 * (sv->res_words + sv->grow_words) + 24 * slots + sv->res_codes +
                         sv->grow_codes + 8 * tslots + 4ull * sv->grow_q;
+  if (need > free_b && give_back()) NGIA_HIP(hipMemGetInfo(&free_b, &total_b));
   if (need > free_b)
     throw HipError{NGIA_ERR_NOMEM, "snapshot and grown part (" + std::to_string(need >> 20) +
                                        " MiB) exceed the free HBM (" + std::to_string(free_b >> 20) +

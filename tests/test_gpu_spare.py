@@ -75,3 +75,25 @@ def test_fast_long(limit):
     with limited(limit) as c:
         want = plain_fast(c, packed, off, lengths, rep, 8, 10)
     assert (want == 0).all()
+
+
+def test_fast_workspace_is_given_back():
+    """An allocation that fails takes back what fast calls of other databases
+    keep: 100,000 records' pair lists of 130 MB."""
+    n = 100000
+    rng = np.random.default_rng(2)
+    packed, off = orc.pack_many([bytes(AMINO[i] for i in rng.integers(20, size=16)) for _ in range(1000)])
+    off = np.tile(off, n // 1000)
+    rep = np.tile(np.maximum(np.arange(n, dtype=np.int64) - 1000, 0).astype(np.uint32), (64, 1))
+    jobs = np.zeros((3000000, 3), dtype=np.uint32)
+    say("fast workspace given back")
+    with limited(52 << 20) as c:
+        db = ng.Database(c, packed, off)
+        db.set_reps(rep, 64)
+        first, _ = db.fast(90)
+        held = c.info()["hbm_free"]
+        assert (c.align(packed, off[:1], jobs, 0.9)[:, 2] == 100).all()
+        assert c.info()["hbm_free"] > held + (100 << 20)
+        again, _ = db.fast(90)
+        db.close()
+    np.testing.assert_array_equal(again, first)
