@@ -685,6 +685,18 @@ bool align_binned(ngia_ctx* ctx, ngia_db* db, uint32_t* jobs, uint32_t count, fl
   return true;
 }
 
+// Scratch for the bucketing of n records: for all of its forms, or without the
+// memory for the full sort.
+void ensure_bucket_scratch(ngia_ctx* ctx, DevBuf* scratch, uint32_t n) {
+  try {
+    SpareSpace spare(ctx);
+    scratch->ensure(bucket_scratch_bytes(n, ctx->bucket_wide));
+  } catch (const HipError& e) {
+    if (e.code != NGIA_ERR_NOMEM) throw;
+    scratch->ensure(bucket_sort_bytes(n, ctx->bucket_wide));
+  }
+}
+
 // The database's representative rows from its signatures: the small form (no
 // host synchronisation) up to kBucketSmallMax records, partitions or the full
 // sort beyond (the latter always under NGIA_BUCKET_WIDE).
@@ -693,8 +705,8 @@ void bucket_rows(ngia_ctx* ctx, ngia_db* db, hipStream_t s) {
     launch_bucket_small(db->sig.as<uint32_t>(), db->n, db->rep.as<uint32_t>(), db->bucket_scratch.p,
                         s);
   else
-    launch_bucket(db->sig.as<uint32_t>(), db->n, db->rep.as<uint32_t>(), db->bucket_scratch.p, s,
-                  ctx->bucket_wide, db->compact ? dna_values(db->n, db->mean_len) : Values::kMany,
+    launch_bucket(db->sig.as<uint32_t>(), db->n, db->rep.as<uint32_t>(), db->bucket_scratch.p,
+                  db->bucket_scratch.bytes, s, ctx->bucket_wide, db->compact ? dna_values(db->n, db->mean_len) : Values::kMany,
                   (uint32_t*)(ctx->pin + kPinOverflow));
 }
 
@@ -806,7 +818,7 @@ void graph_step(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands, b
   const float thr = (float)identity / 100.0f;
   db->sig.ensure(256ull * n);
   db->rep.ensure(256ull * n);
-  db->bucket_scratch.ensure(bucket_scratch_bytes(n, ctx->bucket_wide));
+  ensure_bucket_scratch(ctx, &db->bucket_scratch, n);
   uint32_t h = split ? head_records(db, thr, ctx->head_window) : 0u;
   if (h < ctx->head_min || h >= n) h = 0;  // too few to pay for the split, or nothing beside them
   const uint8_t* codes = db->codes.as<uint8_t>();
@@ -1022,7 +1034,7 @@ extern "C" int ngia_db_bucket(ngia_ctx* ctx, ngia_db* db) {
   if (!db->have_sig) return fail(ctx, NGIA_ERR_STATE, "bucket before sketch");
   return guarded(ctx, [&] {
     db->rep.ensure(256ull * std::max<uint32_t>(db->n, 1));
-    db->bucket_scratch.ensure(bucket_scratch_bytes(db->n, ctx->bucket_wide));
+    ensure_bucket_scratch(ctx, &db->bucket_scratch, db->n);
     NGIA_HIP(hipEventRecord(ctx->ev[6], ctx->stream));
     bucket_rows(ctx, db, ctx->stream);
     NGIA_HIP(hipEventRecord(ctx->ev[7], ctx->stream));
@@ -1287,12 +1299,12 @@ extern "C" int ngia_bucket(ngia_ctx* ctx, const uint32_t* sig, uint32_t n, uint3
     DevBuf dsig, drep, scratch;
     dsig.ensure(256ull * n);
     drep.ensure(256ull * n);
-    scratch.ensure(bucket_scratch_bytes(n, ctx->bucket_wide));
+    ensure_bucket_scratch(ctx, &scratch, n);
     to_device(ctx, dsig.p, sig, 256ull * n);
     if (ctx->bucket_small && n <= kBucketSmallMax)
       launch_bucket_small(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, ctx->stream);
     else
-      launch_bucket(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, ctx->stream,
+      launch_bucket(dsig.as<uint32_t>(), n, drep.as<uint32_t>(), scratch.p, scratch.bytes, ctx->stream,
                     ctx->bucket_wide, ctx->bucket_few ? Values::kTable : Values::kMany);
     to_host(ctx, rep, drep.p, 256ull * n);
     return NGIA_OK;

@@ -78,7 +78,7 @@ __host__ __device__ inline uint32_t lcs_score(uint32_t lcs, uint32_t R, uint32_t
 // All take device pointers and run on `stream`.
 
 // Band-major bucketing of n x 64 signatures into 64 x n representative rows.
-// scratch holds bucket_scratch_bytes(n, force_wide) bytes; force_wide selects
+// scratch holds `bytes`, bucket_scratch_bytes(n, force_wide) at best; force_wide selects
 // the 38-bit-key full sort that large n needs anyway.  Below that, n up to
 // 2.8M takes the partitioned form, which synchronises the stream once (to
 // learn whether a partition had too many values and the full sort must run).
@@ -98,9 +98,14 @@ inline Values dna_values(uint32_t n, double mean_len) {
   return 1.25 * kmers / L * std::log(1 + n * L / kmers) <= 1400 ? Values::kTable : Values::kFew;
 }
 size_t bucket_scratch_bytes(uint32_t n, bool force_wide = false);
+// What the full sort alone needs, which launch_bucket takes when `bytes` of scratch
+// do not hold the other forms: just past a step in the number of partitions, these
+// and the column take 2.3 KB a record (2.1 million records 4.8 GB), the sort's keys
+// and values 1.
+size_t bucket_sort_bytes(uint32_t n, bool force_wide = false);
 // pinned_flag (optional): 4 bytes of pinned host memory that receive the
 // overflow flag of the partitioned form.
-void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch,
+void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch, size_t bytes,
                    hipStream_t stream, bool force_wide = false, Values values = Values::kMany,
                    uint32_t* pinned_flag = nullptr);
 // The same rows for n <= kBucketSmallMax records, without a host

@@ -1320,6 +1320,8 @@ size_t bucket_scratch_bytes(uint32_t n, bool force_wide) {
   return !force_wide && n <= kPartMaxN ? std::max(sorted, value_layout(n).total) : sorted;
 }
 
+size_t bucket_sort_bytes(uint32_t n, bool force_wide) { return bucket_layout(n, force_wide).total; }
+
 namespace {
 // The bucketing of few values; returns false when there were too many (rep then
 // holds no result).
@@ -1376,18 +1378,21 @@ bool bucket_partitioned(const PartLayout& L, const uint32_t* sig, uint32_t n, ui
 }
 }  // namespace
 
-void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch,
+void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch, size_t bytes,
                    hipStream_t stream, bool force_wide, Values values, uint32_t* pinned_flag) {
   if (n == 0) return;
   const BucketLayout L = bucket_layout(n, force_wide);
+  if (bytes < L.total) throw HipError{NGIA_ERR_ARG, "bucketing scratch too small"};
   char* s = (char*)scratch;
   const uint64_t m = (uint64_t)n * 64;
   uint32_t* vals_in = (uint32_t*)(s + L.vals_in);
   uint32_t* vals_out = (uint32_t*)(s + L.vals_out);
   size_t tb = L.temp_bytes;
   const PartLayout P = part_layout(n, force_wide);
-  if (P.use && values == Values::kTable && bucket_values(sig, n, rep, s, stream, pinned_flag)) return;
-  if (P.use && values == Values::kMany && bucket_partitioned(P, sig, n, rep, s, stream, pinned_flag))
+  if (P.use && values == Values::kTable && value_layout(n).total <= bytes &&
+      bucket_values(sig, n, rep, s, stream, pinned_flag)) return;
+  if (P.use && values == Values::kMany && P.total <= bytes &&
+      bucket_partitioned(P, sig, n, rep, s, stream, pinned_flag))
     return;
   // the full sort (also when a partition overflowed), from the identity rows
   hipLaunchKernelGGL(k_rep_identity, dim3(grid_for(n, 256), 64), dim3(256), 0, stream, n, rep);

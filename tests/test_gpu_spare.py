@@ -97,3 +97,29 @@ def test_fast_workspace_is_given_back():
         again, _ = db.fast(90)
         db.close()
     np.testing.assert_array_equal(again, first)
+
+
+@pytest.mark.parametrize("letters,n,L", [(AMINO, 16385, 60), (AMINO, 20000, 60), (b"ACGT", 16385, 400)])
+def test_bucket_and_step(letters, n, L):
+    rng = np.random.default_rng(n)
+    aa = np.frombuffer(letters, dtype=np.uint8)
+    anc = aa[rng.integers(0, len(aa), size=(n // 20 + 1, L))]
+    seqs = anc[np.arange(n) // 20]
+    sub = rng.random(seqs.shape) < 0.03
+    seqs[sub] = aa[rng.integers(0, len(aa), size=int(sub.sum()))]
+    packed, off = orc.pack_many([s.tobytes() for s in seqs])
+    lengths = np.full(n, L, dtype=np.uint32)
+    sig = orc.sketch_all(packed, off)
+    rep = orc.bucket(sig)
+    want, _ = orc.build_graph(packed, off, lengths, rep, 64, 90)
+    say("bucketing without the partitions' room", letters[:4], n)
+    with limited(0) as c:
+        np.testing.assert_array_equal(c.bucket(sig), rep)
+        db = ng.Database(c, packed, off, lengths)
+        db.sketch()
+        db.bucket()
+        np.testing.assert_array_equal(db.reps(), rep)
+        db.step(90)
+        np.testing.assert_array_equal(db.reps(), rep)
+        np.testing.assert_array_equal(db.edges(), want)
+        db.close()
