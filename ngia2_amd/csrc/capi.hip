@@ -399,6 +399,7 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
     for (int g = 0; g < kLongGroups; g++)
       for (int k = 0; k < kTuneClasses; k++) key.push_back(rt.lng[g][k]);
   }
+  key.push_back((uintptr_t)ctx->pin);  // gets the bin counts
   key.push_back(db->t0);
   key.push_back(ctx->seg2_min);
   key.push_back(ctx->lane_fill);

@@ -74,3 +74,23 @@ def test_few_pairs(n, length):
     assert ("wave" in kinds) == few
     db.close()
     c.close()
+
+
+def test_database_on_another_context(ctx):
+    """A round captured on one context and asked for on another: its bin counts
+    reach the caller's."""
+    d = ng.gen_packed(ng.gen_config(1, 0.1, 5))
+    rep = orc.bucket(orc.sketch_all(d.packed, d.word_off))
+    want, _ = orc.build_graph(d.packed, d.word_off, d.lengths, rep, 64, 70)
+    print("one database, two contexts", flush=True)
+    with ng.Context(0) as other:
+        db = ng.Database(ctx, d.packed, d.word_off, d.lengths)
+        db.set_reps(rep, 64)
+        launches = []
+        for c in (ctx, other, ctx, other):
+            db.ctx = c
+            launches.append(db.graph(70)["align_launches"])
+            np.testing.assert_array_equal(db.edges(), want)
+        db.ctx = ctx
+        db.close()
+    assert launches[0] > 0 and launches == launches[:1] * 4
