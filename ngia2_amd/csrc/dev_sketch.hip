@@ -318,7 +318,8 @@ __global__ __launch_bounds__(64) void k_sketch_walk(
           run &= run << 1;
           run &= run << 2;
           run &= run << 4;
-          const uint32_t full = (uint32_t)(run >> 32);
+          const uint32_t left = L - 32 * blk, valid = left < 32 ? (1u << left) - 1u : ~0u;
+          const uint32_t full = (uint32_t)(run >> 32) & valid;  // the record may end within the block
           #pragma unroll
           for (int p = 0; p < 32; p++) {
             const uint32_t x = p < 7 ? __builtin_amdgcn_alignbit(c.lo, pv.lo, p + 25) : c.lo >> (p - 7);
@@ -328,10 +329,8 @@ __global__ __launch_bounds__(64) void k_sketch_walk(
             atomicOr((uint32_t*)((char*)bits + ((idx >> 3) & 0x1FFCu)),
                      ((full >> p) & 1u) << (idx & 31u));
           }
-          other = ~full;
+          other = ~full & valid;
           if (blk == 0) other &= ~0x7Fu;  // no window ends before position 7
-          const uint32_t left = L - 32 * blk;
-          if (left < 32) other &= (1u << left) - 1u;
         }
         // windows with another letter, one at a time
         for (uint64_t who = __builtin_amdgcn_ballot_w64(other != 0); who; who &= who - 1) {

@@ -55,3 +55,22 @@ def test_walk_matches_oracle(ctx, alpha, odd):
         np.testing.assert_array_equal(db.sigs(), want)
     db.close()
     np.testing.assert_array_equal(ctx.sketch(packed, off), want)
+
+
+def test_bits_past_a_record(ctx):
+    """A signature ends with its record, whatever the last block's planes hold
+    past it."""
+    rng = np.random.default_rng(4)
+    seqs = [bytes(b"ACGT"[i] for i in rng.integers(4, size=int(L)))
+            for L in list(range(1377, 1412)) + list(rng.integers(400, 60000, size=150))]
+    recs = [orc.pack(s) for s in seqs]
+    off = np.cumsum([0] + [len(r) for r in recs[:-1]]).astype(np.uint64)
+    want = orc.sketch_all(np.concatenate(recs).astype(np.uint32), off)
+    assert sum(map(len, seqs)) > 4000000
+    for s, r in zip(seqs, recs):
+        left = len(s) % 32
+        for p in range(4 * (left > 0)):  # the codes before, again
+            r[-4 + p] |= (int(r[-8 + p]) >> left << left) & 0xFFFFFFFF
+    packed = np.concatenate(recs).astype(np.uint32)
+    say("four-letter sketch with bits past the records")
+    np.testing.assert_array_equal(ctx.sketch(packed, off), want)
