@@ -535,14 +535,15 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
 }
 
 // Signatures of records [first, n) on the context stream: the four-letter walk
-// where the database's letters allow it, else a hash per window and band.
+// for the records that fit it, else a hash per window and band.
 void sketch_records(ngia_ctx* ctx, ngia_db* db, uint32_t first) {
+  const uint8_t* codes = db->codes.as<uint8_t>();
+  const uint64_t* coff = db->code_off.as<uint64_t>();
+  const uint32_t* len = db->lengths.as<uint32_t>();
+  uint32_t* sig = db->sig.as<uint32_t>();
   const uint32_t n = db->n - first;
-  uint32_t* sig = db->sig.as<uint32_t>() + 64ull * first;
-  const uint64_t* coff = db->code_off.as<uint64_t>() + first;
-  const uint32_t* len = db->lengths.as<uint32_t>() + first;
   if (!db->walk_code) {
-    launch_sketch(db->codes.as<uint8_t>(), coff, len, n, sig, ctx->stream);
+    launch_sketch(codes, coff + first, len + first, n, sig + 64ull * first, ctx->stream);
     return;
   }
   if (ctx->walk_code != db->walk_code) {
@@ -551,9 +552,23 @@ void sketch_records(ngia_ctx* ctx, ngia_db* db, uint32_t first) {
     launch_walk_table(db->walk_code, ctx->walk_table.p, ctx->stream);
     ctx->walk_code = db->walk_code;
   }
-  launch_sketch_walk(db->packed.as<uint32_t>(), db->word_off.as<uint64_t>() + first,
-                     db->codes.as<uint8_t>(), coff, len, n, db->walk_code, ctx->walk_table.p,
-                     (uint32_t)ctx->prop.multiProcessorCount, sig, ctx->stream);
+  const uint32_t* packed = db->packed.as<uint32_t>();
+  const uint64_t* woff = db->word_off.as<uint64_t>();
+  const uint32_t cus = (uint32_t)ctx->prop.multiProcessorCount;
+  if (db->walk_yes.empty()) {
+    launch_sketch_walk(packed, woff + first, codes, coff + first, len + first, n, db->walk_code,
+                       ctx->walk_table.p, cus, sig + 64ull * first, ctx->stream);
+    return;
+  }
+  auto rest = [&](const std::vector<uint32_t>& v) {
+    auto before = [](uint32_t e, uint32_t i) { return (e & ~kHashRecord) < i; };
+    return (uint32_t)(v.end() - std::lower_bound(v.begin(), v.end(), first, before));
+  };
+  const uint32_t yes = rest(db->walk_yes), no = rest(db->walk_no);
+  const uint32_t* end = db->walk_list.as<uint32_t>() + db->walk_yes.size();
+  launch_sketch_walk(packed, woff, codes, coff, len, yes, db->walk_code, ctx->walk_table.p, cus, sig,
+                     ctx->stream, end - yes);
+  launch_sketch(codes, coff, len, no, sig, ctx->stream, end + (db->walk_no.size() - no));
 }
 
 // The fast mode by the batched kernels.  The reference takes the bands one by

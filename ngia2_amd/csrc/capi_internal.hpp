@@ -216,8 +216,12 @@ struct ngia_db {
   bool compact = false;
   ngia::DevBuf slot_codes;
   uint32_t slot_code = 0;
-  // four-letter sketch: sym_code of launch_sketch_walk (0: off)
+  // four-letter sketch: sym_code of launch_sketch_walk (0: off); unless every
+  // record walks, those of its kernel, and those of k_sketch (ascending, but for
+  // kHashRecord)
   uint32_t walk_code = 0;
+  std::vector<uint32_t> walk_yes, walk_no;
+  ngia::DevBuf walk_list;  // walk_yes, then walk_no
   // graph workspace
   ngia::DevBuf flags, pos, sums, jobs, degree, edge_off, ekeys, escores, ekeys_tmp, escores_tmp, fin_temp;
   ngia::DevBuf counters, cnt, keep, off, pairs, score, bin_of, list, plain_scratch, plain_jobs,
@@ -412,9 +416,11 @@ inline uint32_t persistent_blocks(const ngia_ctx* ctx, size_t lds_bytes) {
   return cu * per_cu;
 }
 
-// The letters of the four-letter sketch: the database's four most frequent
-// codes (all of them when there are no more than four).
-inline void walk_letters(ngia_db* db, uint32_t nslots, uint64_t bytes, hipStream_t s) {
+// The four-letter sketch: its letters, the database's four most frequent codes (all
+// of them when there are no more than four), and the records that take it; off
+// when they hold too little to pay for its lists.
+inline void walk_setup(ngia_ctx* ctx, ngia_db* db, uint32_t nslots, uint64_t bytes) {
+  hipStream_t s = ctx->stream;
   uint32_t rare = 0;  // the slot left out
   if (nslots > 4) {
     DevBuf count;
@@ -428,9 +434,38 @@ inline void walk_letters(ngia_db* db, uint32_t nslots, uint64_t bytes, hipStream
     for (uint32_t k = 2; k <= nslots; k++)
       if (c[k] < c[rare]) rare = k;
   }
-  db->walk_code = 0;
   for (uint32_t k = 1, y = 0; k <= nslots; k++)
     if (k != rare) db->walk_code |= ((db->slot_code >> (4 * (k - 1))) & 0xFu) << (4 * y++);
+  const uint32_t n = db->n;
+  db->walk_list.ensure(4ull * n);
+  // written to pinned memory where that has the room: after a copy of 160 KB to
+  // pageable memory the next database's upload took 3.2 ms instead of 1.4 (28 MB)
+  const bool pinned = 4ull * n <= kStages * kStageBytes && stage_ready(ctx);
+  std::vector<uint32_t> copy(pinned ? 0 : n);
+  uint32_t* const others = pinned ? (uint32_t*)ctx->stage : copy.data();
+  launch_walk_others(db->packed.as<uint32_t>(), db->word_off.as<uint64_t>(), db->lengths.as<uint32_t>(),
+                     n, db->walk_code, pinned ? others : db->walk_list.as<uint32_t>(), s);
+  if (pinned)
+    NGIA_HIP(hipStreamSynchronize(s));
+  else
+    to_host(ctx, others, db->walk_list.p, 4ull * n);
+  uint64_t all = 0, fit = 0;
+  for (uint32_t i = 0; i < n; i++) {
+    all += db->host_len[i];
+    if (walk_fits(db->host_len[i], others[i])) fit += db->host_len[i];
+  }
+  if (fit < kWalkResidues) db->walk_code = 0;
+  if (fit < kWalkResidues || fit == all) return;
+  const bool own = (double)(all - fit) >= kHashShare * (double)all;  // a launch for the rest
+  for (uint32_t i = 0; i < n; i++) {
+    const bool fits = walk_fits(db->host_len[i], others[i]);
+    if (fits || !own)
+      db->walk_yes.push_back(fits ? i : i | kHashRecord);
+    else
+      db->walk_no.push_back(i);
+  }
+  h2d(db->walk_list.p, db->walk_yes.data(), 4 * db->walk_yes.size(), s);
+  h2d(db->walk_list.as<uint32_t>() + db->walk_yes.size(), db->walk_no.data(), 4 * db->walk_no.size(), s);
 }
 
 inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64_t n_words,
@@ -474,6 +509,7 @@ inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64
   // entries per word in place of 16.
   db->compact = false;
   db->walk_code = 0;
+  db->walk_yes = db->walk_no = {};
   db->slot_codes.release();
   if (acc && !(ctx->full_alphabet)) {
     DevBuf present;
@@ -496,7 +532,7 @@ inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64
       launch_code_slots(db->codes.as<uint8_t>(), acc, lut, db->slot_codes.as<uint8_t>(), s);
       db->compact = true;
       db->slot_code = slot_code;
-      if (acc >= kWalkResidues) walk_letters(db, slot, acc, s);
+      if (acc >= kWalkResidues) walk_setup(ctx, db, slot, acc);
     }
   }
   NGIA_HIP(hipStreamSynchronize(s));

@@ -257,8 +257,24 @@ void launch_walk_table(uint32_t sym_code, void* table, hipStream_t stream);
 void launch_sketch_walk(const uint32_t* packed, const uint64_t* word_off, const uint8_t* codes,
                         const uint64_t* code_off, const uint32_t* lengths, uint32_t n,
                         uint32_t sym_code, const void* table, uint32_t cus, uint32_t* sig,
-                        hipStream_t stream);
+                        hipStream_t stream, const uint32_t* list = nullptr);
 void launch_sketch(const uint8_t* codes, const uint64_t* code_off, const uint32_t* lengths,
-                   uint32_t n, uint32_t* sig, hipStream_t stream);
+                   uint32_t n, uint32_t* sig, hipStream_t stream, const uint32_t* list = nullptr);
+// others[i]: the windows of record i that hold another letter than the four.
+void launch_walk_others(const uint32_t* packed, const uint64_t* word_off, const uint32_t* lengths,
+                        uint32_t n, uint32_t sym_code, uint32_t* others, hipStream_t stream);
+// Whether the walk is a record's shorter way.  Measured, 20 to 28 million
+// residues in records of one length, a hash per window against the walk: 500
+// bases 254 / 174 us, 400 244 / 326 (many are hashed after all, at fewer
+// wavefronts a CU); 1,400 bases with another letter in 4% of the windows 565 / 226,
+// 8% 570 / 399, 15% 564 / 727, 82% 567 / 3,701.
+constexpr uint32_t kWalkLen = 448;
+inline bool walk_fits(uint32_t L, uint32_t others) { return L >= kWalkLen && others <= L / 9; }
+// The walk's kernel hashes a record a third slower than k_sketch, whose launch of
+// its own lasts as long as its longest record: the records that do not fit get one
+// from this share of the residues on.  20,000 records, a few of them hashed: 231 us
+// here, 282 in two launches.
+constexpr uint32_t kHashRecord = 0x80000000u;
+constexpr double kHashShare = 0.1;
 
 }  // namespace ngia

@@ -100,13 +100,17 @@ __device__ __forceinline__ uint32_t lane_seed_term(uint32_t lane) {
   return seed ^ 61u ^ (seed >> 16);
 }
 
+// kList: the records list[0..n).
+template <bool kList>
 __global__ __launch_bounds__(256) void k_sketch(const uint8_t* __restrict__ codes,
                                                 const uint64_t* __restrict__ code_off,
                                                 const uint32_t* __restrict__ lengths,
-                                                uint32_t n, uint32_t* __restrict__ sig) {
+                                                const uint32_t* __restrict__ list, uint32_t n,
+                                                uint32_t* __restrict__ sig) {
   const uint32_t lane = threadIdx.x & 63;
-  const uint32_t seq = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
-  if (seq >= n) return;
+  const uint32_t item = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (item >= n) return;
+  const uint32_t seq = kList ? __builtin_amdgcn_readfirstlane(list[item]) : item;
   const uint32_t L = __builtin_amdgcn_readfirstlane(lengths[seq]);
   const uint32_t* cw = record_codes(codes, code_off, seq);
   const uint32_t first = first_window(L);
@@ -163,10 +167,14 @@ void launch_sketch_chunks(const uint8_t* codes, const uint64_t* code_off, const 
 }
 
 void launch_sketch(const uint8_t* codes, const uint64_t* code_off, const uint32_t* lengths,
-                   uint32_t n, uint32_t* sig, hipStream_t stream) {
+                   uint32_t n, uint32_t* sig, hipStream_t stream, const uint32_t* list) {
   if (n == 0) return;
-  hipLaunchKernelGGL(k_sketch, dim3((n + 3) / 4), dim3(256), 0, stream, codes, code_off, lengths,
-                     n, sig);
+  if (list)
+    hipLaunchKernelGGL(k_sketch<true>, dim3((n + 3) / 4), dim3(256), 0, stream, codes, code_off,
+                       lengths, list, n, sig);
+  else
+    hipLaunchKernelGGL(k_sketch<false>, dim3((n + 3) / 4), dim3(256), 0, stream, codes, code_off,
+                       lengths, list, n, sig);
   NGIA_HIP(hipGetLastError());
 }
 
@@ -178,7 +186,9 @@ void launch_sketch(const uint8_t* codes, const uint64_t* code_off, const uint32_
 // list until it meets a marked one: with D different 8-mers about 65,536 / D
 // probes on average (4.7 times that for the slowest of 64 lanes), in place of
 // a hash per window.  Windows with any other letter (N, unknown ones) are
-// hashed as before and join the minimum.
+// hashed as before and join the minimum, one after another: a record with many of
+// them, or a short one, is hashed throughout (walk_fits), here while such records
+// are few, else by k_sketch.
 // An 8-mer's place in the bit set comes from the records' bit planes: the two
 // bits of a letter over 32 positions are two words, an 8-mer's bits eight
 // consecutive ones of each.  A list entry holds the place as (byte address
@@ -283,11 +293,56 @@ __device__ __forceinline__ LetterBits letter_bits(const uint32_t* pl, uint32_t s
   return {m[1] | m[3], m[2] | m[3], m[0] | m[1] | m[2] | m[3]};
 }
 
-// sym_code: the code of letter y in bits 4y...
+// The positions of a block that end eight of the four letters in a row; p: the
+// block before.
+__device__ __forceinline__ uint32_t full_windows(uint32_t ok, uint32_t prev_ok) {
+  uint64_t run = ((uint64_t)ok << 32) | prev_ok;
+  run &= run << 1;
+  run &= run << 2;
+  run &= run << 4;
+  return (uint32_t)(run >> 32);
+}
+// The positions of block blk that end a window of a record of L residues.
+__device__ __forceinline__ uint32_t window_ends(uint32_t L, uint32_t blk) {
+  const uint32_t left = L - 32 * blk;
+  return (left < 32 ? (1u << left) - 1u : ~0u) & (blk ? ~0u : ~0x7Fu);
+}
+
+// others[i]: the windows of record i that hold another letter.  Four records a
+// block, a wavefront each; bound by reading the records once, 4 bits a residue.
+__global__ __launch_bounds__(256) void k_walk_others(const uint32_t* __restrict__ packed,
+                                                     const uint64_t* __restrict__ word_off,
+                                                     const uint32_t* __restrict__ lengths, uint32_t n,
+                                                     uint32_t sym_code, uint32_t* __restrict__ others) {
+  const uint32_t lane = threadIdx.x & 63u, seq = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (seq >= n) return;
+  const uint32_t L = lengths[seq], nblk = (L + 31) / 32;
+  const uint32_t* planes = packed + word_off[seq] + 1;
+  uint32_t sum = 0;
+  for (uint32_t blk = lane; blk < nblk; blk += 64) {
+    const uint32_t ok = letter_bits(planes + 4ull * blk, sym_code).ok;
+    const uint32_t prev = blk ? letter_bits(planes + 4ull * blk - 4, sym_code).ok : 0u;
+    sum += __popc(~full_windows(ok, prev) & window_ends(L, blk));
+  }
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+  if (lane == 0) others[seq] = sum;
+}
+
+void launch_walk_others(const uint32_t* packed, const uint64_t* word_off, const uint32_t* lengths,
+                        uint32_t n, uint32_t sym_code, uint32_t* others, hipStream_t stream) {
+  if (n == 0) return;
+  hipLaunchKernelGGL(k_walk_others, dim3((n + 3) / 4), dim3(256), 0, stream, packed, word_off, lengths,
+                     n, sym_code, others);
+  NGIA_HIP(hipGetLastError());
+}
+
+// sym_code: the code of letter y in bits 4y..; the records list[0..n), kHashRecord
+// set in those to be hashed, or, without a list, 0..n-1.
 __global__ __launch_bounds__(64) void k_sketch_walk(
     const uint32_t* __restrict__ packed, const uint64_t* __restrict__ word_off,
     const uint8_t* __restrict__ codes, const uint64_t* __restrict__ code_off,
-    const uint32_t* __restrict__ lengths, uint32_t n, uint32_t sym_code,
+    const uint32_t* __restrict__ lengths, const uint32_t* __restrict__ list, uint32_t n,
+    uint32_t sym_code,
     const uint32_t* __restrict__ table, const uint32_t* __restrict__ depth,
     uint32_t* __restrict__ sig) {
   __shared__ __align__(16) uint32_t bits[2048];
@@ -295,11 +350,13 @@ __global__ __launch_bounds__(64) void k_sketch_walk(
   const uint32_t s1 = lane_seed_term(lane);
   const uint32_t batches = *depth / 8;
   const uint4* const tab = (const uint4*)table + 2 * lane;  // batch q at tab[128 q], tab[128 q + 1]
-  for (uint32_t seq = blockIdx.x; seq < n; seq += gridDim.x) {
+  for (uint32_t item = blockIdx.x; item < n; item += gridDim.x) {
+    const uint32_t entry = list ? __builtin_amdgcn_readfirstlane(list[item]) : item;
+    const uint32_t seq = entry & ~kHashRecord;
     const uint32_t L = __builtin_amdgcn_readfirstlane(lengths[seq]);
     const uint32_t* cw = record_codes(codes, code_off, seq);
     uint32_t mn = 0xFFFFFFFFu;
-    bool direct = (uint64_t)L * L < kWalkMin;
+    bool direct = (uint64_t)L * L < kWalkMin || entry != seq;
     if (!direct) {
       const uint32_t* planes = packed + word_off[seq] + 1;
       #pragma unroll
@@ -313,13 +370,7 @@ __global__ __launch_bounds__(64) void k_sketch_walk(
           const LetterBits c = letter_bits(planes + 4ull * blk, sym_code);
           LetterBits pv = {0u, 0u, 0u};
           if (blk) pv = letter_bits(planes + 4ull * blk - 4, sym_code);
-          // positions that end eight letters in a row
-          uint64_t run = ((uint64_t)c.ok << 32) | pv.ok;
-          run &= run << 1;
-          run &= run << 2;
-          run &= run << 4;
-          const uint32_t left = L - 32 * blk, valid = left < 32 ? (1u << left) - 1u : ~0u;
-          const uint32_t full = (uint32_t)(run >> 32) & valid;  // the record may end within the block
+          const uint32_t ends = window_ends(L, blk), full = full_windows(c.ok, pv.ok) & ends;
           #pragma unroll
           for (int p = 0; p < 32; p++) {
             const uint32_t x = p < 7 ? __builtin_amdgcn_alignbit(c.lo, pv.lo, p + 25) : c.lo >> (p - 7);
@@ -329,8 +380,7 @@ __global__ __launch_bounds__(64) void k_sketch_walk(
             atomicOr((uint32_t*)((char*)bits + ((idx >> 3) & 0x1FFCu)),
                      ((full >> p) & 1u) << (idx & 31u));
           }
-          other = ~full & valid;
-          if (blk == 0) other &= ~0x7Fu;  // no window ends before position 7
+          other = ~full & ends;
         }
         // windows with another letter, one at a time
         for (uint64_t who = __builtin_amdgcn_ballot_w64(other != 0); who; who &= who - 1) {
@@ -417,12 +467,12 @@ __global__ __launch_bounds__(64) void k_sketch_walk(
 void launch_sketch_walk(const uint32_t* packed, const uint64_t* word_off, const uint8_t* codes,
                         const uint64_t* code_off, const uint32_t* lengths, uint32_t n,
                         uint32_t sym_code, const void* table, uint32_t cus, uint32_t* sig,
-                        hipStream_t stream) {
+                        hipStream_t stream, const uint32_t* list) {
   if (n == 0) return;
   const uint32_t* depth = (const uint32_t*)table + (size_t)kWalkCap * 64;
   // 20 wavefronts of 8 KiB per CU
   hipLaunchKernelGGL(k_sketch_walk, dim3(std::min(n, cus * 20u)), dim3(64), 0, stream, packed, word_off,
-                     codes, code_off, lengths, n, sym_code, (const uint32_t*)table, depth, sig);
+                     codes, code_off, lengths, list, n, sym_code, (const uint32_t*)table, depth, sig);
   NGIA_HIP(hipGetLastError());
 }
 

@@ -2,6 +2,8 @@
 letters, of three, and of five with N among them; records short and long, of few
 different 8-mers, with runs of unknown letters, and of lengths around the
 blocks of 32 and the bound below which every window is hashed."""
+import os
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,30 @@ def test_bits_past_a_record(ctx):
     packed = np.concatenate(recs).astype(np.uint32)
     say("four-letter sketch with bits past the records")
     np.testing.assert_array_equal(ctx.sketch(packed, off), want)
+
+
+@pytest.mark.parametrize("alpha,odd", [(b"ACGT", b"NX"), (b"ACGTN", b"X")])
+def test_step_with_records_of_both_forms(alpha, odd):
+    """Records too short, of too many other letters or of five letters are
+    hashed window by window, the others walk; a step's head comes off the front of
+    both lists."""
+    rng = np.random.default_rng(len(alpha))
+    seqs = [bytes(alpha[i] for i in rng.integers(len(alpha), size=L)) for L in range(12000, 12020)]
+    seqs += [odd[:1] * 11500] + [odd[-1:] * 60 + s[:10500] for s in seqs[:3]]
+    seqs = sorted(seqs + records(rng, alpha, odd)[30:], key=len, reverse=True)
+    packed, off = orc.pack_many(seqs)
+    lengths = np.array([len(s) for s in seqs], dtype=np.uint32)
+    want = orc.sketch_all(packed, off)
+    os.environ["NGIA_HEAD_MIN"] = "8"
+    try:
+        c = ng.Context(0)
+    finally:
+        del os.environ["NGIA_HEAD_MIN"]
+    say("four-letter sketch of a step with both forms", alpha, odd)
+    with c:
+        db = ng.Database(c, packed, off, lengths)
+        db.step(90)
+        assert c.timing()["step_head"] >= 8
+        np.testing.assert_array_equal(db.sigs(), want)
+        np.testing.assert_array_equal(db.reps(), orc.bucket(want))
+        db.close()
