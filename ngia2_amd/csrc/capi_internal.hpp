@@ -208,6 +208,7 @@ struct ngia_db {
   uint64_t n_words = 0;
   uint32_t max_len = 0;
   double mean_len = 0;
+  double kmers = 65536;  // 8-mers that records of a compact alphabet can hold (dna_values)
   uint32_t rep_bands = 0;
   bool have_sig = false;
   ngia::DevBuf packed, word_off, lengths, codes, code_off, sig, rep;
@@ -449,11 +450,13 @@ inline void walk_setup(ngia_ctx* ctx, ngia_db* db, uint32_t nslots, uint64_t byt
     NGIA_HIP(hipStreamSynchronize(s));
   else
     to_host(ctx, others, db->walk_list.p, 4ull * n);
-  uint64_t all = 0, fit = 0;
+  uint64_t all = 0, fit = 0, other = 0;
   for (uint32_t i = 0; i < n; i++) {
     all += db->host_len[i];
+    other += others[i];
     if (walk_fits(db->host_len[i], others[i])) fit += db->host_len[i];
   }
+  db->kmers = other <= all / 10 ? 65536 : 390625;
   if (fit < kWalkResidues) db->walk_code = 0;
   if (fit < kWalkResidues || fit == all) return;
   const bool own = (double)(all - fit) >= kHashShare * (double)all;  // a launch for the rest
@@ -532,6 +535,7 @@ inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64
       launch_code_slots(db->codes.as<uint8_t>(), acc, lut, db->slot_codes.as<uint8_t>(), s);
       db->compact = true;
       db->slot_code = slot_code;
+      db->kmers = slot > 4 ? 390625 : 65536;
       if (acc >= kWalkResidues) walk_setup(ctx, db, slot, acc);
     }
   }

@@ -87,14 +87,17 @@ __host__ __device__ inline uint32_t lcs_score(uint32_t lcs, uint32_t R, uint32_t
 // equal signatures outgrow any partition: kFew takes the full sort, kTable
 // tries tables of each band's values first, with a synchronisation of its own.
 enum class Values { kMany, kFew, kTable };
-// kTable or kFew for n records of mean_len residues of four letters.  A band's
-// values are the minima of the 4^8 hashes' ranks over a record's 8-mers, about
-// 4^8 / L ln(n L / 4^8) of them (counted with 20,000 to 1 million random reads of
-// 64 to 1,000 residues: 0.9 to 1.25 of that; related records have fewer).
-// Within the tables: 200,000 16S reads 684 -> 242 us, 2 million 7.3 -> 1.8 ms;
-// past them finding out costs 50 us before a sort of 170 (20,000) to 710.
-inline Values dna_values(uint32_t n, double mean_len) {
-  const double L = mean_len > 1 ? mean_len : 1, kmers = 65536.0;
+// kTable or kFew for n records of mean_len residues that hold `kmers` different
+// 8-mers: 4^8 of four letters, 5^8 of five unless the fifth is rare.  A band's
+// values are the minima of their hashes' ranks over a record's 8-mers, about
+// kmers / L ln(n L / kmers) of them (counted with 20,000 to 1 million random reads
+// of 64 to 1,000 residues of four letters: 0.9 to 1.25 of that; related records
+// have fewer).  Within the tables: 200,000 16S reads 684 -> 242 us, 2 million 7.3 ->
+// 1.8 ms; past them finding out costs 50 us before a sort of 170 (20,000) to 710
+// (20,000 records of 1,400 residues of five equally frequent letters 254 us with
+// 4^8, 173 with 5^8).
+inline Values dna_values(uint32_t n, double mean_len, double kmers) {
+  const double L = mean_len > 1 ? mean_len : 1;
   return 1.25 * kmers / L * std::log(1 + n * L / kmers) <= 1400 ? Values::kTable : Values::kFew;
 }
 size_t bucket_scratch_bytes(uint32_t n, bool force_wide = false);
