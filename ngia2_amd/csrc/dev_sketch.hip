@@ -12,6 +12,7 @@
 // writes sig[64*i + k], one 256-byte coalesced store per wavefront.
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include <rocprim/rocprim.hpp>
 
@@ -980,14 +981,18 @@ __global__ __launch_bounds__(BS) void k_bucket_small(const uint32_t* __restrict_
 // the band's whole column (64 KiB at most, in L2) through LDS, and each of its
 // wavefronts gathers the elements of one partition in index order and passes
 // them, 64 at a time, through a table in LDS from value to last index, which is
-// each element's predecessor.  A block per band sorting 16 elements a thread
-// leaves three CUs in four idle.  8,193 records 70 -> 34 us (4,096 of them the
-// same 68 -> 60), 10,000 73 -> 33 (5,000: 71 -> 68), 16,384 94 -> 47 (8,192:
-// 90 -> 104); at 8,192 the sort's 8 elements a thread take 45, this 34 and, with
-// half of them the same, 43 against 58.
+// each element's predecessor.  A value of kMapOften of the 64 gets registers
+// instead, and its elements their predecessors where they are met: through the
+// table the wavefront of a value that half of the records share took the block two
+// to four times as long.
+// A block per band sorting 16 elements a thread leaves three CUs in four idle:
+// 8,193 records 71 us against 28 (half of them the same 69 / 32, all 66 / 28), 10,000
+// 75 / 27 (72 / 35, 70 / 32), 16,384 97 / 40 (91 / 50, 87 / 44), 200 copies of each 91
+// / 68.  At 8,192 the sort's 8 elements a thread take 45, this 34.
 // Bound: instructions, every wavefront looking at the whole column, and latency,
 // of the LDS round trips of each 64.
 constexpr uint32_t kMapSlots = 1024, kMapRing = 512, kMapLoads = 4, kMapWaves = 8;
+constexpr int kMapOften = 24;  // of 64: a value that is taken straight from the column
 constexpr uint32_t kMapChunk = 4096, kMapPer = kMapChunk / (64 * kMapWaves);
 // Partitions of 512 elements or fewer, half the table, and at least a block's.
 constexpr uint32_t map_bits(uint32_t n) {
@@ -1016,83 +1021,131 @@ __global__ __launch_bounds__(64 * kMapWaves) void k_col_map(const uint32_t* __re
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   uint32_t got = 0, done = 0, values = 0;  // elements gathered, passed on, distinct; uniform
   bool crowded = false;
+  // the frequent value, its slot and its last index plus one (0: none yet)
+  uint32_t hot = 0, hot_slot = 0, hot_last = 0;
   uint32_t next[kMapPer];
   #pragma unroll
   for (uint32_t k = 0; k < kMapPer; k++) {
     const uint32_t i = 64 * kMapWaves * k + t;
     next[k] = c[i < n ? i : n - 1];
   }
-  for (uint32_t q0 = 0; q0 < n; q0 += 64 * kMapLoads) {
-    const uint32_t o = q0 % kMapChunk;
-    if (o == 0) {
-      __syncthreads();  // every wavefront is through the chunk before
+  // The column's elements [q0, stop), which lie in the chunk.  kHot: the frequent
+  // value's rows are written here; without one the loop ends after the round that
+  // finds it, and its place is returned.
+  auto scan = [&](auto has_hot, uint32_t q0, uint32_t stop) {
+    constexpr bool kHot = decltype(has_hot)::value;
+    for (; q0 < stop; q0 += 64 * kMapLoads) {
+      uint32_t h[kMapLoads];
       #pragma unroll
-      for (uint32_t k = 0; k < kMapPer; k++) {
-        const uint32_t i = q0 + kMapChunk + 64 * kMapWaves * k + t;
-        chunk[64 * kMapWaves * k + t] = next[k];
-        next[k] = c[i < n ? i : n - 1];
+      for (uint32_t k = 0; k < kMapLoads; k++) h[k] = chunk[q0 % kMapChunk + 64 * k + lane];
+      if (q0 + 64 * kMapLoads > n) {  // past the column: another partition's
+        #pragma unroll
+        for (uint32_t k = 0; k < kMapLoads; k++)
+          if (q0 + 64 * k + lane >= n) h[k] = (at ^ 1u) << (32 - pb);
       }
-      __syncthreads();
-    }
-    uint32_t h[kMapLoads];
-    #pragma unroll
-    for (uint32_t k = 0; k < kMapLoads; k++) h[k] = chunk[o + 64 * k + lane];
-    if (q0 + 64 * kMapLoads > n) {  // past the column: another partition's
+      bool quiet = true;  // without the frequent value
+      if (kHot) {
+        #pragma unroll
+        for (uint32_t k = 0; k < kMapLoads; k++) {
+          const uint64_t m = __builtin_amdgcn_ballot_w64(h[k] == hot);
+          if (!m) continue;
+          const uint64_t lower = m & ((1ull << lane) - 1ull);
+          const uint32_t prev = lower ? q0 + 64 * k + 63 - __clzll(lower) : hot_last - 1;
+          if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+            row[q0 + 64 * k + lane] = prev;
+            h[k] = (at ^ 1u) << (32 - pb);
+          }
+          hot_last = q0 + 64 * k + 64 - __clzll(m);
+          quiet = false;
+        }
+      }
       #pragma unroll
-      for (uint32_t k = 0; k < kMapLoads; k++)
-        if (q0 + 64 * k + lane >= n) h[k] = (at ^ 1u) << (32 - pb);
+      for (uint32_t k = 0; k < kMapLoads; k++) {
+        const uint64_t m = __builtin_amdgcn_ballot_w64(mine(h[k]));
+        const uint32_t place = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo((uint32_t)m, got));
+        if (__builtin_amdgcn_inverse_ballot_w64(m))
+          ring[place % kMapRing] = make_uint2(h[k], q0 + 64 * k + lane);
+        got += (uint32_t)__popcll(m);
+      }
+      if (crowded) done = got;  // what follows is looked up below
+      // The last round, and the one that finds a frequent value, empties the ring.
+      bool end = q0 + 64 * kMapLoads >= n, found = false;
+      uint32_t often = 0, slot_of_it = 0;
+      while (got - done >= 64 || (end && got != done)) {
+        if (values + 64 > kMapSlots) {
+          crowded = true;
+          done = got;
+          break;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const bool on = done + lane < got;
+        const uint2 e = ring[(done + lane) % kMapRing];
+        const uint32_t id = (e.x << pb) | 1u, step = e.x >> 12 | 1u;  // an odd step meets every slot
+        uint32_t slot = (e.x >> 3) % kMapSlots;
+        bool fresh = false, seek = on;
+        while (seek) {
+          const uint32_t was = atomicCAS(&key[slot], 0u, id);
+          fresh = was == 0;
+          seek = was != 0 && was != id;
+          if (seek) slot = (slot + step) % kMapSlots;
+        }
+        values += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(fresh));
+        uint32_t prev = 0, now = 0;
+        if (on) {
+          prev = __hip_atomic_load(&last[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          atomicMax(&last[slot], e.y + 1);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          now = __hip_atomic_load(&last[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        // a value again further up in the same 64: the lanes of each such value
+        // have the element before them among themselves
+        uint64_t again = __builtin_amdgcn_ballot_w64(on && now != e.y + 1);
+        const int repeats = __popcll(again);
+        while (again) {
+          const uint32_t s = __builtin_amdgcn_readlane(slot, __ffsll((unsigned long long)again) - 1);
+          const uint64_t same = __builtin_amdgcn_ballot_w64(on && slot == s);
+          const uint64_t lower = same & ((1ull << lane) - 1ull);
+          if (on && slot == s && lower) prev = ring[(done + 63 - __clzll(lower)) % kMapRing].y + 1;
+          again &= ~same;
+        }
+        if (repeats >= kMapOften && quiet) {  // perhaps the value of some lane in the middle
+          const uint32_t s = __builtin_amdgcn_readlane(slot, 21);
+          if (__popcll(__builtin_amdgcn_ballot_w64(on && slot == s)) >= kMapOften) {
+            often = __builtin_amdgcn_readlane(e.x, 21);
+            slot_of_it = s;
+            end = found = true;
+            if (!kHot) stop = 0;
+          }
+        }
+        if (prev) row[e.y] = prev - 1;
+        done = got - done > 64 ? done + 64 : got;
+      }
+      if (found) {
+        if (kHot && lane == 0) atomicMax(&last[hot_slot], hot_last);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        hot = often;
+        hot_slot = slot_of_it;
+        hot_last = __builtin_amdgcn_readfirstlane(
+            __hip_atomic_load(&last[hot_slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+      }
     }
+    return q0;
+  };
+  for (uint32_t c0 = 0; c0 < n; c0 += kMapChunk) {
+    __syncthreads();  // every wavefront is through the chunk before
     #pragma unroll
-    for (uint32_t k = 0; k < kMapLoads; k++) {
-      const uint64_t m = __builtin_amdgcn_ballot_w64(mine(h[k]));
-      const uint32_t place = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)m, got));
-      if (__builtin_amdgcn_inverse_ballot_w64(m))
-        ring[place % kMapRing] = make_uint2(h[k], q0 + 64 * k + lane);
-      got += (uint32_t)__popcll(m);
+    for (uint32_t k = 0; k < kMapPer; k++) {
+      const uint32_t i = c0 + kMapChunk + 64 * kMapWaves * k + t;
+      chunk[64 * kMapWaves * k + t] = next[k];
+      next[k] = c[i < n ? i : n - 1];
     }
-    if (crowded) done = got;  // what follows is looked up below
-    const bool end = q0 + 64 * kMapLoads >= n;
-    while (got - done >= 64 || (end && got != done)) {
-      if (values + 64 > kMapSlots) {
-        crowded = true;
-        done = got;
-        break;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      const bool on = done + lane < got;
-      const uint2 e = ring[(done + lane) % kMapRing];
-      const uint32_t id = (e.x << pb) | 1u, step = e.x >> 12 | 1u;  // an odd step meets every slot
-      uint32_t slot = (e.x >> 3) % kMapSlots;
-      bool fresh = false, seek = on;
-      while (seek) {
-        const uint32_t was = atomicCAS(&key[slot], 0u, id);
-        fresh = was == 0;
-        seek = was != 0 && was != id;
-        if (seek) slot = (slot + step) % kMapSlots;
-      }
-      values += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(fresh));
-      uint32_t prev = 0, now = 0;
-      if (on) {
-        prev = __hip_atomic_load(&last[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        atomicMax(&last[slot], e.y + 1);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        now = __hip_atomic_load(&last[slot], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-      // a value again further up in the same 64: the lanes of each such value
-      // have the element before them among themselves
-      uint64_t again = __builtin_amdgcn_ballot_w64(on && now != e.y + 1);
-      while (again) {
-        const uint32_t s = __builtin_amdgcn_readlane(slot, __ffsll((unsigned long long)again) - 1);
-        const uint64_t same = __builtin_amdgcn_ballot_w64(on && slot == s);
-        const uint64_t lower = same & ((1ull << lane) - 1ull);
-        if (on && slot == s && lower) prev = ring[(done + 63 - __clzll(lower)) % kMapRing].y + 1;
-        again &= ~same;
-      }
-      if (prev) row[e.y] = prev - 1;
-      done = got - done > 64 ? done + 64 : got;
-    }
+    __syncthreads();
+    const uint32_t stop = n - c0 < kMapChunk ? n : c0 + kMapChunk;
+    uint32_t q0 = c0;
+    if (!hot_last) q0 = scan(std::false_type(), q0, stop);
+    if (hot_last) scan(std::true_type(), q0, stop);
   }
   // More values than slots: each predecessor looked up in the column.  No
   // signatures of records crowd like that, so this need only be right.

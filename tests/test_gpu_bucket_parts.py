@@ -156,3 +156,20 @@ def test_too_many_values(few, values):
     sig[:, 63] = np.arange(n) // (n // values + 1)  # few in a tile
     print("too many values", values, flush=True)
     np.testing.assert_array_equal(few.bucket(sig), orc.bucket(sig))
+
+
+@pytest.mark.parametrize("n", [8193, 12001, 16384])
+def test_small_frequent_values(small, n):
+    """Values frequent enough for registers: one throughout, one in every other
+    record, several in turns of different lengths that meet in a partition (16 or 32
+    of them for 64 bands of six values), and one that comes back."""
+    rng = np.random.default_rng(n)
+    at = np.arange(n)
+    print("frequent values", n, flush=True)
+    for which in (np.zeros(n, np.int64), np.where(at % 2, 0, -1), at // 17 % 6, at // 64 % 6, at // 1000 % 6,
+                  rng.integers(0, 6, n), np.where(rng.random(n) < 0.8, rng.integers(0, 6, n), -1),
+                  np.where(at // 2048 % 2, 0, rng.integers(-1, 3, n))):
+        sig = rng.integers(0, 1 << 32, size=(n, 64), dtype=np.uint64).astype(np.uint32)
+        values = rng.integers(0, 1 << 32, size=(6, 64), dtype=np.uint64).astype(np.uint32)
+        sig[which >= 0] = values[which[which >= 0]]
+        np.testing.assert_array_equal(small.bucket(sig), orc.bucket(sig))
