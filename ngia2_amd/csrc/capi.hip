@@ -723,7 +723,7 @@ void bucket_rows(ngia_ctx* ctx, ngia_db* db, hipStream_t s) {
   else
     launch_bucket(db->sig.as<uint32_t>(), db->n, db->rep.as<uint32_t>(), db->bucket_scratch.p,
                   db->bucket_scratch.bytes, s, ctx->bucket_wide, db->compact ? dna_values(db->n, db->mean_len, db->kmers) : Values::kMany,
-                  (uint32_t*)(ctx->pin + kPinOverflow));
+                  (uint32_t*)(ctx->pin + kPinBucket));
 }
 
 // The head of a step: the leading run of records whose own band window (the

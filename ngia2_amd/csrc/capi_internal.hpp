@@ -94,11 +94,12 @@ struct Counters {
 constexpr int kStages = 4;  // pinned slots of large transfers
 constexpr size_t kCounterStats = offsetof(Counters, queue);
 // Offsets into ngia_ctx::pin.
-constexpr size_t kPinOverflow = 0, kPinUnique = 8, kPinPairs = 16, kPinHeadPairs = 24,
-                 kPinCnt = 64, kPinCounters = 512, kPinHeadCounters = kPinCounters + kCounterStats,
+constexpr size_t kPinBucket = 64, kPinUnique = 8, kPinPairs = 16, kPinHeadPairs = 24,
+                 kPinCnt = 192, kPinCounters = 512, kPinHeadCounters = kPinCounters + kCounterStats,
                  kPinEdges = (kPinHeadCounters + kCounterStats + 63) / 64 * 64,
                  kPinEdgeBytes = 64 << 10, kPinBytes = kPinEdges + kPinEdgeBytes;
-static_assert(kPinCnt + 4 * kBins <= kPinCounters, "pinned slots overlap");
+static_assert(kPinBucket + kBucketPinned <= kPinCnt && kPinCnt + 4 * kBins <= kPinCounters,
+              "pinned slots overlap");
 
 }  // namespace ngia
 
@@ -160,7 +161,7 @@ struct ngia_ctx {
   // counts, counters, the edge count, the bucketing's overflow flag): a copy
   // into pageable memory is staged and waited for one at a time, about 30 us
   // each; into pinned memory the copies queue and one synchronisation covers
-  // them.  Slots (bytes): kPinOverflow, kPinUnique, kPinCnt, kPinPairs,
+  // them.  Slots (bytes): kPinBucket, kPinUnique, kPinCnt, kPinPairs,
   // kPinHeadPairs, kPinCounters, kPinHeadCounters.
   unsigned char* pin = nullptr;
   // the slots of large transfers (to_device, to_host), allocated at the first

@@ -106,11 +106,12 @@ size_t bucket_scratch_bytes(uint32_t n, bool force_wide = false);
 // and the column take 2.3 KB a record (2.1 million records 4.8 GB), the sort's keys
 // and values 1.
 size_t bucket_sort_bytes(uint32_t n, bool force_wide = false);
-// pinned_flag (optional): 4 bytes of pinned host memory that receive the
-// overflow flag of the partitioned form.
+// pinned (optional): kBucketPinned bytes of pinned host memory for the counts that
+// the host reads.
+constexpr size_t kBucketPinned = 128;
 void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch, size_t bytes,
                    hipStream_t stream, bool force_wide = false, Values values = Values::kMany,
-                   uint32_t* pinned_flag = nullptr);
+                   uint32_t* pinned = nullptr);
 // The same rows for n <= kBucketSmallMax records, without a host
 // synchronisation; scratch holds bucket_small_bytes(n) bytes (no more than
 // bucket_scratch_bytes(n)).

@@ -566,21 +566,30 @@ __global__ __launch_bounds__(256) void k_bucket_rep_wide(const uint64_t* __restr
 //     the low bits of h; each element walks its chain for the largest index
 //     below its own with the same h, which is its predecessor in the
 //     reference's stable (sig, i) order.
-//  4. k_part_long: the partitions that outgrew their room (heavily repeated
-//     signatures), from the column.
-// A partition with more distinct values than it has room for is counted; the
-// host then redoes the whole bucketing with the full sort.
+//  4. the host reads what is left (PartsLeft), as a rule nothing: partitions with
+//     chains too long to walk go to k_part_few, or with more values to k_part_left,
+//     which also takes those past their room (heavily repeated signatures), from the
+//     column.
+// Where that would take longer than the full sort, or a partition has more distinct
+// values than it has room for, the host redoes the whole bucketing with the sort.
 // Bound: memory for the first two, 4 + 8 and 4 + 8 bytes an element; the LDS's
 // latency down the chains and the scattered 4-byte row writes for the third.
 // Bands stay on one XCD (block b takes bands of XCD b mod 8), so that the short
 // runs a partition and a row are written in meet in one L2.
-// All 64 bands, against a radix sort by partition and a block sort for each:
-//   records   20,000  50,000  100,000  300,000    1M     2M
-//   before      395     423      472      694   1434   3379 us
-//   now          47      68       95      273    861   1865 us
-// (1M: k_mix_columns 155, k_part_scatter 220, k_part_chain 450 us), and with one
-// signature set repeated 6,000 times 526 -> 196 us at 50,000 and 3950 -> 1703
-// us at 1M records.
+// All 64 bands, against a radix sort by partition and a block sort for each, us:
+//   records                       20,000  50,000  100,000  300,000     1M
+//   random proteins                  392     422      464      666   1321
+//                                     41      57       84      210    617
+//   one signature set in 2%          393     424      598      963   3647
+//                                    104     154      186      383   1161
+//   in half of them                  554     603      777     1457   3600
+//                                    121     236      402     1041   3000
+//   in all                           261     310      468     1119   3178
+//                                    168     255      412     1011   2938
+//   1,000 copies of each             127     183      264      582   4587
+//                                    133     189      294      691   3739
+// (1M: k_mix_columns 121, k_part_scatter 224, k_part_chain 252; before steps 3 and 4
+// bailed out and shared the work as they do, one set in all 9508, 1,000 copies 12058.)
 constexpr uint32_t kPartMaxN = 2800000;
 constexpr uint32_t kPartCap = 4096;
 constexpr uint32_t kScatterTile = 8192, kScatterThreads = 1024;
@@ -708,14 +717,15 @@ __global__ __launch_bounds__(kScatterThreads) void k_part_scatter(const uint32_t
 // by the low bits of h (a chain ends at element kPartCap, which matches
 // nothing and follows itself), a row written for every
 // element with a predecessor.  A walk takes kChainMax steps at most; past that
-// *many is set and the rows are left to the sort.
-constexpr uint32_t kChainMax = 96;
+// *many is set and the rows are left to k_part_left, at once where the chains are
+// longer than kChainMean on average.  *chains: 0.
+constexpr uint32_t kChainMax = 96, kChainMean = 64;
 // A thread walks the chains of all its elements in step: one after another, each
 // would wait for the longest chain of its wavefront.
 constexpr uint32_t kHeads = 2048;
 template <int BS, int kItems>
 __device__ inline void chain_rows(uint2* el, uint16_t* next, uint32_t* head, uint32_t cnt,
-                                  uint32_t* __restrict__ rep, uint32_t* many) {
+                                  uint32_t* __restrict__ rep, uint32_t* many, uint32_t* chains) {
   const uint32_t t = threadIdx.x;
   #pragma unroll
   for (uint32_t k = 0; k < kHeads / BS; k++) head[t + k * BS] = kPartCap;
@@ -733,12 +743,24 @@ __device__ inline void chain_rows(uint2* el, uint16_t* next, uint32_t* head, uin
     i[j] = x.y;
     best[j] = 0;
   }
+  uint32_t firsts = 0;  // the wavefront's elements that start a chain
   #pragma unroll
   for (int j = 0; j < kItems; j++) {
     const uint32_t e = t + j * BS;
-    if (e < cnt) next[e] = (uint16_t)atomicExch(&head[h[j] % kHeads], e);
+    uint32_t f = 0;
+    if (e < cnt) {
+      f = atomicExch(&head[h[j] % kHeads], e);
+      next[e] = (uint16_t)f;
+    }
+    firsts += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(f == kPartCap));
   }
+  if ((t & 63) == 0) atomicAdd(chains, firsts);
   __syncthreads();
+  if (cnt > kChainMean * *chains) {
+    if (t == 0) *many = 1u;
+    __syncthreads();
+    return;
+  }
   #pragma unroll
   for (int j = 0; j < kItems; j++) f[j] = t + j * BS < cnt ? head[h[j] % kHeads] : kPartCap;
   bool more = true;
@@ -763,53 +785,220 @@ __device__ inline void chain_rows(uint2* el, uint16_t* next, uint32_t* head, uin
   __syncthreads();
 }
 
+constexpr uint32_t kRanges = 2048;
+// Exclusive prefix sums of count[0..kRanges) in place, count[kRanges] the total.
 template <int BS>
-constexpr size_t kSortBytes =
-    std::max(std::max(sizeof(typename rocprim::block_radix_sort<uint64_t, BS, (int)kPartCap / BS>::storage_type),
-                      (size_t)16 * BS),
-             (size_t)8 * kPartCap);
-
-// Long chains: the elements sorted by (h, i) in LDS, each row from the element
-// before it.  kKeep: leaves the last element of each value in el[] and returns
-// how many these are.  The storage overlays the elements.
-template <int BS, bool kKeep>
-__device__ inline uint32_t sort_rows(uint2* el, uint32_t cnt, uint32_t* __restrict__ rep,
-                                     void* storage_raw) {
-  constexpr int kItems = (int)kPartCap / BS;
-  using Sort = rocprim::block_radix_sort<uint64_t, BS, kItems>;
-  auto& storage = *reinterpret_cast<typename Sort::storage_type*>(storage_raw);
+__device__ inline void range_starts(uint32_t* count, uint32_t* wsum) {
+  constexpr uint32_t kPer = kRanges / BS;
   const uint32_t t = threadIdx.x;
-  uint64_t key[kItems];
+  uint32_t c[kPer], sum = 0;
+  #pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) {
+    c[k] = count[t * kPer + k];
+    sum += c[k];
+  }
+  uint32_t run = sum;
+  #pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(run, o);
+    if ((t & 63) >= (uint32_t)o) run += y;
+  }
+  if ((t & 63) == 63) wsum[t >> 6] = run;
+  __syncthreads();
+  run -= sum;
+  for (uint32_t w = 0; w < t >> 6; w++) run += wsum[w];
+  #pragma unroll
+  for (uint32_t k = 0; k < kPer; k++) {
+    count[t * kPer + k] = run;
+    run += c[k];
+  }
+  if (t == BS - 1) count[kRanges] = run;
+  __syncthreads();
+}
+
+// The elements of a partition in LDS brought into index order: counted and placed
+// by 2,048 ranges of indices, then each by its rank within its range, which holds
+// few elements, and at most n / 2048.  start: 2,049 words.
+template <int BS, int kItems>
+__device__ inline void index_order(uint2* el, uint32_t cnt, uint32_t n, uint32_t* start, uint32_t* wsum) {
+  const uint32_t t = threadIdx.x;
+  const uint32_t bits = n > 1 ? 32u - (uint32_t)__builtin_clz(n - 1) : 1u;
+  const uint32_t shift = bits > 11 ? bits - 11 : 0u;
+  for (uint32_t k = t; k < kRanges; k += BS) start[k] = 0;
+  __syncthreads();
+  uint2 x[kItems];
+  uint32_t r[kItems];
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    const uint32_t e = t + j * BS;
+    if (e < cnt) {
+      x[j] = el[e];
+      r[j] = atomicAdd(&start[x[j].y >> shift], 1u);
+    }
+  }
+  __syncthreads();
+  range_starts<BS>(start, wsum);
+  #pragma unroll
+  for (int j = 0; j < kItems; j++)
+    if (t + j * BS < cnt) el[start[x[j].y >> shift] + r[j]] = x[j];
+  __syncthreads();
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    if (t + j * BS >= cnt) continue;
+    const uint32_t first = start[x[j].y >> shift], end = start[(x[j].y >> shift) + 1];
+    r[j] = first;
+    for (uint32_t e = first; e < end; e++) r[j] += el[e].y < x[j].y;
+  }
+  __syncthreads();
+  #pragma unroll
+  for (int j = 0; j < kItems; j++)
+    if (t + j * BS < cnt) el[r[j]] = x[j];
+  __syncthreads();
+}
+
+// The rows of a partition of at most kFewMax values: its elements by value and,
+// within one, by ranges between its first and its last index, in kRanges ranges in
+// all.  An element's predecessor is the largest index below its own in its range or,
+// without one, the largest of the nearest range below that holds any.  False (and
+// nothing written) with more values, or more than kFewCrowd elements in a range.
+constexpr uint32_t kFewMax = 64, kFewSlots = 256, kFewCrowd = 128;
+struct FewValues {
+  uint32_t table[kFewSlots];  // 0, or an element of the slot's value, plus one
+  uint32_t id[kFewSlots];     // the slots in use, counted
+  uint32_t low[kFewMax], high[kFewMax], scale[kFewMax];
+  uint32_t values, crowded;
+};
+template <int BS, int kItems>
+__device__ inline bool few_rows(uint2* el, uint32_t cnt, uint32_t* __restrict__ rep, uint32_t* start,
+                                uint32_t* wsum, FewValues& few) {
+  const uint32_t t = threadIdx.x;
+  for (uint32_t k = t; k < kRanges; k += BS) start[k] = 0;
+  for (uint32_t k = t; k < kFewSlots; k += BS) few.table[k] = 0;
+  if (t < kFewMax) {
+    few.low[t] = ~0u;
+    few.high[t] = 0;
+  }
+  if (t == 0) few.values = few.crowded = 0;
+  __syncthreads();
+  uint2 x[kItems];
+  uint32_t v[kItems], r[kItems];  // value, place in its range
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    const uint32_t e = t + j * BS;
+    x[j] = el[e < cnt ? e : 0];
+    uint32_t s = x[j].x % kFewSlots;
+    // ends at a slot of the value's own, or once there are too many values
+    while (e < cnt && __hip_atomic_load(&few.values, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) <= kFewMax) {
+      uint32_t was = __hip_atomic_load(&few.table[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (was == 0) was = atomicCAS(&few.table[s], 0u, e + 1);
+      if (was == 0) atomicAdd(&few.values, 1u);
+      if (was == 0 || el[was - 1].x == x[j].x) break;
+      s = (s + 1) % kFewSlots;
+    }
+    v[j] = s;
+  }
+  __syncthreads();
+  const uint32_t values = few.values;
+  if (values > kFewMax) return false;
+  if (t < kFewSlots) {
+    const bool used = few.table[t] != 0;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(used);
+    if ((t & 63) == 0) wsum[t >> 6] = (uint32_t)__popcll(m);
+    few.id[t] = (uint32_t)__popcll(m & ((1ull << (t & 63)) - 1ull));
+  }
+  __syncthreads();
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    if (t + j * BS >= cnt) continue;
+    uint32_t id = few.id[v[j]];
+    for (uint32_t w = 0; w < v[j] >> 6; w++) id += wsum[w];
+    v[j] = id;
+    // most do not change them: all at one address, atomics take turns
+    if (x[j].y < __hip_atomic_load(&few.low[id], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+      atomicMin(&few.low[id], x[j].y);
+    if (x[j].y > __hip_atomic_load(&few.high[id], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+      atomicMax(&few.high[id], x[j].y);
+  }
+  __syncthreads();
+  const uint32_t ranges = kRanges / values;  // of a value
+  if (t < values) {
+    const uint32_t span = few.high[t] - few.low[t] + 1;
+    const uint32_t use = ranges < span ? ranges : span - 1;  // the product stays below it
+    few.scale[t] = (uint32_t)(((uint64_t)use << 32) / span);
+  }
+  __syncthreads();
+  auto range_of = [&](uint32_t id, uint32_t i) {
+    return id * ranges + __umulhi(i - few.low[id], few.scale[id]);
+  };
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    if (t + j * BS >= cnt) continue;
+    r[j] = atomicAdd(&start[range_of(v[j], x[j].y)], 1u);
+    if (r[j] >= kFewCrowd) few.crowded = 1;
+  }
+  __syncthreads();
+  if (few.crowded) return false;
+  range_starts<BS>(start, wsum);
+  #pragma unroll
+  for (int j = 0; j < kItems; j++)
+    if (t + j * BS < cnt) el[start[range_of(v[j], x[j].y)] + r[j]] = x[j];
+  __syncthreads();
+  #pragma unroll
+  for (int j = 0; j < kItems; j++) {
+    if (t + j * BS >= cnt) continue;
+    const uint32_t k = range_of(v[j], x[j].y), first = start[k];
+    uint32_t best = 0;  // the predecessor's index + 1
+    for (uint32_t e = first; e < start[k + 1]; e++)
+      if (el[e].y < x[j].y && el[e].y + 1 > best) best = el[e].y + 1;
+    if (!best && first > start[v[j] * ranges])
+      for (uint32_t e = start[range_of(v[j], el[first - 1].y)]; e < first; e++)
+        best = el[e].y + 1 > best ? el[e].y + 1 : best;
+    if (best) rep[x[j].y] = best - 1;
+  }
+  return true;
+}
+
+// Elements in index order sorted in LDS, stably, by the bits of h below the
+// partition's pb; an element's predecessor is the one before it if that has the same
+// h.  kKeep: leaves the last element of each value in el[] and returns how many
+// these are.  The sort's storage overlays the elements.
+template <int BS, int kItems>
+constexpr size_t kSortBytes =
+    std::max(sizeof(typename rocprim::block_radix_sort<uint32_t, BS, kItems, uint32_t>::storage_type),
+             (size_t)8 * BS * kItems);
+template <int BS, int kItems, bool kKeep>
+__device__ inline uint32_t sort_rows(uint2* el, uint32_t cnt, uint32_t pb, uint32_t* __restrict__ rep,
+                                     uint32_t* wsum) {
+  using Sort = rocprim::block_radix_sort<uint32_t, BS, kItems, uint32_t>;
+  static_assert(kSortBytes<BS, kItems> <= kSortBytes<BS, (int)kPartCap / BS>, "more than the room");
+  auto& storage = *reinterpret_cast<typename Sort::storage_type*>(el);
+  const uint32_t t = threadIdx.x;
+  uint32_t key[kItems], val[kItems];
   #pragma unroll
   for (int j = 0; j < kItems; j++) {
     const uint32_t q = t * kItems + j;
-    key[j] = q < cnt ? ((uint64_t)el[q].x << 32) | el[q].y : ~0ull;  // no index is all ones
+    const uint2 x = q < cnt ? el[q] : make_uint2(~0u, ~0u);  // the padding stays last
+    key[j] = x.x;
+    val[j] = x.y;
   }
   __syncthreads();
-  Sort().sort(key, storage);
+  Sort().sort(key, val, storage, 0, 32 - pb);
   __syncthreads();
-  uint64_t* last = reinterpret_cast<uint64_t*>(storage_raw);
-  uint32_t* first = reinterpret_cast<uint32_t*>(last + BS);
-  uint32_t* wsum = first + BS;
-  last[t] = key[kItems - 1];
-  first[t] = (uint32_t)(key[0] >> 32);
+  el[t] = make_uint2(key[kItems - 1], val[kItems - 1]);
+  el[BS + t] = make_uint2(key[0], 0);
   __syncthreads();
-  uint64_t prev = t ? last[t - 1] : ~0ull;
+  uint2 prev = t ? el[t - 1] : make_uint2(~key[0], 0);
+  const uint32_t after = t + 1 < BS ? el[BS + t + 1].x : 0u;  // no element past the last thread's
+  uint32_t keep = 0;  // bit j: the last element of its value
   #pragma unroll
   for (int j = 0; j < kItems; j++) {
-    const uint32_t q = t * kItems + j, i = (uint32_t)key[j];
-    if (q >= 1 && q < cnt && (prev >> 32) == (key[j] >> 32)) rep[i] = (uint32_t)prev;
-    prev = key[j];
+    const uint32_t q = t * kItems + j;
+    if (q < cnt && prev.x == key[j]) rep[val[j]] = prev.y;
+    prev = make_uint2(key[j], val[j]);
+    const uint32_t h = j + 1 < kItems ? key[j + 1 < kItems ? j + 1 : j] : after;
+    if (q < cnt && (q + 1 == cnt || h != key[j])) keep |= 1u << j;
   }
   if (!kKeep) return 0;
-  const uint32_t after = t + 1 < BS ? first[t + 1] : 0u;  // 0 for the last: q + 1 == cnt or no element
-  uint32_t keep = 0;  // bit j: key[j] is the last of its value
-  #pragma unroll
-  for (int j = 0; j < kItems; j++) {
-    const uint32_t q = t * kItems + j, h = (uint32_t)(key[j] >> 32);
-    const uint32_t nh = j + 1 < kItems ? (uint32_t)(key[j + 1 < kItems ? j + 1 : j] >> 32) : after;
-    if (q < cnt && (q + 1 == cnt || nh != h)) keep |= 1u << j;
-  }
   uint32_t x = __popc(keep);
   #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -823,10 +1012,9 @@ __device__ inline uint32_t sort_rows(uint2* el, uint32_t cnt, uint32_t* __restri
     if (w < t >> 6) at += wsum[w];
     total += wsum[w];
   }
-  __syncthreads();  // el overlays the storage
   #pragma unroll
   for (int j = 0; j < kItems; j++)
-    if (keep >> j & 1) el[at++] = make_uint2((uint32_t)(key[j] >> 32), (uint32_t)key[j]);
+    if (keep >> j & 1) el[at++] = make_uint2(key[j], val[j]);
   __syncthreads();
   return total;
 }
@@ -834,98 +1022,177 @@ __device__ inline uint32_t sort_rows(uint2* el, uint32_t cnt, uint32_t* __restri
 // The rows of a partition of any size, from the band's whole column: its
 // elements in index order, as many at a time as the room holds, behind the
 // last element of each value so far.  False when these leave no room.
-// Bound: the latency of the column's loads, eight a thread at a time, and a sort for
-// every 4,096 elements.
+// Bound: a round trip to the column for every 4,096 of its elements, asked for a
+// round ahead (one barrier each; one for every 512 took 0.9 ns an element), and a
+// sort for every 4,096 that are the partition's.
 template <int BS>
 __device__ inline bool long_rows(const uint32_t* __restrict__ col, uint32_t n, uint32_t pb,
                                  uint32_t part, uint2* el, uint32_t* __restrict__ rep,
-                                 uint32_t (*wsum)[BS / 64], void* storage_raw) {
+                                 uint32_t (*wsum)[BS / 64], uint32_t* keep_sum) {
   constexpr uint32_t kLoads = 8;
-  const uint32_t t = threadIdx.x;
-  uint32_t cnt = 0;
+  constexpr int kItems = (int)kPartCap / BS;
+  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  const uint32_t mine = w * 64 * kLoads + lane;  // a wavefront's elements lie together
+  uint32_t cnt = 0, h[kLoads], next[kLoads];
+  #pragma unroll
+  for (uint32_t k = 0; k < kLoads; k++) next[k] = mine + 64 * k < n ? col[mine + 64 * k] : 0u;
   __syncthreads();
-  for (uint32_t q0 = 0; q0 < n; q0 += kLoads * BS) {
-    uint32_t h[kLoads];
-    #pragma unroll
-    for (uint32_t k = 0; k < kLoads; k++) h[k] = q0 + k * BS + t < n ? col[q0 + k * BS + t] : 0u;
+  for (uint32_t q0 = 0, round = 0; q0 < n; q0 += kLoads * BS, round ^= 1) {
+    uint64_t m[kLoads];
+    uint32_t own = 0;  // of the wavefront
     #pragma unroll
     for (uint32_t k = 0; k < kLoads; k++) {
-      const uint32_t i = q0 + k * BS + t;
-      const bool take = i < n && (uint32_t)(((uint64_t)h[k] << pb) >> 32) == part;
-      const uint64_t m = __builtin_amdgcn_ballot_w64(take);
-      if ((t & 63) == 0) wsum[k & 1][t >> 6] = (uint32_t)__popcll(m);
-      __syncthreads();
-      uint32_t at = (uint32_t)__popcll(m & ((1ull << (t & 63)) - 1ull)), total = 0;
-      for (uint32_t w = 0; w < BS / 64; w++) {
-        if (w < t >> 6) at += wsum[k & 1][w];
-        total += wsum[k & 1][w];
+      h[k] = next[k];
+      const uint32_t i = q0 + mine + 64 * k, j = i + kLoads * BS;
+      next[k] = j < n ? col[j] : 0u;
+      m[k] = __builtin_amdgcn_ballot_w64(i < n && (uint32_t)(((uint64_t)h[k] << pb) >> 32) == part);
+      own += (uint32_t)__popcll(m[k]);
+    }
+    if (lane == 0) wsum[round][w] = own;
+    __syncthreads();
+    uint32_t total = 0, before = 0;
+    for (uint32_t v = 0; v < BS / 64; v++) {
+      if (v < w) before += wsum[round][v];
+      total += wsum[round][v];
+    }
+    auto put = [&](uint32_t at) {
+      #pragma unroll
+      for (uint32_t k = 0; k < kLoads; k++) {
+        if ((m[k] >> lane) & 1ull)
+          el[at + (uint32_t)__popcll(m[k] & ((1ull << lane) - 1ull))] = make_uint2(h[k], q0 + mine + 64 * k);
+        at += (uint32_t)__popcll(m[k]);
       }
-      if (cnt + total > kPartCap) {  // the same in every thread
-        cnt = sort_rows<BS, true>(el, cnt, rep, storage_raw);
-        if (cnt + BS > kPartCap) return false;
-      }
-      if (take) el[cnt + at] = make_uint2(h[k], i);
+    };
+    if (cnt + total <= kPartCap) {  // the same in every thread
+      put(cnt + before);
       cnt += total;
+      continue;
+    }
+    // else a wavefront's at a time, sorting in between
+    for (uint32_t v = 0; v < BS / 64; v++) {
+      const uint32_t some = wsum[round][v];
+      if (cnt + some > kPartCap) {
+        __syncthreads();
+        cnt = sort_rows<BS, kItems, true>(el, cnt, pb, rep, keep_sum);
+        if (cnt + 64 * kLoads > kPartCap) return false;
+      }
+      if (v == w) put(cnt);
+      cnt += some;
     }
   }
   __syncthreads();
-  sort_rows<BS, false>(el, cnt, rep, storage_raw);
+  sort_rows<BS, kItems, false>(el, cnt, pb, rep, keep_sum);
   return true;
 }
 
-// cursor: the partitions' sizes; `longer` (a count, then the partitions) takes
-// those with more elements than room or with a long chain, for k_part_long.
+// What k_part_chain leaves, for each XCD's eight bands a run of `list`: from its
+// front the partitions with a long chain, from its end those with more elements
+// than room, whose elements are `most` at most and `elements` in all.  overflow:
+// those of them that had too many values.
+struct PartsLeft {
+  uint32_t overflow, most, elements;
+  uint32_t sorts[8], longs[8];
+};
+static_assert(sizeof(PartsLeft) <= kBucketPinned, "no room in pinned memory");
+
 __global__ __launch_bounds__(512) void k_part_chain(const uint2* __restrict__ entries,
                                                     const uint32_t* __restrict__ cursor, uint32_t n,
                                                     uint32_t pb, uint32_t* __restrict__ rep,
-                                                    uint32_t* __restrict__ longer) {
+                                                    PartsLeft* __restrict__ left,
+                                                    uint32_t* __restrict__ list) {
   __shared__ __align__(16) uint2 el[kPartCap + 2];
-  __shared__ uint32_t head[kHeads], many;
+  __shared__ uint32_t head[kHeads], many, chains;
   __shared__ uint16_t next[kPartCap + 2];
   uint32_t band, at;
   band_block(1u << pb, &band, &at);
   const uint32_t part = (band << pb) + at, cnt = cursor[part];
-  if (threadIdx.x == 0) many = cnt > kPartCap;
-  if (cnt <= kPartCap) {
-    const uint2* const v = entries + (uint64_t)part * kPartCap;
-    for (uint32_t e = threadIdx.x; e < cnt; e += 512) el[e] = v[e];
-    __syncthreads();
-    uint32_t* const row = rep + (uint64_t)band * n;
-    // most partitions hold half the room: four elements a thread, not eight
-    if (cnt <= kPartCap / 2)
-      chain_rows<512, (int)kPartCap / 1024>(el, next, head, cnt, row, &many);
-    else
-      chain_rows<512, (int)kPartCap / 512>(el, next, head, cnt, row, &many);
+  const uint32_t x = band / 8, run = 8u << pb;
+  if (cnt > kPartCap) {
+    if (threadIdx.x == 0) {
+      list[(x + 1) * run - 1 - atomicAdd(&left->longs[x], 1u)] = part;
+      atomicMax(&left->most, cnt);
+      atomicAdd(&left->elements, cnt);
+    }
+    return;
   }
-  if (threadIdx.x == 0 && many) longer[1 + atomicAdd(longer, 1u)] = part;
+  if (threadIdx.x == 0) many = chains = 0;
+  const uint2* const v = entries + (uint64_t)part * kPartCap;
+  for (uint32_t e = threadIdx.x; e < cnt; e += 512) el[e] = v[e];
+  __syncthreads();
+  uint32_t* const row = rep + (uint64_t)band * n;
+  // most partitions hold half the room: four elements a thread, not eight
+  if (cnt <= kPartCap / 2)
+    chain_rows<512, (int)kPartCap / 1024>(el, next, head, cnt, row, &many, &chains);
+  else
+    chain_rows<512, (int)kPartCap / 512>(el, next, head, cnt, row, &many, &chains);
+  if (threadIdx.x == 0 && many) list[x * run + atomicAdd(&left->sorts[x], 1u)] = part;
 }
 
-// The partitions that k_part_chain left: sorted, or, past their room, taken
-// from the column.  A kernel of its own, since the sort's registers would cost
-// k_part_chain a third of its wavefronts (1M records: 940 us against 840).  A
-// partition with too many values is counted in `overflow`.
-__global__ __launch_bounds__(512) void k_part_long(const uint32_t* __restrict__ longer,
+// The partitions with a long chain that few_rows takes: their entries in the list
+// become kDone.  Blocks keep to their XCD's bands, as before.  Bound: latency, three
+// blocks a CU; the next partition's place and size are asked for a round ahead.
+constexpr uint32_t kDone = ~0u;
+constexpr uint32_t kFewBlocks = 768;
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_part_few(
+    const PartsLeft* __restrict__ left, uint32_t* __restrict__ list, const uint2* __restrict__ entries,
+    const uint32_t* __restrict__ cursor, uint32_t n, uint32_t pb, uint32_t* __restrict__ rep) {
+  __shared__ __align__(16) uint2 el[kPartCap];
+  __shared__ uint32_t start[kRanges + 1], sums[8];
+  __shared__ FewValues few;
+  const uint32_t x = blockIdx.x % 8, run = 8u << pb, sorts = left->sorts[x], step = gridDim.x / 8;
+  uint32_t p = blockIdx.x / 8;
+  if (p >= sorts) return;
+  uint32_t part = list[x * run + p], cnt = cursor[part];
+  for (; p < sorts; p += step) {
+    const uint32_t after = p + step < sorts ? p + step : p;
+    const uint32_t next = list[x * run + after], next_cnt = cursor[next];
+    uint32_t* const row = rep + (uint64_t)(part >> pb) * n;
+    const uint2* const v = entries + (uint64_t)part * kPartCap;
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < cnt; e += 512) el[e] = v[e];
+    __syncthreads();
+    // two or four elements a thread for most partitions
+    const bool ok = cnt <= 1024   ? few_rows<512, 2>(el, cnt, row, start, sums, few)
+                    : cnt <= 2048 ? few_rows<512, 4>(el, cnt, row, start, sums, few)
+                                  : few_rows<512, 8>(el, cnt, row, start, sums, few);
+    if (ok && threadIdx.x == 0) list[x * run + p] = kDone;
+    part = next;
+    cnt = next_cnt;
+  }
+}
+
+// The others: those past their room, the longest work, from the column, then the
+// rest sorted.  A kernel of its own for the sort's registers, which would cost
+// k_part_chain a third of its wavefronts (1M records: 940 us against 840).
+__global__ __launch_bounds__(512) void k_part_left(PartsLeft* __restrict__ left,
+                                                   const uint32_t* __restrict__ list,
                                                    const uint2* __restrict__ entries,
                                                    const uint32_t* __restrict__ cursor,
                                                    const uint32_t* __restrict__ col, uint32_t n,
-                                                   uint32_t pb, uint32_t* __restrict__ rep,
-                                                   uint32_t* __restrict__ overflow) {
-  __shared__ __align__(16) unsigned char mem[kSortBytes<512>];
-  __shared__ uint32_t wsum[2][8];
+                                                   uint32_t pb, uint32_t* __restrict__ rep) {
+  constexpr int kItems = (int)kPartCap / 512;
+  __shared__ __align__(16) unsigned char mem[kSortBytes<512, kItems>];
+  __shared__ uint32_t start[kRanges + 1], wsum[2][8], sums[8];
   uint2* const el = (uint2*)mem;
-  const uint32_t parts = longer[0];
-  for (uint32_t p = blockIdx.x; p < parts; p += gridDim.x) {
-    const uint32_t part = longer[1 + p], cnt = cursor[part];
+  const uint32_t x = blockIdx.x % 8, run = 8u << pb;
+  const uint32_t longs = left->longs[x], sorts = left->sorts[x];
+  for (uint32_t p = blockIdx.x / 8; p < longs + sorts; p += gridDim.x / 8) {
+    const uint32_t part = list[p < longs ? (x + 1) * run - 1 - p : x * run + p - longs];
+    if (part == kDone) continue;
+    const uint32_t cnt = cursor[part];
     const uint64_t row = (uint64_t)(part >> pb) * n;
     __syncthreads();
-    if (cnt <= kPartCap) {
-      const uint2* const v = entries + (uint64_t)part * kPartCap;
-      for (uint32_t e = threadIdx.x; e < cnt; e += 512) el[e] = v[e];
-      __syncthreads();
-      sort_rows<512, false>(el, cnt, rep + row, mem);
-    } else if (!long_rows<512>(col + row, n, pb, part & ((1u << pb) - 1u), el, rep + row, wsum, mem)) {
-      if (threadIdx.x == 0) atomicAdd(overflow, 1u);
+    if (p < longs) {
+      if (!long_rows<512>(col + row, n, pb, part & ((1u << pb) - 1u), el, rep + row, wsum, sums) &&
+          threadIdx.x == 0)
+        atomicAdd(&left->overflow, 1u);
+      continue;
     }
+    const uint2* const v = entries + (uint64_t)part * kPartCap;
+    for (uint32_t e = threadIdx.x; e < cnt; e += 512) el[e] = v[e];
+    __syncthreads();
+    index_order<512, kItems>(el, cnt, n, start, sums);
+    sort_rows<512, kItems, false>(el, cnt, pb, rep + row, sums);
   }
 }
 
@@ -1356,11 +1623,11 @@ struct BucketLayout {
   size_t keys_in, keys_out, vals_in, vals_out, temp, temp_bytes, total;
 };
 // partitioned path: the band-major column of h, the partitions, their cursors,
-// the overflow count, the count and the list of the partitions past their room
+// and what the chains left
 struct PartLayout {
   bool use;
   uint32_t bits;  // partition bits pb
-  size_t col, entries, cursor, overflow, total;
+  size_t col, entries, cursor, left, list, total;
 };
 PartLayout part_layout(uint32_t n, bool force_wide) {
   PartLayout L{};
@@ -1372,8 +1639,9 @@ PartLayout part_layout(uint32_t n, bool force_wide) {
   L.col = 0;
   L.entries = L.col + al(256ull * n);
   L.cursor = L.entries + al(8 * parts * kPartCap);
-  L.overflow = L.cursor + al(4 * parts);
-  L.total = L.overflow + al(4 * (parts + 2));
+  L.left = L.cursor + al(4 * parts);
+  L.list = L.left + al(sizeof(PartsLeft));
+  L.total = L.list + al(4 * parts);
   return L;
 }
 // few values: the column, the slots, and, cleared together, the bands' tables,
@@ -1428,7 +1696,7 @@ namespace {
 // The bucketing of few values; returns false when there were too many (rep then
 // holds no result).
 bool bucket_values(const uint32_t* sig, uint32_t n, uint32_t* rep, char* s, hipStream_t stream,
-                   uint32_t* pinned_flag) {
+                   uint32_t* pinned) {
   const ValueLayout L = value_layout(n);
   uint32_t* col = (uint32_t*)(s + L.col);
   uint16_t* slots = (uint16_t*)(s + L.slots);
@@ -1445,43 +1713,68 @@ bool bucket_values(const uint32_t* sig, uint32_t n, uint32_t* rep, char* s, hipS
                      tile_last, overflow, rep);
   NGIA_HIP(hipGetLastError());
   uint32_t local = 0;
-  uint32_t* over = pinned_flag ? pinned_flag : &local;
+  uint32_t* over = pinned ? pinned : &local;
   NGIA_HIP(hipMemcpyAsync(over, overflow, 4, hipMemcpyDeviceToHost, stream));
   NGIA_HIP(hipStreamSynchronize(stream));
   return *over == 0;
 }
 
-// The partitioned bucketing; returns false when a partition overflowed (rep
-// then holds a partial result and the caller redoes it with the full sort).
+// The time of k_part_left for the partitions past their room, a CU each, against the
+// full sort's, in us.  Measured: a column's scan 0.4 ns an element, a partition's
+// sorts 4.6 ns of its; the sort 173 us for 20,000 records, 350 for 100,000, 2,400 for
+// a million.  All records alike 20,000 records 168 us by the one and 204 by the
+// other, 50,000 333 and 255; half of them 100,000 records 401 and 415, a tenth of
+// a million 1,522 and 2,970.
+bool sort_instead(const PartsLeft& left, uint32_t longs, uint32_t n) {
+  const double scan = 0.4e-3 * n, sort = 4.6e-3;
+  const double one = scan + sort * left.most, all = (longs * scan + sort * left.elements) / 256;
+  return 20 + std::max(one, all) > 120 + 2.3e-3 * n;
+}
+
+// The partitioned bucketing; returns false when the full sort must or had better
+// redo it (rep then holds a partial result).
 bool bucket_partitioned(const PartLayout& L, const uint32_t* sig, uint32_t n, uint32_t* rep,
-                        char* s, hipStream_t stream, uint32_t* pinned_flag) {
+                        char* s, hipStream_t stream, uint32_t* pinned) {
   const uint32_t pb = L.bits, parts = 64u << pb;
   uint32_t* col = (uint32_t*)(s + L.col);
   uint2* entries = (uint2*)(s + L.entries);
   uint32_t* cursor = (uint32_t*)(s + L.cursor);
-  uint32_t* overflow = (uint32_t*)(s + L.overflow);
-  uint32_t* longer = overflow + 1;
-  // the cursors and the two counts behind them
-  fill_u32(cursor, 0, (L.overflow - L.cursor) / 4 + 2, stream);
+  PartsLeft* left = (PartsLeft*)(s + L.left);
+  uint32_t* list = (uint32_t*)(s + L.list);
+  // the cursors and the counts behind them
+  fill_u32(cursor, 0, (L.left - L.cursor + sizeof(PartsLeft)) / 4, stream);
   hipLaunchKernelGGL(k_mix_columns, dim3((n + 63) / 64), dim3(256), 0, stream, sig, n, col, rep);
   const uint32_t tiles = (n + kScatterTile - 1) / kScatterTile;
   hipLaunchKernelGGL(k_part_scatter, dim3(64 * tiles), dim3(kScatterThreads), 0, stream, col, n, pb, tiles, cursor,
                      entries);
-  hipLaunchKernelGGL(k_part_chain, dim3(parts), dim3(512), 0, stream, entries, cursor, n, pb, rep,
-                     longer);
-  hipLaunchKernelGGL(k_part_long, dim3(std::min(parts, 512u)), dim3(512), 0, stream, longer, entries,
-                     cursor, col, n, pb, rep, overflow);
+  hipLaunchKernelGGL(k_part_chain, dim3(parts), dim3(512), 0, stream, entries, cursor, n, pb, rep, left,
+                     list);
   NGIA_HIP(hipGetLastError());
-  uint32_t local = 0;
-  uint32_t* over = pinned_flag ? pinned_flag : &local;
-  NGIA_HIP(hipMemcpyAsync(over, overflow, 4, hipMemcpyDeviceToHost, stream));
+  PartsLeft local{};
+  PartsLeft* const got = pinned ? (PartsLeft*)pinned : &local;
+  NGIA_HIP(hipMemcpyAsync(got, left, sizeof(PartsLeft), hipMemcpyDeviceToHost, stream));
   NGIA_HIP(hipStreamSynchronize(stream));
-  return *over == 0;
+  uint32_t most = 0, longs = 0;  // of an XCD, and of all
+  for (int x = 0; x < 8; x++) {
+    most = std::max(most, got->sorts[x] + got->longs[x]);
+    longs += got->longs[x];
+  }
+  if (most == 0) return true;
+  if (longs && sort_instead(*got, longs, n)) return false;
+  hipLaunchKernelGGL(k_part_few, dim3(8 * std::min(most, kFewBlocks / 8)), dim3(512), 0, stream, left, list,
+                     entries, cursor, n, pb, rep);
+  hipLaunchKernelGGL(k_part_left, dim3(8 * std::min(most, 128u)), dim3(512), 0, stream, left, list,
+                     entries, cursor, col, n, pb, rep);
+  NGIA_HIP(hipGetLastError());
+  if (longs == 0) return true;
+  NGIA_HIP(hipMemcpyAsync(got, left, sizeof(PartsLeft), hipMemcpyDeviceToHost, stream));
+  NGIA_HIP(hipStreamSynchronize(stream));
+  return got->overflow == 0;
 }
 }  // namespace
 
 void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch, size_t bytes,
-                   hipStream_t stream, bool force_wide, Values values, uint32_t* pinned_flag) {
+                   hipStream_t stream, bool force_wide, Values values, uint32_t* pinned) {
   if (n == 0) return;
   const BucketLayout L = bucket_layout(n, force_wide);
   if (bytes < L.total) throw HipError{NGIA_ERR_ARG, "bucketing scratch too small"};
@@ -1492,9 +1785,9 @@ void launch_bucket(const uint32_t* sig, uint32_t n, uint32_t* rep, void* scratch
   size_t tb = L.temp_bytes;
   const PartLayout P = part_layout(n, force_wide);
   if (P.use && values == Values::kTable && value_layout(n).total <= bytes &&
-      bucket_values(sig, n, rep, s, stream, pinned_flag)) return;
+      bucket_values(sig, n, rep, s, stream, pinned)) return;
   if (P.use && values == Values::kMany && P.total <= bytes &&
-      bucket_partitioned(P, sig, n, rep, s, stream, pinned_flag))
+      bucket_partitioned(P, sig, n, rep, s, stream, pinned))
     return;
   // the full sort (also when a partition overflowed), from the identity rows
   hipLaunchKernelGGL(k_rep_identity, dim3(grid_for(n, 256), 64), dim3(256), 0, stream, n, rep);

@@ -173,3 +173,58 @@ def test_small_frequent_values(small, n):
         values = rng.integers(0, 1 << 32, size=(6, 64), dtype=np.uint64).astype(np.uint32)
         sig[which >= 0] = values[which[which >= 0]]
         np.testing.assert_array_equal(small.bucket(sig), orc.bucket(sig))
+
+
+def families(rng, n, size, order):
+    """Records of n / size signature sets: in random order, one set after another, or
+    so with one of each set's records far from the others."""
+    fam = rng.integers(0, max(n // size, 1), n)
+    if order != "mixed":
+        fam.sort()
+    if order == "strays":
+        stray = rng.integers(0, n, n // size)
+        fam[stray] = rng.integers(0, max(n // size, 1), len(stray))
+    pool = rng.integers(0, 1 << 32, size=(max(n // size, 1), 64), dtype=np.uint64).astype(np.uint32)
+    return pool[fam]
+
+
+@pytest.mark.parametrize("order", ["mixed", "sorted", "strays"])
+@pytest.mark.parametrize("n,size", [(20000, 70), (20000, 200), (20000, 1000), (40000, 4000), (50000, 1000),
+                                    (120001, 1500)])
+def test_families(ctx, n, size, order):
+    """Partitions of few values and long runs, within their room and past it."""
+    sig = families(np.random.default_rng(n + size), n, size, order)
+    print("families", n, size, order, flush=True)
+    np.testing.assert_array_equal(ctx.bucket(sig), orc.bucket(sig))
+
+
+@pytest.mark.parametrize("distinct", [1, 2, 63, 64, 65, 200, 2000])
+@pytest.mark.parametrize("size", [97, 1024, 1025, 2048, 2049, 4095, 4096, 4097, 9000])
+def test_long_chains(ctx, distinct, size):
+    """`size` elements in a few partitions, half of them of one value, the others of
+    `distinct`: the ends of each capacity and of the values that a partition's table
+    takes."""
+    n = 17000
+    rng = np.random.default_rng(distinct * 10000 + size)
+    sig = signatures(n, size)
+    for b in (0, 9, 33, 63):
+        # the partition of all ones, which other records' mixed values rarely reach
+        top = np.uint32(0xFFF00000)
+        h = top | rng.choice(1 << 20, size=distinct + 1, replace=False).astype(np.uint32)
+        rows = rng.permutation(n)[:size] if b != 33 else np.arange(size)
+        which = np.where(rng.random(size) < 0.5, 0, 1 + rng.integers(0, distinct, size))
+        sig[rows, b] = unmix(h[which])
+    print("long chains", distinct, size, flush=True)
+    np.testing.assert_array_equal(ctx.bucket(sig), orc.bucket(sig))
+
+
+@pytest.mark.parametrize("n", [20000, 50000, 300000])
+@pytest.mark.parametrize("share", [0.02, 0.3, 1.0])
+def test_one_frequent_value(ctx, n, share):
+    """One signature set in a share of the records: partitions past their room by the
+    column's scan, or the full sort instead."""
+    rng = np.random.default_rng(n)
+    sig = signatures(n, n + 3)
+    sig[rng.random(n) < share] = sig[7]
+    print("one frequent value", n, share, flush=True)
+    np.testing.assert_array_equal(ctx.bucket(sig), orc.bucket(sig))
