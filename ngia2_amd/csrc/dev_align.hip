@@ -182,11 +182,7 @@ __device__ inline void plain_job(const AlignArgs& A, uint32_t* __restrict__ jobs
   const uint32_t* rr = A.packed + A.word_off[rep];
   const uint32_t* tr = A.packed + A.word_off[tar];
   const uint32_t T = tr[0];
-  if (length_rejects(R, T, A.thr)) {
-    // ngia_align scores it 0; ngia_align_noalloc leaves the caller's value
-    if (!kPlanes) jobs[3 * job + 2] = 0;
-    return;
-  }
+  if (length_rejects(R, T, A.thr)) return;
   const uint32_t nw = (R + 31) / 32;
   for (uint32_t w = 0; w < nw; w++) rows[(uint64_t)w * stride] = 0xFFFFFFFFu;
   const Band bd = band_edges(R, T, A.thr);
@@ -252,6 +248,8 @@ __global__ __launch_bounds__(64) void k_align_plain(AlignArgs A, uint32_t* __res
   const uint32_t tid = blockIdx.x * 64 + lane;
   if (count_ptr) count = *count_ptr;
   uint64_t ran = 0;  // tally: reference tiles of the jobs run
+  // what a job that the length filter rejects scores
+  for (uint32_t job = tid; job < count; job += stride) jobs[3 * job + 2] = 0;
   for (uint32_t job = tid; job < count; job += stride) {
     const uint32_t R = A.packed[A.word_off[jobs[3 * job]]];
     plain_job<false>(A, jobs, job, R, scratch + tid, stride, peq, lane);
