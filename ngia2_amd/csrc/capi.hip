@@ -1002,16 +1002,16 @@ extern "C" int ngia_sync(ngia_ctx* ctx) {
   });
 }
 
-extern "C" int ngia_db_create(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words,
-                              const uint64_t* word_off, const uint32_t* lengths, uint32_t n,
-                              ngia_db** out) {
+namespace ngia {
+int create_db(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words, const uint64_t* word_off,
+              const uint32_t* lengths, uint32_t n, bool sketched, ngia_db** out) {
   if (!ctx || !out || (n && (!packed || !word_off))) return fail(ctx, NGIA_ERR_ARG, "null argument");
   if (n >= 0x7FFFFFFFu) return fail(ctx, NGIA_ERR_ARG, "too many sequences");
   *out = nullptr;
   auto db = std::make_unique<ngia_db>();
   db->ctx = ctx;
   int rc = guarded(ctx, [&] {
-    db_upload(ctx, db.get(), packed, n_words, word_off, lengths, n);
+    db_upload(ctx, db.get(), packed, n_words, word_off, lengths, n, sketched);
     return NGIA_OK;
   });
   if (rc != NGIA_OK) return rc;
@@ -1033,6 +1033,13 @@ extern "C" void ngia_db_destroy(ngia_db* db) {
 
 extern "C" int ngia_db_sketch(ngia_ctx* ctx, ngia_db* db) {
   if (!ctx || !db) return fail(ctx, NGIA_ERR_ARG, "null argument");
+}  // namespace ngia
+
+extern "C" int ngia_db_create(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words,
+                              const uint64_t* word_off, const uint32_t* lengths, uint32_t n,
+                              ngia_db** out) {
+  return create_db(ctx, packed, n_words, word_off, lengths, n, /*sketched=*/true, out);
+}
   return guarded(ctx, [&] {
     db->sig.ensure(256ull * std::max<uint32_t>(db->n, 1));
     NGIA_HIP(hipEventRecord(ctx->ev[6], ctx->stream));
@@ -1336,7 +1343,7 @@ extern "C" int ngia_align(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_word
       return fail(ctx, NGIA_ERR_ARG, "job index out of range");
   if (count == 0) return NGIA_OK;
   ngia_db* db = nullptr;
-  int rc = ngia_db_create(ctx, packed, n_words, word_off, nullptr, n_seqs, &db);
+  int rc = create_db(ctx, packed, n_words, word_off, nullptr, n_seqs, /*sketched=*/false, &db);
   if (rc != NGIA_OK) return rc;
   rc = guarded(ctx, [&] {
     hipStream_t s = ctx->stream;
@@ -1367,7 +1374,7 @@ extern "C" int ngia_build_graph(ngia_ctx* ctx, const uint32_t* packed, uint64_t 
   *edges = nullptr;
   *n_edges = 0;
   ngia_db* db = nullptr;
-  int rc = ngia_db_create(ctx, packed, n_words, word_off, lengths, n, &db);
+  int rc = create_db(ctx, packed, n_words, word_off, lengths, n, /*sketched=*/false, &db);
   if (rc == NGIA_OK) rc = ngia_db_set_reps(ctx, db, rep_rows, bands);
   if (rc == NGIA_OK) rc = ngia_db_graph(ctx, db, identity, bands, flags, stats);
   if (rc == NGIA_OK) {

@@ -473,8 +473,9 @@ inline void walk_setup(ngia_ctx* ctx, ngia_db* db, uint32_t nslots, uint64_t byt
 }
 
 inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64_t n_words,
-               const uint64_t* word_off, const uint32_t* lengths, uint32_t n) {
+               const uint64_t* word_off, const uint32_t* lengths, uint32_t n, bool sketched) {
   std::vector<uint32_t> len_v;
+// sketched: what the four-letter sketch needs is made too.
   if (!lengths) {
     len_v.resize(n);
     for (uint32_t i = 0; i < n; i++) len_v[i] = packed[word_off[i]];
@@ -537,7 +538,7 @@ inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64
       db->compact = true;
       db->slot_code = slot_code;
       db->kmers = slot > 4 ? 390625 : 65536;
-      if (acc >= kWalkResidues) walk_setup(ctx, db, slot, acc);
+      if (sketched && acc >= kWalkResidues) walk_setup(ctx, db, slot, acc);
     }
   }
   NGIA_HIP(hipStreamSynchronize(s));

@@ -171,7 +171,7 @@ extern "C" int ngia_autotune(ngia_ctx* ctx, uint32_t identity, ngia_tune_point* 
         pack_record(res.data(), T, packed.data() + woff[2 * i + 1]);
       }
       db.ctx = ctx;
-      db_upload(ctx, &db, packed.data(), packed.size(), woff.data(), nullptr, nseq);
+      db_upload(ctx, &db, packed.data(), packed.size(), woff.data(), nullptr, nseq, /*sketched=*/false);
       return R;
     };
     // Two passes: proteins (the 16-code table) and DNA, whose window kernels
