@@ -82,3 +82,26 @@ def test_score_column_is_overwritten(ctx, count, thr):
     jobs[:, 2] = 77
     print("align with an old score column", count, thr, flush=True)
     np.testing.assert_array_equal(ctx.align(packed, off, jobs, thr), want)
+
+
+@pytest.mark.parametrize("lengths", [(500,), (60, 500), (60, 500, 1100), (60, 500, 1100, 2400),
+                                     (60, 300, 500, 800, 1100, 1900, 2400, 5200)])
+def test_one_to_many_kernels(ctx, lengths):
+    """A call whose jobs one kernel aligns runs on one stream, others on as many
+    side streams as kernels; calls in a row, each waiting for the one before."""
+    rng = np.random.default_rng(len(lengths))
+    seqs = []
+    for L in lengths:
+        anc = bytes(AMINO[i] for i in rng.integers(20, size=L))
+        seqs += [anc] + [mutate(rng, anc, 0.04, 0.01)[:L] for _ in range(3)]
+    packed, off = orc.pack_many(seqs)
+    for count in (16, 200, 7000):
+        jobs = np.zeros((count, 3), dtype=np.uint32)
+        jobs[:, 0] = rng.integers(0, len(seqs), count)
+        jobs[:, 1] = jobs[:, 0] // 4 * 4 + rng.integers(0, 4, count)
+        for thr in (0.5, 0.8):
+            print("align streams", lengths, count, thr, flush=True)
+            want = orc.align_jobs(packed, off, jobs, thr)
+            assert (want[:, 2] > 0).any()
+            for _ in range(2):
+                np.testing.assert_array_equal(ctx.align(packed, off, jobs, thr), want)
