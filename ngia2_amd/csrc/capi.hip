@@ -621,17 +621,16 @@ uint64_t fast_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t ba
                       uint32_t* parent) {
   hipStream_t s = ctx->stream;
   const uint32_t n = db->n;
-  DevBuf valid, total;
-  valid.ensure(8ull * n);
-  total.ensure(8);
-  fill_u32(total.as<uint32_t>(), 0, 2, s);
+  db->valid.ensure(8ull * (n + 1ull));
+  unsigned long long* total = db->valid.as<unsigned long long>() + n;
+  fill_u32((uint32_t*)total, 0, 2, s);
   const bool split = n >= kFastSplit && bands > 2 * kFastBands;
   for (uint32_t lo = 0; lo < bands;) {
     const uint32_t hi = split && lo == 0 ? kFastBands : bands;
     FastRound f;
     f.parent = parent;
     f.bands = (hi < 64 ? (1ull << hi) - 1ull : ~0ull) & ~((1ull << lo) - 1ull);
-    f.valid = valid.as<uint64_t>();
+    f.valid = db->valid.as<uint64_t>();
     f.last = hi == bands;
     enqueue_bins(ctx, db, identity, bands, s, f);
     NGIA_HIP(hipStreamSynchronize(s));
@@ -641,11 +640,11 @@ uint64_t fast_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t ba
     if ((mask >> kBinPlain) & 1u) ensure_plain_bin_space(db, bands);
     enqueue_scores(ctx, db, (float)identity / 100.0f, (uint64_t)n * bands, mask, false, false, s, false);
     fast_resolve(n, db->off.as<uint64_t>(), db->pairs.as<uint2>(), db->score.as<uint32_t>(),
-                 db->keep.as<uint64_t>(), f, total.as<unsigned long long>(), s);
+                 db->keep.as<uint64_t>(), f, total, s);
     lo = hi;
   }
   unsigned long long t = 0;
-  d2h(&t, total.p, 8, s);
+  d2h(&t, total, 8, s);
   NGIA_HIP(hipStreamSynchronize(s));
   return t;
 }

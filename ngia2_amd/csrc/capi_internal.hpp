@@ -252,6 +252,9 @@ struct ngia_db {
   // the fast mode's round workspace (ngia_db_fast), with views likewise; null
   // while a fast call uses it
   std::unique_ptr<ngia_db> fast;
+  // (fast only) the bands of each target that have a representative, and the
+  // reference's pair count behind them
+  ngia::DevBuf valid;
   // (head only) its records' sketch in chunks of positions: (record, first
   // position) per chunk
   ngia::DevBuf sketch_chunks;
