@@ -31,11 +31,14 @@ void ensure_edge_space(ngia_db* db, uint64_t m) {
   db->escores.ensure(4 * m);
   db->ekeys_tmp.ensure(8 * m);
   db->escores_tmp.ensure(4 * m);
-  db->fin_temp.ensure(finalize_scratch_bytes(m));
 }
 
 void finalize(ngia_ctx* ctx, ngia_db* db, uint64_t m) {
   Counters* dc = db->counters.as<Counters>();
+  db->n_edges = 0;
+  // here, since the batched round has its list without a sort, as a rule: a
+  // one-shot graph spends more on its allocations than on its kernels
+  db->fin_temp.ensure(finalize_scratch_bytes(std::max<uint64_t>(m, 1)));
   finalize_edges(db->ekeys.as<uint64_t>(), db->escores.as<uint32_t>(), m, db->n,
                  db->ekeys_tmp.as<uint64_t>(), db->escores_tmp.as<uint32_t>(), db->fin_temp.p,
                  db->fin_temp.bytes, &dc->unique, ctx->stream);
