@@ -1033,6 +1033,13 @@ int create_db(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words, const uin
   ctx->dbs.push_back(*out);
   return NGIA_OK;
 }
+}  // namespace ngia
+
+extern "C" int ngia_db_create(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words,
+                              const uint64_t* word_off, const uint32_t* lengths, uint32_t n,
+                              ngia_db** out) {
+  return create_db(ctx, packed, n_words, word_off, lengths, n, /*sketched=*/true, out);
+}
 
 extern "C" void ngia_db_destroy(ngia_db* db) {
   if (!db) return;
@@ -1047,13 +1054,6 @@ extern "C" void ngia_db_destroy(ngia_db* db) {
 
 extern "C" int ngia_db_sketch(ngia_ctx* ctx, ngia_db* db) {
   if (!ctx || !db) return fail(ctx, NGIA_ERR_ARG, "null argument");
-}  // namespace ngia
-
-extern "C" int ngia_db_create(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words,
-                              const uint64_t* word_off, const uint32_t* lengths, uint32_t n,
-                              ngia_db** out) {
-  return create_db(ctx, packed, n_words, word_off, lengths, n, /*sketched=*/true, out);
-}
   return guarded(ctx, [&] {
     db->sig.ensure(256ull * std::max<uint32_t>(db->n, 1));
     NGIA_HIP(hipEventRecord(ctx->ev[6], ctx->stream));

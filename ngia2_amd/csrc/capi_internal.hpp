@@ -475,10 +475,10 @@ inline void walk_setup(ngia_ctx* ctx, ngia_db* db, uint32_t nslots, uint64_t byt
   h2d(db->walk_list.as<uint32_t>() + db->walk_yes.size(), db->walk_no.data(), 4 * db->walk_no.size(), s);
 }
 
+// sketched: what the four-letter sketch needs is made too.
 inline void db_upload(ngia_ctx* ctx, ngia_db* db, const uint32_t* packed, uint64_t n_words,
                const uint64_t* word_off, const uint32_t* lengths, uint32_t n, bool sketched) {
   std::vector<uint32_t> len_v;
-// sketched: what the four-letter sketch needs is made too.
   if (!lengths) {
     len_v.resize(n);
     for (uint32_t i = 0; i < n; i++) len_v[i] = packed[word_off[i]];
