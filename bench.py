@@ -60,9 +60,10 @@ def sketch_work(lengths):
     return ops, nbytes
 
 
-def kernel_name(b):
+def kernel_name(b, table):
+    """table: whether a window bin's kernel has its match masks in LDS."""
     if b["kind"] == "window":
-        return ("k_align_win<%d>" if b["width"] <= 8 else "k_align_lanes<%d>") % b["width"]
+        return ("k_align_win<%d>" if table else "k_align_lanes<%d>") % b["width"]
     if b["kind"] == "wave":
         return "k_align_wave<%d>" % b["width"]
     if b["kind"] == "seg":
@@ -308,7 +309,7 @@ def serving_bench(ng, np, ctx, d, params, identity, n_queries, seed):
     return out
 
 
-def align_rooflines(m, peak):
+def align_rooflines(m, peak, dna):
     """Per alignment kernel and for the whole phase: `achieved` counts the
     reference tiles of the blocks the kernels ran (run_tiles, from the tally
     round; an early exit skips the rest of a failing pair), so `frac` is the
@@ -316,12 +317,18 @@ def align_rooflines(m, peak):
     reference tile of the pairs, the work the reference's loop does for them:
     with early exits it can exceed the peak, as it measures skipped work too."""
     rows = []
+    widths = set()
     for b in m["bins"]:
+        # a width's first bin is k_align_win's up to 8 words, 16 of DNA; a second
+        # one, for few pairs, k_align_lanes'
+        table = b["kind"] == "window" and b["width"] <= (16 if dna else 8) and b["width"] not in widths
+        if table:
+            widths.add(b["width"])
         if b["kind"] not in ("window", "wave", "seg", "seg2", "seg3", "seg4", "plain") or not b["pairs"] or b["ms"] <= 0:
             continue
         sec = b["ms"] * 1e-3
         ach = b["run_tiles"] * OPS_PER_TILE / sec / 1e12
-        rows.append({"kernel": kernel_name(b), "pairs": b["pairs"], "ref_tiles": b["ref_tiles"],
+        rows.append({"kernel": kernel_name(b, table), "pairs": b["pairs"], "ref_tiles": b["ref_tiles"],
                      "run_tiles": b["run_tiles"], "kernel_ms": round(b["ms"], 4),
                      "achieved": round(ach, 3), "frac": round(ach / peak, 4),
                      "ref_rate": round(b["ref_tiles"] * OPS_PER_TILE / sec / 1e12, 3)})
@@ -561,7 +568,7 @@ def main():
                    "algorithmic_bytes": nbytes,
                    "hbm_gbps": round(nbytes / (sk_ms * 1e-3) / 1e9, 2),
                    "hbm_frac": round(nbytes / (sk_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 5)}
-    align_rows, phase = align_rooflines(m, peak)
+    align_rows, phase = align_rooflines(m, peak, params.dna)
     # the dominant kernel: the one with the most device time per step
     roofline = sketch_roof
     if align_rows and align_rows[0]["kernel_ms"] > sk_ms:
@@ -661,7 +668,7 @@ def main():
             plain = 0 if args.no_plain else (3 if cfg != 3 else 1)
             m2 = measure(ng, np, ctx, info, d2, ident, args.steps, args.warmup, plain,
                          "config %d -i %d" % (cfg, ident), split=not args.no_split)
-            rows2, phase2 = align_rooflines(m2, peak)
+            rows2, phase2 = align_rooflines(m2, peak, p2.dna)
             r = {"identity": ident, "routing_tuned_at_identity": tuned_at,
                  "value": round(m2["value"], 1),
                  "ms_per_step": round(m2["ms_per_step"], 3),

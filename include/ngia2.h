@@ -92,8 +92,8 @@ int ngia_sync(ngia_ctx* ctx);
  * No reference counterpart: replaces the reference's wall-clock phase timers
  * (buildGraph.hpp:272, 352-361). */
 typedef struct {
-  double sketch_ms;   /* k_sketch of the last ngia_db_sketch */
-  double bucket_ms;   /* transpose + radix sort + predecessor of the last ngia_db_bucket */
+  double sketch_ms;   /* the signatures of the last ngia_db_sketch */
+  double bucket_ms;   /* the representative rows of the last ngia_db_bucket */
   double graph_ms;    /* candidates .. raw edges of the last ngia_db_graph */
   double finalize_ms; /* the sorted edge list of the last ngia_db_graph */
   double align_ms;    /* alignment bins alone (NGIA_GRAPH_BATCHED_EAGER only, else 0) */

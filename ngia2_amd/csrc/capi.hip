@@ -657,8 +657,9 @@ uint64_t fast_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t ba
 // threshold is none the bins are made for.
 // From kAlignBinned jobs on, against one thread a job over rows in global memory
 // (the call, with the records' upload): 5,000 log-normal proteins 16 jobs 544 ->
-// 382 us (one 696 -> 745), 1,000 1006 -> 401, 20,000 1331 -> 583; 20,000 DNA
-// reads 16 jobs 2.0 -> 1.2 ms, 20,000 2.2 -> 1.4.
+// 382 us, 1,000 1006 -> 401, 20,000 1331 -> 583; 20,000 DNA reads 16 jobs 2.0 -> 1.2
+// ms, 20,000 2.2 -> 1.4; eight records of 500 residues at 50% 16 jobs 303 -> 176 us, of
+// 50 residues, the least to align, 149 -> 158.
 constexpr uint32_t kAlignBinned = 16;
 bool align_binned(ngia_ctx* ctx, ngia_db* db, uint32_t* jobs, uint32_t count, float thr) {
   if (!(thr > 0.0f && thr < 1.0f)) return false;

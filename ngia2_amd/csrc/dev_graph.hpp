@@ -106,8 +106,8 @@ constexpr uint32_t kShapeSeg8 = NGIA_SHAPE_SEG8;
 constexpr uint32_t kShapes = kShapeSeg8 + 1;
 constexpr int kTuneClasses = NGIA_TUNE_CLASSES;
 // Window bin W holding c pairs is aligned with shape[W][k], k the last size
-// class with class_size[k] <= c (class 0 below class_size[0]).  A zeroed table
-// keeps every window bin on k_align_win<W>.
+// class with class_size[k] <= c (class 0 below class_size[0]).  Under a zeroed
+// table the sizes of the bins and of the round decide (k_bin_offsets).
 // Groups of 17..60-word windows: lng[g][k] = NGIA_LONG_* for group g
 // (17..21, 22..30, 32..45, 46..60 words) in size class k.
 constexpr int kLongGroups = NGIA_LONG_GROUPS;

@@ -477,7 +477,7 @@ void launch_batch(ngia_serve* sv, uint32_t k, const uint8_t* res, const uint64_t
       longest = std::max(longest, Lq);
     }
   }
-  // One wavefront sketches a position in about 55 ns: past two chunks the
+  // A lone wavefront sketches a position in about 38 ns: past two chunks the
   // longest query would keep the batch waiting (1.1 ms for 8,192 log-normal
   // queries, 20,000 residues the longest).
   const bool in_chunks = longest > 2 * kSketchChunk;
