@@ -392,12 +392,14 @@ struct HeadRound {
 
 // The batched round: its first part captured once per (identity, bands), its
 // second once per set of bins that hold pairs, both replayed (or launched
-// eagerly, with the alignment phase timed).  With a head round, the main
-// round's targets start at db->t0 and the head's edges join it in the list.
+// eagerly, with the alignment phase timed; or, on a database of one call, just
+// launched).  With a head round, the main round's targets start at db->t0 and the
+// head's edges join it in the list.
 void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands,
                    ngia_graph_stats* st, bool eager, bool tally, const HeadRound* head = nullptr) {
   hipStream_t s = ctx->stream;
   const uint32_t n = db->n;
+  const bool captured = !eager && !db->one_call;
   ensure_batched_space(db, bands);
   // Everything the captured kernels were given: a replay is valid while none
   // of it changed (a grown buffer moves, a new tuning changes the routing).
@@ -420,7 +422,7 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
   key.push_back(ctx->lane_fill);
   const bool reuse = db->gexec && db->g_identity == identity && db->g_bands == bands &&
                      db->g_key == key;
-  if (!eager && !reuse) {
+  if (captured && !reuse) {
     drop_graphs(db);
     db->gexec = capture(s, [&] { enqueue_bins(ctx, db, identity, bands, s); });
     db->g_identity = identity;
@@ -428,10 +430,10 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
     db->g_key = key;
   }
   NGIA_HIP(hipEventRecord(ctx->ev[0], s));
-  if (eager)
-    enqueue_bins(ctx, db, identity, bands, s);
-  else
+  if (captured)
     NGIA_HIP(hipGraphLaunch(db->gexec, s));
+  else
+    enqueue_bins(ctx, db, identity, bands, s);
   // the bins that hold pairs pick the second part
   uint32_t cnt[kBins];
   NGIA_HIP(hipStreamSynchronize(s));
@@ -450,9 +452,10 @@ void graph_batched(ngia_ctx* ctx, ngia_db* db, uint32_t identity, uint32_t bands
     }
     db->gexec2.swap(keep);
   }
-  if (eager) {
-    // Same kernels without the graph, with events around the alignment phase.
-    enqueue_align(ctx, db, identity, bands, mask, /*time_align=*/true, tally, s);
+  if (!captured) {
+    // Same kernels without the graph; eagerly, with events around the alignment
+    // phase.
+    enqueue_align(ctx, db, identity, bands, mask, /*time_align=*/eager, tally, s);
   } else {
     hipGraphExec_t g2 = nullptr;
     for (const auto& e : db->gexec2)
@@ -1019,14 +1022,15 @@ extern "C" int ngia_sync(ngia_ctx* ctx) {
 
 namespace ngia {
 int create_db(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words, const uint64_t* word_off,
-              const uint32_t* lengths, uint32_t n, bool sketched, ngia_db** out) {
+              const uint32_t* lengths, uint32_t n, bool one_call, ngia_db** out) {
   if (!ctx || !out || (n && (!packed || !word_off))) return fail(ctx, NGIA_ERR_ARG, "null argument");
   if (n >= 0x7FFFFFFFu) return fail(ctx, NGIA_ERR_ARG, "too many sequences");
   *out = nullptr;
   auto db = std::make_unique<ngia_db>();
   db->ctx = ctx;
   int rc = guarded(ctx, [&] {
-    db_upload(ctx, db.get(), packed, n_words, word_off, lengths, n, sketched);
+    db_upload(ctx, db.get(), packed, n_words, word_off, lengths, n, !one_call);
+    db->one_call = one_call;
     return NGIA_OK;
   });
   if (rc != NGIA_OK) return rc;
@@ -1039,7 +1043,7 @@ int create_db(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words, const uin
 extern "C" int ngia_db_create(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words,
                               const uint64_t* word_off, const uint32_t* lengths, uint32_t n,
                               ngia_db** out) {
-  return create_db(ctx, packed, n_words, word_off, lengths, n, /*sketched=*/true, out);
+  return create_db(ctx, packed, n_words, word_off, lengths, n, /*one_call=*/false, out);
 }
 
 extern "C" void ngia_db_destroy(ngia_db* db) {
@@ -1358,7 +1362,7 @@ extern "C" int ngia_align(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_word
       return fail(ctx, NGIA_ERR_ARG, "job index out of range");
   if (count == 0) return NGIA_OK;
   ngia_db* db = nullptr;
-  int rc = create_db(ctx, packed, n_words, word_off, nullptr, n_seqs, /*sketched=*/false, &db);
+  int rc = create_db(ctx, packed, n_words, word_off, nullptr, n_seqs, /*one_call=*/true, &db);
   if (rc != NGIA_OK) return rc;
   rc = guarded(ctx, [&] {
     hipStream_t s = ctx->stream;
@@ -1389,7 +1393,7 @@ extern "C" int ngia_build_graph(ngia_ctx* ctx, const uint32_t* packed, uint64_t 
   *edges = nullptr;
   *n_edges = 0;
   ngia_db* db = nullptr;
-  int rc = create_db(ctx, packed, n_words, word_off, lengths, n, /*sketched=*/false, &db);
+  int rc = create_db(ctx, packed, n_words, word_off, lengths, n, /*one_call=*/true, &db);
   if (rc == NGIA_OK) rc = ngia_db_set_reps(ctx, db, rep_rows, bands);
   if (rc == NGIA_OK) rc = ngia_db_graph(ctx, db, identity, bands, flags, stats);
   if (rc == NGIA_OK) {

@@ -212,6 +212,7 @@ struct ngia_db {
   double kmers = 65536;  // 8-mers that records of a compact alphabet can hold (dna_values)
   uint32_t rep_bands = 0;
   bool have_sig = false;
+  bool one_call = false;  // lives for one call (create_db): its round is not captured
   ngia::DevBuf packed, word_off, lengths, codes, code_off, sig, rep;
   // compact alphabet (at most kSlotCodes nonzero codes occur): slot of every
   // residue, laid out as codes; slot_code as in AlignArgs

@@ -155,7 +155,7 @@ extern "C" int ngia_build_graph_chunked(ngia_ctx* ctx, const uint32_t* packed, u
       }
       ngia_db* db = nullptr;
       ngia_graph_stats st;
-      rc = create_db(ctx, lpacked.data(), lpacked.size(), loff.data(), llen.data(), nl, /*sketched=*/false, &db);
+      rc = create_db(ctx, lpacked.data(), lpacked.size(), loff.data(), llen.data(), nl, /*one_call=*/true, &db);
       if (rc == NGIA_OK) rc = ngia_db_set_reps(ctx, db, lrep.data(), bands);
       if (rc == NGIA_OK) rc = ngia_db_graph(ctx, db, identity, bands, NGIA_GRAPH_BATCHED, &st);
       uint64_t m = 0;

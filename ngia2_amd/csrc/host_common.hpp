@@ -51,10 +51,11 @@ void pack_records(const uint8_t* res, const uint64_t* res_off, const uint32_t* r
                   uint32_t first, uint32_t count, const uint64_t* word_pos, uint64_t word_base,
                   uint32_t* dst);
 
-// ngia_db_create; sketched: whether the records' signatures may be asked for (without
-// what only these need they come out the same, more slowly).
+// ngia_db_create; one_call: the database lives for one graph or align call and is not
+// sketched.  Its round is launched without a capture, and the upload makes nothing
+// for the sketch.
 int create_db(ngia_ctx* ctx, const uint32_t* packed, uint64_t n_words, const uint64_t* word_off,
-              const uint32_t* lengths, uint32_t n, bool sketched, ngia_db** out);
+              const uint32_t* lengths, uint32_t n, bool one_call, ngia_db** out);
 
 // Frees device workspaces that ctx only keeps for a later call, before its free
 // memory is asked for.

@@ -226,7 +226,7 @@ extern "C" int ngia_cluster(ngia_ctx* ctx, const char* packed_path, const char* 
     ngia_free(e);
   } else {
     ngia_db* db = nullptr;
-    rc = create_db(ctx, pdb.packed, pdb.n_words, pdb.word_off, pdb.lengths, pdb.n, /*sketched=*/false, &db);
+    rc = create_db(ctx, pdb.packed, pdb.n_words, pdb.word_off, pdb.lengths, pdb.n, /*one_call=*/true, &db);
     if (rc == NGIA_OK) rc = ngia_db_set_reps(ctx, db, pdb.rep_rows, bands);
     if (rc == NGIA_OK) rc = ngia_db_graph(ctx, db, identity, bands, flags, stats);
     if (rc == NGIA_OK) rc = ngia_db_get_edges(ctx, db, nullptr, 0, &m);
